@@ -160,6 +160,14 @@ _SIGNATURES: dict[str, list] = {
     "ftx_expcode_decode_d2d": [_vp, _vp, _sz, _sz, ctypes.c_int, _vp],
     "ftx_expcode_encode_dense": [_vp, _sz, _vp, _sz, ctypes.POINTER(_sz)],
     "ftx_expcode_decode_dense_d2d": [_vp, _vp, _sz, _sz, ctypes.c_int, _vp],
+    "ftx_attention_workspace": [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _int, _int, _int, ctypes.POINTER(_sz)],
+    "ftx_attention": [_vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _int, _int, _int, _vp, _int,
+                      ctypes.c_int64, ctypes.c_float, _vp, _sz, _vp],
+    "ftx_norm": [_vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64, _int, _vp, _vp, _vp, _vp, ctypes.c_int64, _int,
+                 _int, _int, ctypes.c_float, _vp],
+    "ftx_rope_cache": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64, _int, _int, _int,
+                       ctypes.c_int64, _vp, _vp],
+    "ftx_silu_mul": [_vp, _vp, _vp, ctypes.c_int64, _vp],
     "ftx_fp8_linear_fused": [_vp, ctypes.c_int, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, _vp,
                              _vp, _sz, _vp],
 }
@@ -167,6 +175,11 @@ _SIGNATURES: dict[str, list] = {
 FP8_EPILOGUE_NONE = 0
 FP8_EPILOGUE_SWIGLU = 1
 FP8_EPILOGUE_RESIDUAL = 2
+
+NORM_NONE = 0
+NORM_RMS = 1
+NORM_LAYER = 2
+NORM_ADALN = 3
 
 _lib: ctypes.CDLL | None = None
 _lock = threading.Lock()

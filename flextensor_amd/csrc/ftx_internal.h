@@ -99,6 +99,56 @@ constexpr int kMfmaProbe16x16x32 = 0;  // v_mfma_f32_16x16x32_bf16, the prefill 
 constexpr int kMfmaProbe32x32x16 = 1;  // v_mfma_f32_32x32x16_bf16
 hipError_t launch_mfma_probe(int shape, int workgroups, int iters, float *sink, hipStream_t stream);
 
+// One attention call (ftx_attention.hip). Strides are in elements: [batch, position, head].
+struct AttentionLaunch {
+  const uint16_t *q, *k, *v;  // bf16
+  uint16_t *o;                // bf16
+  float *part;                // per-split values, maxima and sums (part_bytes), when splits > 1
+  int64_t q_stride[3], k_stride[3], v_stride[3], o_stride[3];
+  int batch, t, s, heads, kv_heads, d;
+  int causal, pos;            // causal: query t sees the keys up to pos + t
+  float scale_log2;           // the score scale times log2(e)
+  // planned
+  int rep, rows, waves, row_tiles, splits, split_tiles, xcds;
+  int64_t items;
+  size_t part_bytes;
+};
+// Fills the planned members from the shapes.
+void plan_attention(AttentionLaunch *p, int cus, int xcds);
+hipError_t launch_attention(const AttentionLaunch &p, hipStream_t stream);
+
+// The operations between a layer's matrix products (ftx_layers.hip). dim is a multiple of 8.
+constexpr int kNormMaxDim = 32768;
+constexpr int kNormNone = FTX_NORM_NONE, kNormRms = FTX_NORM_RMS, kNormAffine = FTX_NORM_LAYER,
+              kNormAdaln = FTX_NORM_ADALN;
+constexpr int kNormNoResidual = 0, kNormResidual = 1, kNormGatedResidual = 2;
+struct NormLaunch {
+  const uint16_t *x;      // bf16 [rows, dim]
+  const uint16_t *delta;  // bf16 [rows, dim]: added to x (times the gate when gated) before the norm
+  uint16_t *x_out;        // bf16 [rows, dim]: the sum, when there is a delta
+  uint16_t *y;            // bf16 [rows, dim]: the normalised rows (unless norm is kNormNone)
+  const uint16_t *w, *b;  // bf16 [dim]: RMS weight, or LayerNorm weight and bias
+  const uint16_t *mod;    // bf16 [6, dim]: AdaLN modulation
+  const uint16_t *e;      // bf16 [rows / rows_per_batch, 6, dim]: timestep embedding, added to mod
+  int64_t rows, rows_per_batch;
+  int dim, norm, residual;
+  int gate, scale, shift; // which of the six AdaLN terms
+  float eps;
+};
+hipError_t launch_norm(const NormLaunch &p, hipStream_t stream);
+
+struct RopeLaunch {
+  const uint16_t *q, *k, *v;  // bf16 [batch, t, heads or kv_heads, d], contiguous
+  uint16_t *q_out;            // like q
+  uint16_t *cache_k, *cache_v;
+  const float *cos, *sin;     // fp32 [positions, d]
+  int64_t k_stride[3], v_stride[3];  // of the caches, in elements: batch, position, head
+  int64_t pos;
+  int batch, t, heads, kv_heads, d;  // d a multiple of 16
+};
+hipError_t launch_rope_cache(const RopeLaunch &p, hipStream_t stream);
+hipError_t launch_silu_mul(const uint16_t *g, const uint16_t *u, uint16_t *y, int64_t n, hipStream_t stream);
+
 // Staged copies from pageable host memory and the parallel host memcpy
 // (ftx_staged.hip).
 int staged_copy_h2d(void *dst, const void *src, size_t nbytes, hipStream_t stream);

@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdio>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -1099,6 +1100,228 @@ int ftx_fp8_linear_static(const void *x, const void *w, const void *scale, void 
     if (rc != FTX_OK) return rc;
   }
   return run_fp8(p, x, &w, &scale, &y, ws, p.workspace_bytes, true, stream);
+}
+
+namespace {
+
+// The checks that every operand of a layer operation shares: aligned device memory that holds its extent.
+int check_operand(const void *p, int64_t elements, int64_t item, const char *what) {
+  if (!p) return ftx::fail(FTX_ERR_INVALID, std::string(what) + " is null");
+  if (reinterpret_cast<uintptr_t>(p) % 16 != 0)
+    return ftx::fail(FTX_ERR_INVALID, std::string(what) + " needs 16-byte alignment");
+  return ftx::check_device_range(p, static_cast<size_t>(elements * item), what);
+}
+
+// Elements from the first to the last of a [n0, n1, n2, d] view, or -1 for a stride that is negative, not a
+// multiple of 8 or beyond any memory.
+int64_t view_extent(const int64_t *stride, int64_t n0, int64_t n1, int64_t n2, int64_t d) {
+  const int64_t n[3] = {n0, n1, n2};
+  int64_t extent = d;
+  for (int i = 0; i < 3; ++i) {
+    if (stride[i] < 0 || stride[i] % 8 != 0 || stride[i] > (int64_t(1) << 40)) return -1;
+    extent += (n[i] - 1) * stride[i];
+  }
+  return extent;
+}
+
+int plan_attention_call(int64_t batch, int64_t t, int64_t s, int heads, int kv_heads, int d, ftx::AttentionLaunch *p) {
+  constexpr int64_t kMax = int64_t(1) << 24;
+  if (batch < 0 || t < 0 || s < 0) return ftx::fail(FTX_ERR_INVALID, "negative dimension");
+  if (heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0)
+    return ftx::fail(FTX_ERR_INVALID, "attention needs heads that are a multiple of kv_heads");
+  if (d != 64 && d != 128) return ftx::fail(FTX_ERR_UNSUPPORTED, "attention runs at head dimensions 64 and 128");
+  if (s == 0) return ftx::fail(FTX_ERR_INVALID, "attention over no keys");
+  if (batch > kMax || t > kMax || s > kMax || heads > 65536 || t * (heads / kv_heads) > kMax ||
+      batch * heads * std::max<int64_t>(t, 1) > (int64_t(1) << 30))
+    return ftx::fail(FTX_ERR_INVALID, "attention dimensions too large");
+  p->batch = static_cast<int>(batch);
+  p->t = static_cast<int>(t);
+  p->s = static_cast<int>(s);
+  p->heads = heads;
+  p->kv_heads = kv_heads;
+  p->d = d;
+  if (batch == 0 || t == 0) return FTX_OK;
+  int cus = 256, xcds = 8;
+  ftx::DeviceState *st = nullptr;
+  if (ftx::device_state(&st) == FTX_OK) {
+    cus = st->cu_count;
+    xcds = st->xcd_count;
+  }
+  ftx::plan_attention(p, cus, xcds);
+  return FTX_OK;
+}
+
+}  // namespace
+
+int ftx_attention_workspace(int64_t batch, int64_t t, int64_t s, int heads, int kv_heads, int d, size_t *bytes) {
+  if (!bytes) return ftx::fail(FTX_ERR_INVALID, "bytes is null");
+  ftx::AttentionLaunch p{};
+  int rc = plan_attention_call(batch, t, s, heads, kv_heads, d, &p);
+  if (rc != FTX_OK) return rc;
+  *bytes = p.part_bytes;
+  return FTX_OK;
+}
+
+int ftx_attention(const void *q, const void *k, const void *v, void *o, int64_t batch, int64_t t, int64_t s, int heads,
+                  int kv_heads, int d, const int64_t *strides, int causal, int64_t pos, float scale, void *workspace,
+                  size_t workspace_bytes, void *stream) {
+  FTX_REQUIRE_LIVE();
+  ftx::AttentionLaunch p{};
+  int rc = plan_attention_call(batch, t, s, heads, kv_heads, d, &p);
+  if (rc != FTX_OK) return rc;
+  if (batch == 0 || t == 0) return FTX_OK;
+  if (!strides) return ftx::fail(FTX_ERR_INVALID, "strides is null");
+  if (!(scale > 0.f) || std::isinf(scale)) return ftx::fail(FTX_ERR_INVALID, "attention needs a positive scale");
+  if (causal && (pos < 0 || pos > (int64_t(1) << 24)))
+    return ftx::fail(FTX_ERR_INVALID, "causal attention needs a position in [0, 2^24]");
+  const int64_t extent[4] = {view_extent(strides, batch, t, heads, d), view_extent(strides + 3, batch, s, kv_heads, d),
+                             view_extent(strides + 6, batch, s, kv_heads, d),
+                             view_extent(strides + 9, batch, t, heads, d)};
+  const void *ptr[4] = {q, k, v, o};
+  const char *name[4] = {"attention q", "attention k", "attention v", "attention o"};
+  for (int i = 0; i < 4; ++i) {
+    if (extent[i] < 0)
+      return ftx::fail(FTX_ERR_INVALID, std::string(name[i]) + ": strides must be multiples of 8 and not negative");
+    rc = check_operand(ptr[i], extent[i], 2, name[i]);
+    if (rc != FTX_OK) return rc;
+  }
+  // one head's keys are addressed by 32-bit byte offsets, rows of a last partial tile included
+  if ((s + 256) * 2 * std::max(strides[4], strides[7]) >= int64_t(1) << 31)
+    return ftx::fail(FTX_ERR_UNSUPPORTED, "attention: one head's keys must span less than 2^31 bytes");
+  if (p.part_bytes > 0) {
+    if (workspace_bytes < p.part_bytes)
+      return ftx::fail(FTX_ERR_INVALID, "attention needs a workspace of " + std::to_string(p.part_bytes) +
+                                            " bytes (ftx_attention_workspace)");
+    rc = check_operand(workspace, static_cast<int64_t>(p.part_bytes), 1, "attention workspace");
+    if (rc != FTX_OK) return rc;
+  }
+  p.q = static_cast<const uint16_t *>(q);
+  p.k = static_cast<const uint16_t *>(k);
+  p.v = static_cast<const uint16_t *>(v);
+  p.o = static_cast<uint16_t *>(o);
+  p.part = static_cast<float *>(workspace);
+  for (int i = 0; i < 3; ++i) {
+    p.q_stride[i] = strides[i];
+    p.k_stride[i] = strides[3 + i];
+    p.v_stride[i] = strides[6 + i];
+    p.o_stride[i] = strides[9 + i];
+  }
+  p.causal = causal != 0;
+  p.pos = causal ? static_cast<int>(pos) : 0;
+  p.scale_log2 = scale * 1.44269504088896340736f;
+  FTX_HIP(ftx::launch_attention(p, static_cast<hipStream_t>(stream)));
+  return FTX_OK;
+}
+
+int ftx_norm(const void *x, const void *delta, void *x_out, void *y, int64_t rows, int64_t dim, int norm,
+             const void *w, const void *b, const void *mod, const void *e, int64_t rows_per_batch, int gate, int scale,
+             int shift, float eps, void *stream) {
+  FTX_REQUIRE_LIVE();
+  if (rows < 0 || dim <= 0 || rows > (int64_t(1) << 31) - 1) return ftx::fail(FTX_ERR_INVALID, "norm dimensions");
+  if (dim % 8 != 0 || dim > ftx::kNormMaxDim)
+    return ftx::fail(FTX_ERR_UNSUPPORTED, "norm rows hold a multiple of 8 values, at most 32768");
+  if (norm < FTX_NORM_NONE || norm > FTX_NORM_ADALN) return ftx::fail(FTX_ERR_INVALID, "unknown norm");
+  if (gate > 5 || (gate >= 0 && !delta)) return ftx::fail(FTX_ERR_INVALID, "the gate is one of six terms on a delta");
+  if (norm == FTX_NORM_ADALN && (scale < 0 || scale > 5 || shift < 0 || shift > 5))
+    return ftx::fail(FTX_ERR_INVALID, "scale and shift are each one of six terms");
+  if (rows == 0) return FTX_OK;
+  const int64_t n = rows * dim;
+  int rc = check_operand(x, n, 2, "norm input");
+  if (rc == FTX_OK && delta) rc = check_operand(delta, n, 2, "norm delta");
+  if (rc == FTX_OK && delta) rc = check_operand(x_out, n, 2, "norm sum");
+  if (rc == FTX_OK && norm != FTX_NORM_NONE) rc = check_operand(y, n, 2, "norm output");
+  if (rc == FTX_OK && (norm == FTX_NORM_RMS || norm == FTX_NORM_LAYER)) rc = check_operand(w, dim, 2, "norm weight");
+  if (rc == FTX_OK && norm == FTX_NORM_LAYER) rc = check_operand(b, dim, 2, "norm bias");
+  if (rc == FTX_OK && (gate >= 0 || norm == FTX_NORM_ADALN)) {
+    if (rows_per_batch <= 0) return ftx::fail(FTX_ERR_INVALID, "rows_per_batch must be positive");
+    rc = check_operand(mod, 6 * dim, 2, "norm modulation");
+    if (rc == FTX_OK) rc = check_operand(e, (rows + rows_per_batch - 1) / rows_per_batch * 6 * dim, 2, "norm embedding");
+  }
+  if (rc != FTX_OK) return rc;
+  ftx::NormLaunch p{};
+  p.x = static_cast<const uint16_t *>(x);
+  p.delta = static_cast<const uint16_t *>(delta);
+  p.x_out = static_cast<uint16_t *>(x_out);
+  p.y = static_cast<uint16_t *>(y);
+  p.w = static_cast<const uint16_t *>(w);
+  p.b = static_cast<const uint16_t *>(b);
+  p.mod = static_cast<const uint16_t *>(mod);
+  p.e = gate >= 0 || norm == FTX_NORM_ADALN ? static_cast<const uint16_t *>(e) : nullptr;
+  p.rows = rows;
+  p.rows_per_batch = rows_per_batch;
+  p.dim = static_cast<int>(dim);
+  p.norm = norm;
+  p.residual = !delta ? ftx::kNormNoResidual : gate >= 0 ? ftx::kNormGatedResidual : ftx::kNormResidual;
+  p.gate = gate;
+  p.scale = scale;
+  p.shift = shift;
+  p.eps = eps;
+  FTX_HIP(ftx::launch_norm(p, static_cast<hipStream_t>(stream)));
+  return FTX_OK;
+}
+
+int ftx_rope_cache(const void *q, const void *k, const void *v, const void *cos, const void *sin, void *q_out,
+                   void *cache_k, void *cache_v, int64_t batch, int64_t t, int heads, int kv_heads, int d, int64_t pos,
+                   const int64_t *cache_strides, void *stream) {
+  FTX_REQUIRE_LIVE();
+  if (batch < 0 || t < 0 || heads <= 0 || kv_heads <= 0 || d <= 0 || pos < 0)
+    return ftx::fail(FTX_ERR_INVALID, "rope dimensions");
+  if (d % 16 != 0 || d > 4096 || heads > 65536 || kv_heads > 65536 || pos > (int64_t(1) << 30))
+    return ftx::fail(FTX_ERR_UNSUPPORTED, "rope heads hold a multiple of 16 values, at most 4096");
+  if (batch > (int64_t(1) << 24) || t > (int64_t(1) << 24) ||
+      batch * t * (heads + 2 * static_cast<int64_t>(kv_heads)) * d > int64_t(1) << 35)
+    return ftx::fail(FTX_ERR_INVALID, "rope dimensions too large");
+  if (batch == 0 || t == 0) return FTX_OK;
+  if (!cache_strides) return ftx::fail(FTX_ERR_INVALID, "cache_strides is null");
+  const int64_t ke = view_extent(cache_strides, batch, pos + t, kv_heads, d);
+  const int64_t ve = view_extent(cache_strides + 3, batch, pos + t, kv_heads, d);
+  if (ke < 0 || ve < 0)
+    return ftx::fail(FTX_ERR_INVALID, "cache strides must be multiples of 8 and not negative");
+  const int64_t nq = batch * t * heads * d, nk = batch * t * kv_heads * d;
+  int rc = check_operand(q, nq, 2, "rope q");
+  if (rc == FTX_OK) rc = check_operand(k, nk, 2, "rope k");
+  if (rc == FTX_OK) rc = check_operand(v, nk, 2, "rope v");
+  if (rc == FTX_OK) rc = check_operand(q_out, nq, 2, "rope q output");
+  if (rc == FTX_OK) rc = check_operand(cos, (pos + t) * d, 4, "rope cos");
+  if (rc == FTX_OK) rc = check_operand(sin, (pos + t) * d, 4, "rope sin");
+  if (rc == FTX_OK) rc = check_operand(cache_k, ke, 2, "key cache");
+  if (rc == FTX_OK) rc = check_operand(cache_v, ve, 2, "value cache");
+  if (rc != FTX_OK) return rc;
+  ftx::RopeLaunch p{};
+  p.q = static_cast<const uint16_t *>(q);
+  p.k = static_cast<const uint16_t *>(k);
+  p.v = static_cast<const uint16_t *>(v);
+  p.q_out = static_cast<uint16_t *>(q_out);
+  p.cache_k = static_cast<uint16_t *>(cache_k);
+  p.cache_v = static_cast<uint16_t *>(cache_v);
+  p.cos = static_cast<const float *>(cos);
+  p.sin = static_cast<const float *>(sin);
+  for (int i = 0; i < 3; ++i) {
+    p.k_stride[i] = cache_strides[i];
+    p.v_stride[i] = cache_strides[3 + i];
+  }
+  p.pos = pos;
+  p.batch = static_cast<int>(batch);
+  p.t = static_cast<int>(t);
+  p.heads = heads;
+  p.kv_heads = kv_heads;
+  p.d = d;
+  FTX_HIP(ftx::launch_rope_cache(p, static_cast<hipStream_t>(stream)));
+  return FTX_OK;
+}
+
+int ftx_silu_mul(const void *g, const void *u, void *y, int64_t n, void *stream) {
+  FTX_REQUIRE_LIVE();
+  if (n < 0 || n > (int64_t(1) << 40)) return ftx::fail(FTX_ERR_INVALID, "silu_mul size");
+  if (n % 8 != 0) return ftx::fail(FTX_ERR_UNSUPPORTED, "silu_mul takes a multiple of 8 values");
+  if (n == 0) return FTX_OK;
+  int rc = check_operand(g, n, 2, "silu_mul gate");
+  if (rc == FTX_OK) rc = check_operand(u, n, 2, "silu_mul up");
+  if (rc == FTX_OK) rc = check_operand(y, n, 2, "silu_mul output");
+  if (rc != FTX_OK) return rc;
+  FTX_HIP(ftx::launch_silu_mul(static_cast<const uint16_t *>(g), static_cast<const uint16_t *>(u),
+                               static_cast<uint16_t *>(y), n, static_cast<hipStream_t>(stream)));
+  return FTX_OK;
 }
 
 int ftx_scatter_plan_create(const ftx_desc *descs, int n_desc, size_t tile_bytes, ftx_scatter_plan **plan) {

@@ -11,6 +11,7 @@ as a CPU ``uint8`` tensor without copying.
 from __future__ import annotations
 
 import ctypes
+import math
 from collections.abc import Iterator
 from contextlib import contextmanager
 from typing import Any
@@ -334,6 +335,139 @@ def checksum(t: torch.Tensor, stream: HipStream | None = None) -> int:
         raise ValueError("checksum needs a contiguous device tensor")
     s = stream if stream is not None else current_stream(t.device)
     return nat.checksum64(t.data_ptr(), t.numel() * t.element_size(), s.handle)
+
+
+def kernel_call(*tensors: torch.Tensor) -> bool:
+    """Whether a call on these tensors may run a library kernel in place of torch operations: bf16 tensors on the
+    current GPU, and nothing around the call that has to see torch operations - autograd, forward-mode
+    differentiation, a function or dispatch mode (an offload manager's discovery is one), a functorch transform,
+    autocast, or a trace."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_function_stack()
+            or torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda")):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in _PLAIN_TYPES or t.dtype != torch.bfloat16 or not t.is_cuda or (grad and t.requires_grad):
+            return False
+    return tensors[0].get_device() == torch.cuda.current_device() and \
+        all(t.get_device() == tensors[0].get_device() for t in tensors[1:])
+
+
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _packed(*tensors: torch.Tensor) -> bool:
+    """Whether every tensor is contiguous and starts at a 16-byte boundary."""
+    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _stream() -> int:
+    return torch.cuda.current_stream().cuda_stream
+
+
+def _strided_heads(t: torch.Tensor) -> bool:
+    """Whether a [batch, position, head, d] tensor can be read 16 bytes at a time: contiguous along d, every
+    other stride (of more than one element) a multiple of 8, a 16-byte aligned start."""
+    return t.stride(3) == 1 and t.data_ptr() % 16 == 0 and all(t.stride(i) % 8 == 0 for i in range(3) if t.shape[i] > 1)
+
+
+def _strides(t: torch.Tensor) -> tuple[int, int, int]:
+    return tuple(t.stride(i) if t.shape[i] > 1 else 0 for i in range(3))
+
+
+def attention_eligible(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether :func:`attention` takes these [batch, position, head, d] tensors."""
+    if not kernel_call(q, k, v) or q.dim() != 4 or k.dim() != 4 or k.shape != v.shape:
+        return False
+    b, t, h, d = q.shape
+    s, kv = k.shape[1], k.shape[2]
+    return (k.shape[0] == b and k.shape[3] == d and d in (64, 128) and b > 0 and t > 0 and s > 0 and kv > 0
+            and h > 0 and h % kv == 0 and max(b, t * (h // kv), s) <= 1 << 24 and h <= 65536 and b * h * t <= 1 << 30
+            and (s + 256) * 2 * max(k.stride(1), v.stride(1)) < 1 << 31
+            and _strided_heads(q) and _strided_heads(k) and _strided_heads(v))
+
+
+_ATTENTION_WORKSPACE: dict[tuple, int] = {}
+
+
+def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: int | None = None) -> torch.Tensor:
+    """``softmax(q k^T / sqrt(d)) v`` over bf16 [batch, position, head, d] tensors (``ftx_attention``).
+
+    ``k`` and ``v`` may have fewer heads than ``q`` (each shared by a group) and any strides; the result is laid
+    out as q is. ``pos``: query t sees the keys up to ``pos + t``; None: every key.
+    """
+    b, t, h, d = q.shape
+    s, kv = k.shape[1], k.shape[2]
+    out = torch.empty_like(q)
+    key = (b, t, s, h, kv, d)
+    ws_bytes = _ATTENTION_WORKSPACE.get(key)
+    if ws_bytes is None:
+        got = ctypes.c_size_t(0)
+        nat.call("ftx_attention_workspace", b, t, s, h, kv, d, ctypes.byref(got))
+        if len(_ATTENTION_WORKSPACE) >= 4096:  # a decode's key count grows by one a step
+            _ATTENTION_WORKSPACE.clear()
+        ws_bytes = _ATTENTION_WORKSPACE[key] = int(got.value)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    strides = (ctypes.c_int64 * 12)(*_strides(q), *_strides(k), *_strides(v), *_strides(out))
+    nat.call("ftx_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, t, s, h, kv, d, strides,
+             int(pos is not None), pos or 0, 1.0 / math.sqrt(d), ws.data_ptr() if ws is not None else None, ws_bytes,
+             _stream())
+    return out
+
+
+NORM_MAX_DIM = 32768
+
+
+def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor | None:
+    """``bf16(x * rsqrt(mean(x^2) + eps) * weight)`` over the last dimension in one launch (``ftx_norm``), or
+    None when the kernel does not take the call."""
+    dim = x.shape[-1] if x.dim() else 0
+    if (not dim or dim % 8 or dim > NORM_MAX_DIM or not x.numel() or x.numel() // dim >= 1 << 31
+            or not kernel_call(x, weight) or weight.shape != (dim,) or not _packed(x, weight)):
+        return None
+    y = torch.empty_like(x)
+    nat.call("ftx_norm", x.data_ptr(), None, None, y.data_ptr(), x.numel() // dim, dim, nat.NORM_RMS,
+             weight.data_ptr(), None, None, None, 1, -1, -1, -1, eps, _stream())
+    return y
+
+
+def rope_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: int,
+               cache_k: torch.Tensor, cache_v: torch.Tensor) -> torch.Tensor | None:
+    """The rotated queries of [batch, t, head, d] ``q``; the rotated ``k`` and ``v`` go to positions ``pos ..
+    pos + t - 1`` of the caches, in one launch (``ftx_rope_cache``). None when the kernel does not take the
+    call."""
+    b, t, h, d = q.shape
+    kv = k.shape[2]
+    if (type(pos) is not int or pos < 0 or d % 16 or not q.numel() or not kernel_call(q, k, v, cache_k, cache_v)
+            or k.shape != (b, t, kv, d) or v.shape != k.shape or not _packed(q, k, v)):
+        return None
+    for table in (cos, sin):
+        if (type(table) not in _PLAIN_TYPES or table.dtype != torch.float32 or table.dim() != 2
+                or table.shape[1] != d or table.shape[0] < pos + t or table.device != q.device
+                or (table.requires_grad and torch.is_grad_enabled()) or not _packed(table)):
+            return None
+    for cache in (cache_k, cache_v):
+        if (cache.dim() != 4 or cache.shape[0] < b or cache.shape[1] < pos + t or cache.shape[2:] != (kv, d)
+                or not _strided_heads(cache) or 0 in cache.stride()):
+            return None
+    if cache_k.data_ptr() == cache_v.data_ptr():
+        return None
+    out = torch.empty_like(q)
+    strides = (ctypes.c_int64 * 6)(*_strides(cache_k), *_strides(cache_v))
+    nat.call("ftx_rope_cache", q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+             out.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), b, t, h, kv, d, pos, strides, _stream())
+    return out
+
+
+def silu_mul(g: torch.Tensor, u: torch.Tensor) -> torch.Tensor | None:
+    """``bf16(bf16(silu(g)) * u)`` in one launch (``ftx_silu_mul``), or None when the kernel does not take the
+    call."""
+    if g.shape != u.shape or not g.numel() or g.numel() % 8 or not kernel_call(g, u) or not _packed(g, u):
+        return None
+    y = torch.empty_like(g)
+    nat.call("ftx_silu_mul", g.data_ptr(), u.data_ptr(), y.data_ptr(), g.numel(), _stream())
+    return y
 
 
 FP8_DECODE_MAX_ROWS = 64  # more rows run the tiled prefill kernel

@@ -223,6 +223,9 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim, dtype=dtype))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        fused = hip.rms_norm(x, self.weight, self.eps)
+        if fused is not None:
+            return fused
         xf = x.float()
         y = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)
         return (y * self.weight.float()).to(x.dtype)
@@ -255,6 +258,10 @@ class Attention(nn.Module):
         q = q.view(b, t, s.n_heads, s.head_dim)
         k = k.view(b, t, s.n_kv_heads, s.head_dim)
         v = v.view(b, t, s.n_kv_heads, s.head_dim)
+        fused = hip.rope_cache(q, k, v, cos, sin, pos, cache_k, cache_v)
+        if fused is not None and hip.attention_eligible(fused, cache_k[:b, : pos + t], cache_v[:b, : pos + t]):
+            o = hip.attention(fused, cache_k[:b, : pos + t], cache_v[:b, : pos + t], pos)
+            return self._output(o.view(b, t, s.n_heads * s.head_dim), residual)
         c = cos[pos: pos + t].view(1, t, 1, -1).to(q.dtype)
         sn = sin[pos: pos + t].view(1, t, 1, -1).to(q.dtype)
         q, k = _rotate(q, c, sn), _rotate(k, c, sn)
@@ -276,6 +283,10 @@ class Attention(nn.Module):
             scores = scores.masked_fill(mask, float("-inf"))
         p = torch.softmax(scores, dim=-1).to(vh.dtype)
         o = torch.matmul(p, vh).transpose(1, 2).reshape(b, t, s.n_heads * s.head_dim)
+        return self._output(o, residual)
+
+    def _output(self, o: torch.Tensor, residual: torch.Tensor | None) -> torch.Tensor:
+        """The output projection of ``o``, plus ``residual`` when given."""
         if residual is None:
             return self.wo(o)
         fused = fp8_residual(o, self.wo, residual)
@@ -300,7 +311,9 @@ class DecoderLayer(nn.Module):
         if act is None:
             gu = fp8_group(h, [self.gate, self.up])
             g, u = gu if gu is not None else (self.gate(h), self.up(h))
-            act = F.silu(g) * u
+            act = hip.silu_mul(g, u)
+            if act is None:
+                act = F.silu(g) * u
         out = fp8_residual(act, self.down, x)
         return out if out is not None else x + self.down(act)
 
@@ -405,11 +418,15 @@ WAN_DIT = DiTShape()
 def sdpa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
     """Attention over [batch, heads, seq, head_dim].
 
-    On the GPU only the fused flash / memory-efficient kernels are allowed (a
+    On the GPU bf16 heads of 64 or 128 values run the library's attention
+    kernel; other calls only torch's fused flash / memory-efficient kernels (a
     32760-token score matrix does not belong in HBM, and the unfused path runs
     batched products on transposed views); without a fused kernel this raises.
     """
     if q.device.type == "cuda":
+        heads = [t.transpose(1, 2) for t in (q, k, v)] if q.dim() == k.dim() == v.dim() == 4 else None
+        if heads is not None and q.shape[1] == k.shape[1] and hip.attention_eligible(*heads):
+            return hip.attention(*heads).transpose(1, 2)
         from torch.nn.attention import SDPBackend, sdpa_kernel
 
         with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):

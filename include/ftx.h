@@ -335,6 +335,58 @@ int ftx_fp8_linear_fused(const void *x, int group, const void *const *w, const v
 int ftx_fp8_linear_static(const void *x, const void *w, const void *scale, void *y, int64_t m, int64_t n, int64_t k,
                           void *stream);
 
+/* ---- a transformer layer around its matrix products ------------------------
+ * No reference counterpart: the reference streams weights for whatever modules
+ * the user's model holds and leaves their operations to PyTorch. These are the
+ * operations of a decoder layer and of a diffusion-transformer block, one
+ * launch each. bf16 storage, fp32 arithmetic; every pointer is 16-byte aligned
+ * device memory and every stride a multiple of 8 elements.
+ *
+ * Attention. o[b, t, h] = sum_s softmax_s(scale * q[b, t, h] . k[b, s, h / rep])
+ * v[b, s, h / rep], rep = heads / kv_heads, over vectors of d = 64 or 128
+ * values. strides holds twelve element strides: batch, position and head of
+ * q, k, v and o; the last dimension is contiguous, and one head's keys (and
+ * values) span less than 2^31 bytes. causal: query t sees keys 0 .. pos + t
+ * (pos >= 0; ignored otherwise). Scores and sums are fp32, probabilities bf16.
+ * workspace: ftx_attention_workspace bytes (0 unless the keys are split over
+ * workgroups). Empty batches and t = 0 launch nothing; s = 0 and a scale that is
+ * not positive are refused. */
+int ftx_attention_workspace(int64_t batch, int64_t t, int64_t s, int heads, int kv_heads, int d, size_t *bytes);
+int ftx_attention(const void *q, const void *k, const void *v, void *o, int64_t batch, int64_t t, int64_t s, int heads,
+                  int kv_heads, int d, const int64_t *strides, int causal, int64_t pos, float scale, void *workspace,
+                  size_t workspace_bytes, void *stream);
+
+/* Rows of dim values (a multiple of 8, at most 32768), contiguous:
+ *   x' = x, or bf16(x + delta), or bf16(x + delta * m[gate]) (gate >= 0);
+ *        stored to x_out when delta is given
+ *   y  = FTX_NORM_NONE   nothing
+ *        FTX_NORM_RMS    x' * rsqrt(mean(x'^2) + eps) * w
+ *        FTX_NORM_LAYER  (x' - mean) * rsqrt(var + eps) * w + b
+ *        FTX_NORM_ADALN  (x' - mean) * rsqrt(var + eps) * (1 + m[scale]) + m[shift]
+ * m[i] = mod[i] + e[row / rows_per_batch][i]: bf16 [6, dim] and [batch, 6, dim],
+ * added in fp32; needed when gate >= 0 or under FTX_NORM_ADALN. x_out may be x
+ * or delta. */
+#define FTX_NORM_NONE 0
+#define FTX_NORM_RMS 1
+#define FTX_NORM_LAYER 2
+#define FTX_NORM_ADALN 3
+int ftx_norm(const void *x, const void *delta, void *x_out, void *y, int64_t rows, int64_t dim, int norm,
+             const void *w, const void *b, const void *mod, const void *e, int64_t rows_per_batch, int gate, int scale,
+             int shift, float eps, void *stream);
+
+/* Rotary embedding and KV-cache write of t new positions: q and k [batch, t,
+ * heads or kv_heads, d] (contiguous, d a multiple of 16) are rotated by the
+ * fp32 tables cos and sin [>= pos + t, d] (halves against each other), q into
+ * q_out, k into cache_k at positions pos .. pos + t - 1; v is copied to
+ * cache_v. cache_strides: batch, position and head strides of cache_k, then of
+ * cache_v. The caches must not overlap each other or the inputs. */
+int ftx_rope_cache(const void *q, const void *k, const void *v, const void *cos, const void *sin, void *q_out,
+                   void *cache_k, void *cache_v, int64_t batch, int64_t t, int heads, int kv_heads, int d, int64_t pos,
+                   const int64_t *cache_strides, void *stream);
+
+/* y = bf16(bf16(silu(g)) * u) over n values (a multiple of 8). */
+int ftx_silu_mul(const void *g, const void *u, void *y, int64_t n, void *stream);
+
 /* ---- checksums (size-independent parity checks on device data) ----------- */
 /* Order-sensitive 64-bit checksum of nbytes at dev (FNV-1a over 8-byte lanes,
  * folded per 4 KiB block); result written to *out after stream sync. */

@@ -1,0 +1,241 @@
+"""The attention, norm, rotary and SwiGLU kernels against float64 restatements of the same operations.
+
+Tolerances are relative 2-norms of bf16 roundings: bf16 has eight significant bits, so a value rounded once (half a
+unit in the last place) is off by at most 2^-8 of itself, and an output whose last product's inputs were rounded as
+well (attention's probabilities) by at most 2^-7.
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ONE_ROUNDING = 2.0 ** -8
+TWO_ROUNDINGS = 2.0 ** -7
+
+
+def _rel(got: torch.Tensor, want: torch.Tensor) -> float:
+    return float((got.double() - want).norm() / want.norm())
+
+
+def _randn(gpu, *shape: int, seed: int = 0) -> torch.Tensor:
+    gen = torch.Generator(device=gpu).manual_seed(seed + sum(shape))
+    return torch.randn(*shape, device=gpu, generator=gen).to(torch.bfloat16)
+
+
+def _attend64(q, k, v, pos):
+    b, t, h, d = q.shape
+    rep = h // k.shape[2]
+    q, k, v = (x.double().cpu() for x in (q, k, v))
+    out = torch.empty_like(q)
+    mask = torch.ones(t, k.shape[1], dtype=torch.bool).triu(pos + 1) if pos is not None else None
+    for i in range(b):
+        for j in range(h):
+            s = q[i, :, j] @ k[i, :, j // rep].t() / math.sqrt(d)
+            if mask is not None:
+                s = s.masked_fill(mask, float("-inf"))
+            out[i, :, j] = torch.softmax(s, -1) @ v[i, :, j // rep]
+    return out
+
+
+# batch, queries, keys, heads, kv heads, d, position of the first query (None: every key is seen).
+_ATTENTION = [
+    (1, 1, 1, 1, 1, 128, 0), (2, 1, 31, 4, 4, 64, 30), (1, 1, 528, 32, 32, 128, 527), (8, 1, 1024, 64, 8, 128, 1023),
+    (3, 1, 97, 10, 2, 128, 96), (1, 2, 65, 8, 1, 64, 63),  # one wave, split over the keys or not
+    (1, 7, 200, 8, 2, 128, 193), (1, 33, 33, 2, 2, 128, 0), (1, 100, 612, 8, 8, 64, 512),  # splits of causal rows
+    (2, 64, 64, 256, 32, 128, 0), (4, 40, 40, 64, 64, 64, 0), (4, 127, 127, 64, 64, 128, 0),  # 2 and 4 waves
+    (1, 257, 257, 128, 64, 128, 0), (1, 300, 301, 128, 128, 64, 1), (1, 512, 512, 128, 128, 128, 0),  # 8 waves
+    (1, 64, 16, 4, 4, 128, None), (1, 200, 77, 40, 40, 128, None), (2, 520, 129, 64, 64, 64, None),
+    (1, 1030, 1027, 64, 64, 128, None),
+]
+
+
+@pytest.mark.parametrize("b,t,s,h,kv,d,pos", _ATTENTION)
+def test_attention_matches_float64(gpu, b, t, s, h, kv, d, pos):
+    """Queries, a longer KV cache and a head-major layout are read in place; the keys past the last one hold
+    infinities, which must not reach the result."""
+    from flextensor_amd import hip
+
+    print(f"attention b={b} t={t} s={s} h={h}/{kv} d={d} pos={pos}", flush=True)
+    q = _randn(gpu, b, t, h, d)
+    cache_k, cache_v = _randn(gpu, b, s + 5, kv, d, seed=1), _randn(gpu, b, s + 5, kv, d, seed=2)
+    cache_k[:, s:], cache_v[:, s:] = float("inf"), float("inf")
+    k, v = cache_k[:, :s], cache_v[:, :s]
+    want = _attend64(q, k, v, pos)
+    assert hip.attention_eligible(q, k, v)
+    got = hip.attention(q, k, v, pos)
+    assert got.is_contiguous() and _rel(got.cpu(), want) < TWO_ROUNDINGS
+    head_major = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in (q, k, v)]
+    got = hip.attention(*head_major, pos)
+    assert got.stride() == head_major[0].stride() and _rel(got.cpu(), want) < TWO_ROUNDINGS
+
+
+def test_attention_with_large_scores_and_rising_maxima(gpu):
+    """Keys that grow along the sequence raise the maximum at every tile; scores reach the hundreds."""
+    from flextensor_amd import hip
+
+    q, k, v = (_randn(gpu, 1, 300, 4, 128, seed=i) for i in range(3))
+    k = (k.float() * torch.linspace(0.1, 12.0, 300, device=gpu).view(1, -1, 1, 1)).to(torch.bfloat16)
+    for pos in (None, 0):
+        assert _rel(hip.attention(q, k, v, pos).cpu(), _attend64(q, k, v, pos)) < TWO_ROUNDINGS
+
+
+def test_attention_passes_nan_and_infinite_scores_on(gpu):
+    """A NaN query row gives NaN in its row only, as softmax does; other rows are untouched."""
+    from flextensor_amd import hip
+
+    q, k, v = (_randn(gpu, 1, 40, 2, 128, seed=i) for i in range(3))
+    clean = hip.attention(q, k, v)
+    q[0, 5, 1] = float("nan")
+    got = hip.attention(q, k, v)
+    assert bool(got[0, 5, 1].isnan().all())
+    got[0, 5, 1] = clean[0, 5, 1]
+    assert torch.equal(got, clean)
+    k[0, 7, 0] = float("inf")  # scores of both signs: infinite, so NaN or a weight of one or zero, as in torch
+    s = torch.softmax((q[0, :, 0].double() @ k[0, :, 0].double().t()), -1)
+    assert torch.equal(hip.attention(q, k, v)[0, :, 0].isnan().all(-1), s.isnan().any(-1))
+
+
+def test_attention_refuses_what_the_kernel_cannot_address(gpu):
+    from flextensor_amd import _native as nat
+    from flextensor_amd import hip
+
+    q = _randn(gpu, 1, 8, 4, 128)
+    assert not hip.attention_eligible(q, q[..., 1:], q[..., 1:])
+    assert not hip.attention_eligible(q.float(), q.float(), q.float())
+    assert not hip.attention_eligible(q[..., :96].contiguous(), q[..., :96].contiguous(), q[..., :96].contiguous())
+    assert not hip.attention_eligible(q, q[:, :0], q[:, :0])
+    shifted = torch.empty(q.numel() + 4, dtype=torch.bfloat16, device=gpu)[4:].view_as(q)
+    assert not hip.attention_eligible(shifted, q, q)
+    with pytest.raises(nat.FtxError, match="head dimensions"):
+        hip.attention(*[q[..., :96].contiguous()] * 3)
+    with pytest.raises(nat.FtxError, match="no keys"):
+        hip.attention(q, q[:, :0], q[:, :0])
+
+
+@pytest.mark.parametrize("rows", [1, 5, 513])
+@pytest.mark.parametrize("dim", [8, 200, 2048, 2056, 5120, 8192, 8200, 32768])
+def test_rms_norm_matches_float64(gpu, rows, dim):
+    from flextensor_amd import workloads as W
+
+    x, w = _randn(gpu, rows, dim), _randn(gpu, dim, seed=1)
+    norm = W.RMSNorm(dim, 1e-5, torch.bfloat16).to(gpu)
+    with torch.no_grad():
+        norm.weight.copy_(w)
+        got = norm(x)
+    xd = x.double()
+    want = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert _rel(got, want) < ONE_ROUNDING
+
+
+@pytest.mark.parametrize("b,t,h,kv,d,pos", [(1, 1, 1, 1, 16, 0), (2, 3, 8, 2, 64, 5), (1, 65, 5, 5, 128, 0), (3, 1, 64, 8, 128, 40)])
+def test_rope_cache_matches_float64(gpu, b, t, h, kv, d, pos):
+    """Rotated queries, and keys and values at their positions; the rest of the caches is left alone."""
+    from flextensor_amd import hip
+
+    q, k, v = _randn(gpu, b, t, h, d), _randn(gpu, b, t, kv, d, seed=1), _randn(gpu, b, t, kv, d, seed=2)
+    ang = torch.rand(pos + t + 2, d, device=gpu, generator=torch.Generator(device=gpu).manual_seed(3)) * 6.3
+    cos, sin = ang.cos(), ang.sin()
+    ck, cv = torch.full((2, b + 1, pos + t + 3, kv, d), 7.0, dtype=torch.bfloat16, device=gpu)
+    got = hip.rope_cache(q, k, v, cos, sin, pos, ck, cv)
+
+    def rotate(x):
+        x = x.double()
+        half = d // 2
+        c, s = (a[pos: pos + t].double().view(1, t, 1, d) for a in (cos, sin))
+        return x * c + torch.cat((-x[..., half:], x[..., :half]), -1) * s
+
+    assert _rel(got, rotate(q)) < ONE_ROUNDING
+    assert _rel(ck[:b, pos: pos + t], rotate(k)) < ONE_ROUNDING
+    assert torch.equal(cv[:b, pos: pos + t], v)
+    for c in (ck, cv):
+        assert bool((c[:b, :pos] == 7).all()) and bool((c[:b, pos + t:] == 7).all()) and bool((c[b:] == 7).all())
+    assert hip.rope_cache(q, k, v, cos, sin, pos + 3, ck, cv) is None  # past the tables: torch raises for these
+    assert hip.rope_cache(q, k, v, cos, sin, pos, ck[:, : pos], cv) is None
+
+
+@pytest.mark.parametrize("n", [8, 2040, 2056, 1 << 20])
+def test_silu_mul_matches_float64(gpu, n):
+    from flextensor_amd import hip
+
+    g, u = _randn(gpu, n), _randn(gpu, n, seed=1)
+    gd = g.double()
+    want = (gd / (1 + torch.exp(-gd))).to(torch.bfloat16).double() * u.double()
+    assert _rel(hip.silu_mul(g, u), want) < TWO_ROUNDINGS
+    assert hip.silu_mul(g[1:], u[1:]) is None
+
+
+def test_operations_that_must_be_seen_run_in_torch(gpu):
+    """Autograd, forward-mode differentiation, function and dispatch modes, functorch transforms and autocast get
+    torch's operations; a plain call gets the kernel."""
+    import torch.autograd.forward_ad as fwd
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from flextensor_amd import hip
+    from flextensor_amd import workloads as W
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    norm = W.RMSNorm(64, 1e-5, torch.bfloat16).to(gpu)
+    x = _randn(gpu, 4, 64)
+    with torch.no_grad():
+        assert hip.rms_norm(x, norm.weight, 1e-5) is not None
+        for mode in (Function(), Dispatch(), torch.autocast("cuda", dtype=torch.bfloat16)):
+            with mode:
+                assert hip.rms_norm(x, norm.weight, 1e-5) is None
+        with fwd.dual_level():
+            dual = fwd.make_dual(x, torch.ones_like(x))
+            assert fwd.unpack_dual(norm(dual)).tangent is not None
+        assert torch.func.vmap(norm)(x.view(2, 2, 64)).shape == (2, 2, 64)
+    assert hip.rms_norm(x, norm.weight, 1e-5) is None
+    y = norm(x.requires_grad_())
+    y.float().sum().backward()
+    assert x.grad is not None and norm.weight.grad is not None
+
+
+def test_decoder_layer_kernels_against_torch_operations(gpu, monkeypatch):
+    """A small decoder's prompt and a decode step, with the kernels and with each call refused, against each
+    other and captured in a graph."""
+    from flextensor_amd import hip
+    from flextensor_amd import workloads as W
+
+    s = W.LlamaShape(n_layers=2, hidden=256, n_heads=4, n_kv_heads=2, head_dim=64, inter=512, vocab=300, max_seq=64)
+    model = W.build_llama(s, seed=1).to(gpu)
+    prompt = W.prompt_tokens(3, 17, s.vocab, seed=1).to(gpu)
+    tok = W.prompt_tokens(3, 1, s.vocab, seed=2).to(gpu)
+
+    def passes():
+        model.init_cache(3, 40, torch.device(gpu))
+        with torch.no_grad():
+            return [model(prompt, 0), model(tok, 17)], [c.clone() for c in model.cache_k]
+
+    got, cache = passes()
+    with monkeypatch.context() as m:
+        m.setattr(hip, "kernel_call", lambda *ts: False)
+        want, want_cache = passes()
+    for a, b in zip(got + cache, want + want_cache):
+        assert _rel(a, b.double()) < 2e-2  # two bf16 layers
+    passes()
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.stream(side):
+        model(tok, 17)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            static = model(tok, 17)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(static, got[1])
+    del graph
