@@ -432,6 +432,36 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor 
     return y
 
 
+def residual_norm(x: torch.Tensor, eps: float, delta: torch.Tensor | None = None, gate: int = -1,
+                  affine: tuple[torch.Tensor, torch.Tensor] | None = None,
+                  adaln: tuple[torch.Tensor, torch.Tensor] | None = None, scale: int = -1,
+                  shift: int = -1) -> tuple[torch.Tensor, torch.Tensor | None] | None:
+    """``(sum, normalised)`` of bf16 [batch, n, dim] rows in one launch (``ftx_norm``), or None when the kernel
+    does not take the call.
+
+    The sum is ``x``, ``x + delta``, or ``x + delta * m[gate]``; the normalised rows (None for none of the two)
+    are its LayerNorm with ``affine`` (weight, bias), or ``LayerNorm(sum) * (1 + m[scale]) + m[shift]`` for a
+    ``scale`` that is not negative. ``m = modulation + e`` from ``adaln``: [1, 6, dim] and [batch, 6, dim].
+    """
+    if x.dim() != 3 or not x.numel():
+        return None
+    b, n, dim = x.shape
+    tensors = [t for t in (x, delta, *(affine or ()), *(adaln or ())) if t is not None]
+    if (dim % 8 or dim > NORM_MAX_DIM or b * n >= 1 << 31 or not kernel_call(*tensors) or not _packed(*tensors)
+            or (delta is not None and delta.shape != x.shape)
+            or (affine is not None and not affine[0].shape == affine[1].shape == (dim,))
+            or (adaln is not None and (adaln[0].shape != (1, 6, dim) or adaln[1].shape != (b, 6, dim)))):
+        return None
+    norm = nat.NORM_ADALN if scale >= 0 else nat.NORM_LAYER if affine is not None else nat.NORM_NONE
+    total = torch.empty_like(x) if delta is not None else x
+    y = torch.empty_like(x) if norm != nat.NORM_NONE else None
+    ptr = [t.data_ptr() if t is not None else None for t in (delta, total, y, *(affine or (None, None)),
+                                                             *(adaln or (None, None)))]
+    nat.call("ftx_norm", x.data_ptr(), ptr[0], ptr[1], ptr[2], b * n, dim, norm, ptr[3], ptr[4], ptr[5], ptr[6], n,
+             gate, scale, shift, eps, _stream())
+    return total, y
+
+
 def rope_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: int,
                cache_k: torch.Tensor, cache_v: torch.Tensor) -> torch.Tensor | None:
     """The rotated queries of [batch, t, head, d] ``q``; the rotated ``k`` and ``v`` go to positions ``pos ..

@@ -471,14 +471,38 @@ class DiTBlock(nn.Module):
     def _norm(self, x: torch.Tensor) -> torch.Tensor:
         return F.layer_norm(x.float(), (self.s.dim,), eps=self.s.eps).to(x.dtype)
 
+    def _modulate(self, x: torch.Tensor, m: torch.Tensor, scale: int, shift: int) -> torch.Tensor:
+        return (self._norm(x).float() * (1 + m[:, scale: scale + 1]) + m[:, shift: shift + 1]).to(x.dtype)
+
     def forward(self, x: torch.Tensor, e: torch.Tensor, ctx: torch.Tensor, attn=None) -> torch.Tensor:
-        m = (self.modulation.float() + e.float()).chunk(6, dim=1)
-        h = (self._norm(x).float() * (1 + m[1]) + m[0]).to(x.dtype)
-        x = (x.float() + self.self_attn(h, h, attn).float() * m[2]).to(x.dtype)
-        x = x + self.cross_attn(self.norm3(x), ctx, attn)
-        h = (self._norm(x).float() * (1 + m[4]) + m[3]).to(x.dtype)
+        """Each residual add and the norm that reads its sum are one launch where the kernel takes the call."""
+        adaln = (self.modulation, e)
+        eps = self.s.eps
+
+        def m() -> torch.Tensor:
+            return self.modulation.float() + e.float()
+
+        fused = hip.residual_norm(x, eps, adaln=adaln, scale=1, shift=0)
+        h = fused[1] if fused is not None else self._modulate(x, m(), 1, 0)
+        y = self.self_attn(h, h, attn)
+        n3 = self.norm3
+        plain = type(n3) is nn.LayerNorm and _plain_call(n3)
+        fused = hip.residual_norm(x, n3.eps, y, 2, (n3.weight, n3.bias), adaln) if plain else None
+        if fused is not None:
+            x, h = fused
+        else:
+            x = (x.float() + y.float() * m()[:, 2:3]).to(x.dtype)
+            h = n3(x)
+        y = self.cross_attn(h, ctx, attn)
+        fused = hip.residual_norm(x, eps, y, adaln=adaln, scale=4, shift=3)
+        if fused is not None:
+            x, h = fused
+        else:
+            x = x + y
+            h = self._modulate(x, m(), 4, 3)
         y = self.fc2(F.gelu(self.fc1(h), approximate="tanh"))
-        return (x.float() + y.float() * m[5]).to(x.dtype)
+        fused = hip.residual_norm(x, eps, y, 5, adaln=adaln)
+        return fused[0] if fused is not None else (x.float() + y.float() * m()[:, 5:6]).to(x.dtype)
 
 
 class DiTModel(nn.Module):

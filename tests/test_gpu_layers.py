@@ -132,6 +132,35 @@ def test_rms_norm_matches_float64(gpu, rows, dim):
     assert _rel(got, want) < ONE_ROUNDING
 
 
+@pytest.mark.parametrize("b,n,dim", [(1, 1, 8), (2, 3, 512), (1, 9, 2056), (3, 5, 5120), (1, 2, 16384)])
+@pytest.mark.parametrize("residual", ["none", "add", "gated"])
+@pytest.mark.parametrize("norm", ["none", "affine", "adaln"])
+def test_residual_norm_matches_float64(gpu, b, n, dim, residual, norm):
+    """The sum rounds once; the norm of the sum as stored rounds once more."""
+    from flextensor_amd import hip
+
+    x, delta = _randn(gpu, b, n, dim) + 0.5, _randn(gpu, b, n, dim, seed=1)
+    w, bias = _randn(gpu, dim, seed=2), _randn(gpu, dim, seed=3)
+    mod, e = _randn(gpu, 1, 6, dim, seed=4), _randn(gpu, b, 6, dim, seed=5)
+    total, y = hip.residual_norm(x, 1e-6, None if residual == "none" else delta, 2 if residual == "gated" else -1,
+                                 (w, bias) if norm == "affine" else None, (mod, e),
+                                 *((4, 3) if norm == "adaln" else ()))
+    m = mod.double() + e.double()
+    want = x.double()
+    if residual != "none":
+        want = want + delta.double() * (m[:, 2:3] if residual == "gated" else 1)
+    assert _rel(total, want) < ONE_ROUNDING
+    if norm == "none":
+        assert y is None
+        return
+    u = total.double()
+    u = u - u.mean(-1, keepdim=True)
+    u = u * torch.rsqrt(u.pow(2).mean(-1, keepdim=True) + 1e-6)
+    want = u * w.double() + bias.double() if norm == "affine" else u * (1 + m[:, 4:5]) + m[:, 3:4]
+    assert _rel(y, want) < ONE_ROUNDING
+    assert hip.residual_norm(x, 1e-6, delta[:, :, : dim // 2], adaln=(mod, e)) is None
+
+
 @pytest.mark.parametrize("b,t,h,kv,d,pos", [(1, 1, 1, 1, 16, 0), (2, 3, 8, 2, 64, 5), (1, 65, 5, 5, 128, 0), (3, 1, 64, 8, 128, 40)])
 def test_rope_cache_matches_float64(gpu, b, t, h, kv, d, pos):
     """Rotated queries, and keys and values at their positions; the rest of the caches is left alone."""
