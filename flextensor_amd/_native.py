@@ -160,6 +160,8 @@ _SIGNATURES: dict[str, list] = {
     "ftx_expcode_decode_d2d": [_vp, _vp, _sz, _sz, ctypes.c_int, _vp],
     "ftx_expcode_encode_dense": [_vp, _sz, _vp, _sz, ctypes.POINTER(_sz)],
     "ftx_expcode_decode_dense_d2d": [_vp, _vp, _sz, _sz, ctypes.c_int, _vp],
+    "ftx_fp8_linear_scratch": [ctypes.c_int64, _vp, _int, ctypes.c_int64, _int, ctypes.POINTER(_sz)],
+    "ftx_bf16_linear": [_vp, _int, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64, _int, _vp, _vp],
     "ftx_attention_workspace": [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _int, _int, _int, ctypes.POINTER(_sz)],
     "ftx_attention": [_vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _int, _int, _int, _vp, _int,
                       ctypes.c_int64, ctypes.c_float, _vp, _sz, _vp],

@@ -86,6 +86,8 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
   return static_cast<uint16_t>(u >> 16);
 }
 
+__device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
+
 // Bytes of one weight row loaded per iteration: 16 lanes x 16 bytes, so one
 // load instruction covers 4 rows x 256 contiguous bytes. Fewer, longer runs
 // per instruction keep HBM near its streaming rate; the MFMA layout (16 rows
@@ -277,8 +279,6 @@ constexpr int kReduceThreads = 256;
 // took 45 us (median) against 5 us alone, the q/k/v reduce 26 against 5.
 constexpr unsigned kReduceLdsToken = 512;
 
-__device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
-
 // Sum over slices of kReduceVec consecutive partials starting at i0 (fewer at the end of MN).
 __device__ __forceinline__ void sum_slices(const float *__restrict__ p, int64_t MN, int64_t i0, int splits,
                                            float (&acc)[kReduceVec]) {
@@ -345,10 +345,201 @@ __global__ __launch_bounds__(kReduceThreads) void fp8_linear_reduce_kernel(const
   }
 }
 
+// ---- a few rows: one launch, no partial sums in memory ----------------------
+//
+// One workgroup of eight waves owns 16 output channels over the whole of K. The waves take turns along K
+// (wave w the 256-byte windows w, w + 8, ... of every row), so the workgroup streams whole rows, and their
+// sums meet in LDS in wave order at the end, where the epilogue is applied. Against the split-K kernel this
+// saves the partial sums' trip through memory and the reduce launch that reads them (3.5 to 5 us a call).
+// Under SwiGLU a workgroup owns the same 16 channels of gate and of up.
+//
+// Weights and the window of x that meets them go through per-wave LDS tiles, as the weights do in
+// fp8_linear_kernel: loads cover whole rows and MFMA operands are read back in their layout. Weights are e4m3
+// (with a scale per channel) or bf16 (without): a 256-byte window is 256 or 128 values of k, a 64-byte step
+// two MFMAs or one. Two windows are in flight per wave and two workgroups fit a CU; 32 channels per
+// workgroup read x half as often but need 140 registers, one workgroup per CU (28672 x 8192 fp8 in 57
+// against 41 us).
+//
+// The sum's order depends on K alone, not on the grouping or on M: a projection gives the same bits on its
+// own and in a group.
+//
+// Bound by the weight bytes. Measured in a row on distinct weights, us: fp8 at 1 / 8 rows, before (split-K
+// and reduce) and here: 1024 x 8192 7.7 / 8.6 and 6.6 / 8.2, 4096 x 4096 8.8 / 10.0 and 6.7 / 7.2,
+// 28672 x 8192 44.0 / 48.5 and 41.5 / 45.6 (5.7 TB/s); bf16 at 1 row, the library's GEMM and here:
+// 4096 x 4096 15.4 and 8.4, 11008 x 4096 26.8 and 19.2, 4096 x 11008 38.1 and 18.9, 8192 x 28672 87.6 and 75.0.
+constexpr int kDirectWaves = 8;
+
+// XL loads of 1 KB bring a window of x: 2 XL rows of 512 bytes (fp8) or 4 XL rows of 256 (bf16).
+template <bool FP8, int XL, bool SWIGLU>
+__global__ __launch_bounds__(kDirectWaves * kWave) void direct_linear_kernel(const uint8_t *__restrict__ x,
+                                                                             SegTable seg, int M, int K,
+                                                                             const uint16_t *__restrict__ residual) {
+  constexpr int kWindowX = FP8 ? 2 * kIterK : kIterK;  // bytes of a row of x in one window
+  constexpr int kXLanes = kWindowX / 16;               // lanes that load one row of it
+  constexpr int kXRows = XL * kWave / kXLanes;
+  constexpr int kXRow = kWindowX + 16;
+  constexpr int kWaveBytes = kTileBytes + kXRows * kXRow;
+  constexpr int kMatrices = SWIGLU ? 2 : 1;
+  static_assert(kWaveBytes >= kMatrices * 256 * 4, "the waves' sums fit where the tiles were");
+  __shared__ __align__(16) uint8_t lds[kDirectWaves * kWaveBytes];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  int s = 0;
+  while (s + 1 < seg.count && static_cast<int>(blockIdx.x) >= seg.rg0[s + 1]) ++s;
+  const int N = seg.n[s];
+  const int n0 = (blockIdx.x - seg.rg0[s]) * 16;
+  const int64_t row_bytes = FP8 ? K : 2 * static_cast<int64_t>(K);
+  const int64_t x_bytes = 2 * static_cast<int64_t>(K);
+
+  const int lrow = lane >> 4;
+  const int lcol = (lane & 15) * kPieceBytes;
+  int64_t row_at[kLoads];  // rows past N read the last row
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) row_at[j] = min(n0 + j * kRowsPerLoad + lrow, N - 1) * row_bytes + lcol;
+  const int xrow = lane / kXLanes;
+  const int xcol = lane % kXLanes * 16;
+  const uint8_t *xp = x + xrow * x_bytes + xcol;
+  const int windows = static_cast<int>((row_bytes + kIterK - 1) / kIterK);
+
+  // Pieces that start at or past the end of the row read as zero (rows are whole pieces).
+  auto load_w = [&](u32x4(&v)[kLoads], const uint8_t *w, int win) {
+    const int64_t at = static_cast<int64_t>(win) * kIterK;
+    const bool ok = at + lcol < row_bytes;
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j)
+      v[j] = ok ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w + row_at[j] + at)) : u32x4{0u, 0u, 0u, 0u};
+  };
+  auto load_x = [&](u32x4(&v)[XL], int win) {
+    const int64_t at = static_cast<int64_t>(win) * kWindowX;
+#pragma unroll
+    for (int j = 0; j < XL; ++j) {
+      const int m = j * (kWave / kXLanes) + xrow;
+      v[j] = m < M && at + xcol < x_bytes
+                 ? *reinterpret_cast<const u32x4 *>(xp + j * (kWave / kXLanes) * x_bytes + at)
+                 : u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  uint8_t *tile = lds + wave * kWaveBytes;
+  uint8_t *xt = tile + kTileBytes;
+  // this lane's column of x: row r (columns past those loaded repeat the last one and are not stored)
+  const uint8_t *xcolumn = xt + min(r, kXRows - 1) * kXRow + g * (FP8 ? 32 : 16);
+  // Tiles are written and read back by different lanes of this wave: order each side's accesses explicitly.
+  auto order = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto stage_x = [&](const u32x4(&v)[XL]) {
+#pragma unroll
+    for (int j = 0; j < XL; ++j)
+      *reinterpret_cast<u32x4 *>(xt + (j * (kWave / kXLanes) + xrow) * kXRow + xcol) = v[j];
+  };
+  auto multiply = [&](const u32x4(&v)[kLoads], f32x4 &acc) {
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j)
+      *reinterpret_cast<u32x4 *>(tile + (j * kRowsPerLoad + lrow) * kTileRow + lcol) = v[j];
+    order();
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) {
+      const u32x4 a = *reinterpret_cast<const u32x4 *>(tile + r * kTileRow + st * kStepBytes + g * kPieceBytes);
+      const u32x4 *xv = reinterpret_cast<const u32x4 *>(xcolumn + st * (kWindowX / kSteps));
+      if (FP8) {
+        bf16x8 lo, hi;
+        fp8x16_to_bf16(a, lo, hi);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, as_bf16x8(xv[0]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, as_bf16x8(xv[1]), acc, 0, 0, 0);
+      } else {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(xv[0]), acc, 0, 0, 0);
+      }
+    }
+    order();
+  };
+
+  f32x4 acc[kMatrices];
+#pragma unroll
+  for (int b = 0; b < kMatrices; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint8_t *w = seg.w[s];
+  u32x4 wa[kLoads], wb[kLoads], xa[XL], xb[XL];
+  if (SWIGLU) {  // a window of gate and the same one of up in flight; x serves both
+    const uint8_t *up = seg.w[1];
+    if (wave < windows) {
+      load_w(wa, w, wave);
+      load_x(xa, wave);
+      load_w(wb, up, wave);
+    }
+    for (int win = wave; win < windows; win += kDirectWaves) {
+      const bool more = win + kDirectWaves < windows;
+      stage_x(xa);
+      multiply(wa, acc[0]);
+      if (more) {
+        load_w(wa, w, win + kDirectWaves);
+        load_x(xa, win + kDirectWaves);
+      }
+      multiply(wb, acc[kMatrices - 1]);
+      if (more) load_w(wb, up, win + kDirectWaves);
+    }
+  } else {
+    if (wave < windows) {
+      load_w(wa, w, wave);
+      load_x(xa, wave);
+    }
+    if (wave + kDirectWaves < windows) {
+      load_w(wb, w, wave + kDirectWaves);
+      load_x(xb, wave + kDirectWaves);
+    }
+    for (int win = wave; win < windows; win += 2 * kDirectWaves) {
+      stage_x(xa);
+      multiply(wa, acc[0]);
+      if (win + 2 * kDirectWaves < windows) {
+        load_w(wa, w, win + 2 * kDirectWaves);
+        load_x(xa, win + 2 * kDirectWaves);
+      }
+      if (win + kDirectWaves < windows) {
+        stage_x(xb);
+        multiply(wb, acc[0]);
+        if (win + 3 * kDirectWaves < windows) {
+          load_w(wb, w, win + 3 * kDirectWaves);
+          load_x(xb, win + 3 * kDirectWaves);
+        }
+      }
+    }
+  }
+
+  // Lane l holds channels 4 (l / 16) .. + 3 of column l % 16 of each matrix.
+  __syncthreads();  // the last tiles have been read
+  float *sums = reinterpret_cast<float *>(lds);  // [wave][matrix][column][channel]
+#pragma unroll
+  for (int b = 0; b < kMatrices; ++b)
+    *reinterpret_cast<f32x4 *>(sums + ((wave * kMatrices + b) * 16 + r) * 16 + 4 * g) = acc[b];
+  __syncthreads();
+  const int t = threadIdx.x;
+  const int m = t / 16;
+  const int n = n0 + t % 16;
+  if (m >= M || n >= N) return;
+  auto output = [&](int matrix, int at) {  // M <= 16, so t < 256
+    float v = 0.f;
+#pragma unroll
+    for (int q = 0; q < kDirectWaves; ++q) v += sums[q * kMatrices * 256 + at];
+    return f32_to_bf16_bits(FP8 ? v * bf16_bits_to_f32(seg.scale[matrix][n]) : v);
+  };
+  const int64_t i = static_cast<int64_t>(m) * N + n;
+  if (SWIGLU) {  // the epilogues round as fp8_linear_reduce_kernel's do
+    const float gate = bf16_bits_to_f32(output(0, t));
+    const float up = bf16_bits_to_f32(output(1, t + 256));
+    const float act = bf16_bits_to_f32(f32_to_bf16_bits(gate / (1.0f + expf(-gate))));
+    seg.y[0][i] = f32_to_bf16_bits(act * up);
+    return;
+  }
+  const uint16_t out = output(s, t);
+  seg.y[s][i] = residual ? f32_to_bf16_bits(bf16_bits_to_f32(residual[i]) + bf16_bits_to_f32(out)) : out;
+}
+
 SegTable seg_table(const Fp8LinearLaunch &p) {
   SegTable t{};
   t.count = p.group;
-  const int64_t rows = p.prefill ? kPTileN : 16 * static_cast<int64_t>(p.waves);
+  const int64_t rows = p.prefill ? kPTileN : 16 * static_cast<int64_t>(p.waves);  // of one workgroup
   int rg = 0, rb = 0;
   int64_t off = 0;
   for (int s = 0; s < p.group; ++s) {
@@ -821,6 +1012,26 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
   return p;
 }
 
+// Where the one-launch kernel is the faster one. Its workgroups read all of x from L2, M / 8 bytes per fp8
+// weight, which the split-K kernel's 128-channel workgroups do not. Up to 4 rows it always wins (above). Of
+// 5 to 8 rows it loses where K is long and N does not make up for it: 8192 x 28672 at 8 rows in 48.1 us
+// against 45.1, 4096 x 11008 in 13.5 against 15.9. From 9 to 16 rows it wins on small matrices only: at 16
+// rows 4096 x 11008 in 15.6 against 20.0, 11008 x 4096 in 19.6 against 19.8, 8192 x 28672 in 64 against 62.
+// bf16 weights are twice the bytes for the same x, and the library's GEMM takes longer at every size.
+bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k) {
+  if (m <= 4) return true;
+  return m <= 8 ? k <= 16384 : m <= kDirectMaxRows && n_total * k <= int64_t(48) << 20;
+}
+
+void plan_direct_linear(Fp8LinearLaunch *p) {
+  p->direct = true;
+  p->splits = 1;
+  p->waves = 1;  // blocks of 16 channels per workgroup
+  p->row_groups = 0;
+  for (int s = 0; s < p->group; ++s) p->row_groups += (p->n[s] + 15) / 16;
+  p->grid = p->row_groups;
+}
+
 hipError_t launch_mfma_probe(int shape, int workgroups, int iters, float *sink, hipStream_t stream) {
   if (shape == kMfmaProbe32x32x16)
     hipLaunchKernelGGL(mfma_probe_32x32_kernel, dim3(static_cast<unsigned>(workgroups)), dim3(256), 0, stream, sink,
@@ -831,7 +1042,33 @@ hipError_t launch_mfma_probe(int shape, int workgroups, int iters, float *sink, 
   return hipGetLastError();
 }
 
+template <bool FP8, int XL>
+hipError_t launch_direct_rows(const Fp8LinearLaunch &p, hipStream_t stream) {
+  const SegTable seg = seg_table(p);
+  const auto *x = static_cast<const uint8_t *>(p.x);
+  const auto *residual = p.epilogue == kFp8EpilogueResidual ? static_cast<const uint16_t *>(p.residual) : nullptr;
+  const dim3 block(kDirectWaves * kWave);
+  const int m = static_cast<int>(p.m), k = static_cast<int>(p.k);
+  if (p.epilogue == kFp8EpilogueSwiglu)  // the grid covers the channels of one matrix
+    hipLaunchKernelGGL((direct_linear_kernel<FP8, XL, true>), dim3(static_cast<unsigned>(seg.rg0[1])), block, 0, stream,
+                       x, seg, m, k, residual);
+  else
+    hipLaunchKernelGGL((direct_linear_kernel<FP8, XL, false>), dim3(static_cast<unsigned>(seg.rg0[p.group])), block, 0,
+                       stream, x, seg, m, k, residual);
+  return hipGetLastError();
+}
+
+hipError_t launch_direct(const Fp8LinearLaunch &p, hipStream_t stream) {
+  if (p.bf16) {
+    if (p.m <= 4) return launch_direct_rows<false, 1>(p, stream);
+    return p.m <= 8 ? launch_direct_rows<false, 2>(p, stream) : launch_direct_rows<false, 4>(p, stream);
+  }
+  if (p.m <= 2) return launch_direct_rows<true, 1>(p, stream);
+  return p.m <= 8 ? launch_direct_rows<true, 4>(p, stream) : launch_direct_rows<true, 8>(p, stream);
+}
+
 hipError_t launch_fp8_linear(const Fp8LinearLaunch &p, hipStream_t stream) {
+  if (p.direct) return launch_direct(p, stream);
   if (p.prefill) {
     const SegTable seg = seg_table(p);
     // 32-bit load offsets reach every byte of x and of each weight matrix (kept under 2^31, so they read

@@ -88,7 +88,13 @@ struct Fp8LinearLaunch {
   bool prefill;       // more than kFp8LinearMaxRows rows: the tiled prefill kernel (no split, no workspace)
   int64_t m_tiles;    // prefill: tiles of 128 activation rows (row_groups then counts tiles of 128 channels)
   int xcds;           // prefill: L2 domains the block order is arranged for
+  bool direct;        // the one-launch decode kernel: no workspace, a workgroup per 16 channels
+  bool bf16;          // direct only: bf16 weights without scales
 };
+// The one-launch decode kernel: its most rows, whether it is the faster one for an fp8 call, and its plan.
+constexpr int kDirectMaxRows = 16;
+bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k);
+void plan_direct_linear(Fp8LinearLaunch *p);
 constexpr int kFp8LinearMaxRows = 64;
 constexpr size_t kFp8LinearMaxLds = 64 * 1024;
 Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t k, int cus, int xcds, int waves,

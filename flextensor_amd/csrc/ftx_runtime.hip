@@ -913,6 +913,14 @@ int ftx_set_fp8_linear_config(int waves, int slice_k) {
 
 namespace {
 
+// The checks that every operand of the layer operations shares: aligned device memory that holds its extent.
+int check_operand(const void *p, int64_t elements, int64_t item, const char *what) {
+  if (!p) return ftx::fail(FTX_ERR_INVALID, std::string(what) + " is null");
+  if (reinterpret_cast<uintptr_t>(p) % 16 != 0)
+    return ftx::fail(FTX_ERR_INVALID, std::string(what) + " needs 16-byte alignment");
+  return ftx::check_device_range(p, static_cast<size_t>(elements * item), what);
+}
+
 int plan_fp8(int64_t m, const int64_t *n, int group, int64_t k, ftx::Fp8LinearLaunch *p,
              int epilogue = ftx::kFp8EpilogueNone) {
   if (group < 1 || group > ftx::kFp8MaxGroup)
@@ -964,10 +972,20 @@ int plan_fp8(int64_t m, const int64_t *n, int group, int64_t k, ftx::Fp8LinearLa
   }
   *p = ftx::plan_fp8_linear(m, n, group, k, cus, xcds, waves, slice_k, epilogue);
   if (p->grid > (int64_t(1) << 31) - 1) return ftx::fail(FTX_ERR_INVALID, "fp8 linear grid too large");
+  if (!waves && !slice_k && ftx::direct_linear_wins(m, p->n_total, k)) ftx::plan_direct_linear(p);
   return FTX_OK;
 }
 
 }  // namespace
+
+int ftx_fp8_linear_scratch(int64_t m, const int64_t *n, int group, int64_t k, int epilogue, size_t *bytes) {
+  if (!bytes) return ftx::fail(FTX_ERR_INVALID, "bytes is null");
+  ftx::Fp8LinearLaunch p;
+  int rc = plan_fp8(m, n, group, k, &p, epilogue);
+  if (rc != FTX_OK) return rc;
+  *bytes = p.direct ? 0 : p.workspace_bytes;
+  return FTX_OK;
+}
 
 int ftx_fp8_linear_workspace(int64_t m, int64_t n, int64_t k, size_t *bytes) {
   return ftx_fp8_linear_group_workspace(m, &n, 1, k, bytes);
@@ -1023,7 +1041,7 @@ int run_fp8(ftx::Fp8LinearLaunch &p, const void *x, const void *const *w, const 
     int rc = ftx::check_device_range(p.residual, static_cast<size_t>(m * p.n[0] * 2), "fp8 linear residual");
     if (rc != FTX_OK) return rc;
   }
-  if (p.workspace_bytes > 0 && !static_workspace) {
+  if (p.workspace_bytes > 0 && !static_workspace && !p.direct) {
     if (!workspace || workspace_bytes < p.workspace_bytes)
       return ftx::fail(FTX_ERR_INVALID, "fp8 linear needs a workspace of " + std::to_string(p.workspace_bytes) +
                                             " bytes (ftx_fp8_linear_workspace)");
@@ -1081,6 +1099,72 @@ int ftx_fp8_linear_fused(const void *x, int group, const void *const *w, const v
   return run_fp8(p, x, w, scale, ys, workspace, workspace_bytes, false, stream);
 }
 
+int ftx_bf16_linear(const void *x, int group, const void *const *w, void *const *y, const int64_t *n, int64_t m,
+                    int64_t k, int epilogue, const void *residual, void *stream) {
+  FTX_REQUIRE_LIVE();
+  if (group < 1 || group > ftx::kFp8MaxGroup)
+    return ftx::fail(FTX_ERR_INVALID, "a grouped linear takes 1 to " + std::to_string(ftx::kFp8MaxGroup) +
+                                          " weight matrices");
+  if (!n || !w || !y) return ftx::fail(FTX_ERR_INVALID, "null pointer");
+  if (m < 0 || k < 0) return ftx::fail(FTX_ERR_INVALID, "negative dimension");
+  if (m > ftx::kDirectMaxRows)
+    return ftx::fail(FTX_ERR_UNSUPPORTED, "the bf16 linear runs up to " + std::to_string(ftx::kDirectMaxRows) + " rows");
+  if (k % 8 != 0) return ftx::fail(FTX_ERR_INVALID, "k must be a multiple of 8");
+  ftx::Fp8LinearLaunch p{};
+  for (int s = 0; s < group; ++s) {
+    if (n[s] < 0) return ftx::fail(FTX_ERR_INVALID, "negative dimension");
+    if (n[s] > (int64_t(1) << 30)) return ftx::fail(FTX_ERR_INVALID, "linear dimensions too large");
+    p.n[s] = n[s];
+    p.n_total += n[s];
+  }
+  if (p.n_total > (int64_t(1) << 30) || k > (int64_t(1) << 29))
+    return ftx::fail(FTX_ERR_INVALID, "linear dimensions too large");
+  if (epilogue == ftx::kFp8EpilogueSwiglu) {
+    if (group != 2 || n[0] != n[1])
+      return ftx::fail(FTX_ERR_INVALID, "the SwiGLU epilogue takes two matrices (gate, up) with the same n");
+  } else if (epilogue == ftx::kFp8EpilogueResidual) {
+    if (group != 1) return ftx::fail(FTX_ERR_INVALID, "the residual epilogue takes one matrix");
+  } else if (epilogue != ftx::kFp8EpilogueNone) {
+    return ftx::fail(FTX_ERR_INVALID, "unknown linear epilogue");
+  }
+  if (m == 0 || p.n_total == 0) return FTX_OK;
+  p.m = m;
+  p.k = k;
+  p.group = group;
+  p.epilogue = epilogue;
+  p.bf16 = true;
+  for (int s = 0; s < group; ++s) {
+    if (n[s] == 0) continue;
+    if (epilogue != ftx::kFp8EpilogueSwiglu || s == 0) {
+      if (!y[s] || reinterpret_cast<uintptr_t>(y[s]) % 2 != 0)
+        return ftx::fail(FTX_ERR_INVALID, "linear output is null or not 2-byte aligned");
+      int rc = ftx::check_device_range(y[s], static_cast<size_t>(m * n[s] * 2), "linear output");
+      if (rc != FTX_OK) return rc;
+      p.y[s] = y[s];
+    }
+    if (k > 0) {
+      int rc = check_operand(w[s], n[s] * k, 2, "linear weight");
+      if (rc != FTX_OK) return rc;
+    }
+    p.w[s] = w[s];
+  }
+  if (k > 0) {
+    int rc = check_operand(x, m * k, 2, "linear input");
+    if (rc != FTX_OK) return rc;
+  }
+  if (epilogue == ftx::kFp8EpilogueResidual) {
+    if (!residual || reinterpret_cast<uintptr_t>(residual) % 2 != 0)
+      return ftx::fail(FTX_ERR_INVALID, "the residual epilogue needs a 2-byte aligned residual");
+    int rc = ftx::check_device_range(residual, static_cast<size_t>(m * n[0] * 2), "linear residual");
+    if (rc != FTX_OK) return rc;
+  }
+  p.x = x;
+  p.residual = residual;
+  ftx::plan_direct_linear(&p);
+  FTX_HIP(ftx::launch_fp8_linear(p, static_cast<hipStream_t>(stream)));
+  return FTX_OK;
+}
+
 int ftx_fp8_linear_static(const void *x, const void *w, const void *scale, void *y, int64_t m, int64_t n, int64_t k,
                           void *stream) {
   FTX_REQUIRE_LIVE();
@@ -1103,14 +1187,6 @@ int ftx_fp8_linear_static(const void *x, const void *w, const void *scale, void 
 }
 
 namespace {
-
-// The checks that every operand of a layer operation shares: aligned device memory that holds its extent.
-int check_operand(const void *p, int64_t elements, int64_t item, const char *what) {
-  if (!p) return ftx::fail(FTX_ERR_INVALID, std::string(what) + " is null");
-  if (reinterpret_cast<uintptr_t>(p) % 16 != 0)
-    return ftx::fail(FTX_ERR_INVALID, std::string(what) + " needs 16-byte alignment");
-  return ftx::check_device_range(p, static_cast<size_t>(elements * item), what);
-}
 
 // Elements from the first to the last of a [n0, n1, n2, d] view, or -1 for a stride that is negative, not a
 // multiple of 8 or beyond any memory.

@@ -515,6 +515,17 @@ def fp8_linear_workspace_bytes(m: int, n: int, k: int) -> int:
     return got
 
 
+def _fp8_scratch_bytes(m: int, ns: tuple[int, ...], k: int, epilogue: int) -> int:
+    """Bytes of workspace a call touches under the launch shape in force (cached per shape)."""
+    key = ("scratch", epilogue, m, k) + ns
+    got = _FP8_WORKSPACE.get(key)
+    if got is None:
+        b = ctypes.c_size_t(0)
+        nat.call("ftx_fp8_linear_scratch", m, (ctypes.c_int64 * len(ns))(*ns), len(ns), k, epilogue, ctypes.byref(b))
+        got = _FP8_WORKSPACE[key] = int(b.value)
+    return got
+
+
 def _check_fp8_operands(what: str, x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> tuple[int, int, int]:
     """Ranks, dtypes, shapes and devices of an fp8 linear's operands; returns (m, k, n)."""
     if x.dim() != 2 or weight.dim() != 2 or scale.dim() != 1:
@@ -537,9 +548,9 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> to
     ``x``: bf16 ``[m, k]``; ``weight``: float8 e4m3fn ``[n, k]``; ``scale``:
     bf16 ``[n]``; all on one device. The weights are widened to bf16 in
     registers, so the products are those of dequantizing and running a bf16
-    GEMM. Up to 64 rows run the split-K decode kernel, more rows the tiled
-    prefill kernel. Runs on torch's current stream; a split-K workspace comes
-    from torch's allocator on that stream.
+    GEMM. A few rows run in one launch, up to 64 the split-K decode kernel,
+    more rows the tiled prefill kernel. Runs on torch's current stream; a
+    split-K workspace comes from torch's allocator on that stream.
     """
     m, k, n = _check_fp8_operands("fp8_linear", x, weight, scale)
     if not weight.is_contiguous() or weight.data_ptr() % 16:
@@ -549,7 +560,7 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> to
     if not scale.is_contiguous():
         scale = scale.contiguous()
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    ws_bytes = fp8_linear_workspace_bytes(m, n, k)
+    ws_bytes = _fp8_scratch_bytes(m, (n,), k, nat.FP8_EPILOGUE_NONE)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     nat.call("ftx_fp8_linear", x.data_ptr(), weight.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k,
              ws.data_ptr() if ws is not None else None, ws_bytes, torch.cuda.current_stream(x.device).cuda_stream)
@@ -593,7 +604,7 @@ def fp8_linear_group(x: torch.Tensor, weights: list[torch.Tensor], scales: list[
     g = len(weights)
     ns = (ctypes.c_int64 * g)(*[w.shape[0] for w in weights])
     outs = [torch.empty((m, w.shape[0]), dtype=torch.bfloat16, device=x.device) for w in weights]
-    ws_bytes = fp8_linear_group_workspace_bytes(m, list(ns), k)
+    ws_bytes = _fp8_scratch_bytes(m, tuple(ns), k, nat.FP8_EPILOGUE_NONE)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     ptrs = [(ctypes.c_void_p * g)(*[t.data_ptr() for t in ts]) for ts in (weights, scales, outs)]
     nat.call("ftx_fp8_linear_group", x.data_ptr(), g, *(ctypes.cast(a, ctypes.c_void_p) for a in ptrs),
@@ -635,13 +646,13 @@ def _fp8_fused(x: torch.Tensor, weights: list[torch.Tensor], scales: list[torch.
     g = len(weights)
     ns = [w.shape[0] for w in weights]
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    ws_bytes = fp8_linear_fused_workspace_bytes(m, ns, k, epilogue)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+    ws_bytes = _fp8_scratch_bytes(m, tuple(ns), k, epilogue)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     arrays = [(ctypes.c_void_p * g)(*[t.data_ptr() for t in ts]) for ts in (weights, scales)]
     n_arr = (ctypes.c_int64 * g)(*ns)
     nat.call("ftx_fp8_linear_fused", x.data_ptr(), g, *(ctypes.cast(a, ctypes.c_void_p) for a in arrays),
              y.data_ptr(), ctypes.cast(n_arr, ctypes.c_void_p), m, k, epilogue,
-             residual.data_ptr() if residual is not None else None, ws.data_ptr(), ws_bytes,
+             residual.data_ptr() if residual is not None else None, ws.data_ptr() if ws is not None else None, ws_bytes,
              torch.cuda.current_stream(x.device).cuda_stream)
     return y
 
@@ -663,6 +674,32 @@ def fp8_linear_residual(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tens
     (``FTX_FP8_EPILOGUE_RESIDUAL``): a decoder's output projection and its residual connection. Decode
     batches only (at most 64 rows); the same bits as the separate linear and bf16 add."""
     return _fp8_fused(x, [weight], [scale], nat.FP8_EPILOGUE_RESIDUAL, residual, "fp8_linear_residual")
+
+
+BF16_LINEAR_MAX_ROWS = 16
+
+
+def bf16_linear_eligible(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+    """Whether :func:`bf16_linear` takes ``x`` [..., k] and these weights [n, k]."""
+    k = x.shape[-1] if x.dim() else 0
+    return (k > 0 and 0 < x.numel() <= BF16_LINEAR_MAX_ROWS * k and k % 8 == 0 and kernel_call(x, *weights)
+            and all(w.dim() == 2 and w.shape[1] == k and w.shape[0] > 0 for w in weights)
+            and _packed(x, *weights))
+
+
+def bf16_linear(x: torch.Tensor, weights: list[torch.Tensor], epilogue: int = nat.FP8_EPILOGUE_NONE,
+                residual: torch.Tensor | None = None) -> list[torch.Tensor]:
+    """``[x @ w.T for w in weights]`` for up to 16 bf16 rows in one launch (``ftx_bf16_linear``); under an
+    epilogue one output: ``silu(g) * u`` of two weights, or ``residual + x @ w.T`` of one."""
+    k = x.shape[-1]
+    m, g = x.numel() // k, len(weights)
+    n_out = 1 if epilogue == nat.FP8_EPILOGUE_SWIGLU else g
+    outs = [torch.empty((*x.shape[:-1], w.shape[0]), dtype=torch.bfloat16, device=x.device) for w in weights[:n_out]]
+    ptrs = ctypes.c_void_p * g
+    nat.call("ftx_bf16_linear", x.data_ptr(), g, ptrs(*[w.data_ptr() for w in weights]),
+             ptrs(*[y.data_ptr() for y in outs]), (ctypes.c_int64 * g)(*[w.shape[0] for w in weights]), m, k, epilogue,
+             residual.data_ptr() if residual is not None else None, _stream())
+    return outs
 
 
 def fp8_linear_static(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor, out: torch.Tensor) -> torch.Tensor:

@@ -158,6 +158,15 @@ class Fp8Linear(nn.Module):
         return F.linear(x, w) * self.scale
 
 
+class Linear(nn.Linear):
+    """``nn.Linear`` whose forward on a few bf16 GPU rows (a decode batch) is the library's one-launch kernel."""
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if self.bias is None and hip.bf16_linear_eligible(x, self.weight):
+            return hip.bf16_linear(x, [self.weight])[0]
+        return super().forward(x)
+
+
 def _plain_call(module: nn.Module) -> bool:
     """Whether calling ``module`` would run its class's forward and nothing else: no forward set on the
     instance (an offload manager's enter/exit trap is one) and no forward hooks. Only then may a caller
@@ -212,8 +221,36 @@ def fp8_residual(x: torch.Tensor, lin: nn.Module, residual: torch.Tensor) -> tor
     return y.view(residual.shape)
 
 
+def _bf16_fusable(x: torch.Tensor, layers: list[nn.Module]) -> bool:
+    """Whether a call of these layers on ``x`` is one launch of the bf16 decode kernel."""
+    return (all(type(lin) is Linear and lin.bias is None and _plain_call(lin) for lin in layers)
+            and hip.bf16_linear_eligible(x, *[lin.weight for lin in layers]))
+
+
+def linear_group(x: torch.Tensor, layers: list[nn.Module]) -> list[torch.Tensor] | None:
+    """The outputs of several linear layers on one input in one launch, or None when no kernel takes the group."""
+    if _bf16_fusable(x, layers):
+        return hip.bf16_linear(x, [lin.weight for lin in layers])
+    return fp8_group(x, layers)
+
+
+def linear_swiglu(x: torch.Tensor, gate: nn.Module, up: nn.Module) -> torch.Tensor | None:
+    """``F.silu(gate(x)) * up(x)`` in one launch, or None when no kernel takes the call."""
+    if _bf16_fusable(x, [gate, up]) and gate.weight.shape == up.weight.shape:
+        return hip.bf16_linear(x, [gate.weight, up.weight], hip.nat.FP8_EPILOGUE_SWIGLU)[0]
+    return fp8_swiglu(x, gate, up)
+
+
+def linear_residual(x: torch.Tensor, lin: nn.Module, residual: torch.Tensor) -> torch.Tensor | None:
+    """``residual + lin(x)`` in one launch, or None when no kernel takes the call."""
+    if _bf16_fusable(x, [lin]) and hip.kernel_call(residual) and residual.is_contiguous() and \
+            residual.shape == (*x.shape[:-1], lin.weight.shape[0]):
+        return hip.bf16_linear(x, [lin.weight], hip.nat.FP8_EPILOGUE_RESIDUAL, residual)[0]
+    return fp8_residual(x, lin, residual)
+
+
 def _proj(s: LlamaShape, n_in: int, n_out: int, dtype: torch.dtype) -> nn.Module:
-    return Fp8Linear(n_in, n_out) if s.fp8 else nn.Linear(n_in, n_out, bias=False, dtype=dtype)
+    return Fp8Linear(n_in, n_out) if s.fp8 else Linear(n_in, n_out, bias=False, dtype=dtype)
 
 
 class RMSNorm(nn.Module):
@@ -250,10 +287,10 @@ class Attention(nn.Module):
     def forward(self, x: torch.Tensor, pos: int, cos: torch.Tensor, sin: torch.Tensor,
                 cache_k: torch.Tensor, cache_v: torch.Tensor, residual: torch.Tensor | None = None) -> torch.Tensor:
         """The attention block's output, plus ``residual`` when given (folded into the output projection's
-        reduce for fp8 decode batches)."""
+        launch for decode batches)."""
         s = self.s
         b, t, _ = x.shape
-        qkv = fp8_group(x, [self.wq, self.wk, self.wv])
+        qkv = linear_group(x, [self.wq, self.wk, self.wv])
         q, k, v = qkv if qkv is not None else (self.wq(x), self.wk(x), self.wv(x))
         q = q.view(b, t, s.n_heads, s.head_dim)
         k = k.view(b, t, s.n_kv_heads, s.head_dim)
@@ -289,7 +326,7 @@ class Attention(nn.Module):
         """The output projection of ``o``, plus ``residual`` when given."""
         if residual is None:
             return self.wo(o)
-        fused = fp8_residual(o, self.wo, residual)
+        fused = linear_residual(o, self.wo, residual)
         return fused if fused is not None else residual + self.wo(o)
 
 
@@ -307,14 +344,14 @@ class DecoderLayer(nn.Module):
                 cache_k: torch.Tensor, cache_v: torch.Tensor) -> torch.Tensor:
         x = self.attn(self.attn_norm(x), pos, cos, sin, cache_k, cache_v, residual=x)
         h = self.mlp_norm(x)
-        act = fp8_swiglu(h, self.gate, self.up)
+        act = linear_swiglu(h, self.gate, self.up)
         if act is None:
-            gu = fp8_group(h, [self.gate, self.up])
+            gu = linear_group(h, [self.gate, self.up])
             g, u = gu if gu is not None else (self.gate(h), self.up(h))
             act = hip.silu_mul(g, u)
             if act is None:
                 act = F.silu(g) * u
-        out = fp8_residual(act, self.down, x)
+        out = linear_residual(act, self.down, x)
         return out if out is not None else x + self.down(act)
 
 
@@ -325,7 +362,7 @@ class LlamaModel(nn.Module):
         self.embed = nn.Embedding(s.vocab, s.hidden, dtype=dtype)
         self.layers = nn.ModuleList(DecoderLayer(s, dtype) for _ in range(s.n_layers))
         self.norm = RMSNorm(s.hidden, s.eps, dtype)
-        self.lm_head = nn.Linear(s.hidden, s.vocab, bias=False, dtype=dtype)
+        self.lm_head = Linear(s.hidden, s.vocab, bias=False, dtype=dtype)
         inv = 1.0 / (s.rope_theta ** (torch.arange(0, s.head_dim, 2, dtype=torch.float32) / s.head_dim))
         ang = torch.outer(torch.arange(s.max_seq, dtype=torch.float32), inv)
         self.register_buffer("rope_cos", torch.cat([ang.cos(), ang.cos()], -1), persistent=False)

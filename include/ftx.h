@@ -266,7 +266,9 @@ int ftx_scatter(const void *chunk, const ftx_desc *descs, int n_desc, void *stre
  * contiguous, 16-byte aligned; scale: bf16 [n]; y: bf16 [m, n] contiguous;
  * k a multiple of 16. The weights are widened to bf16 in registers and
  * multiplied on the MFMA units in fp32; no bf16 copy of them is written.
- * Up to 64 rows (decode) K is split over workgroups; each slice's partial
+ * A few rows (up to 16 on small matrices) run in one launch that sums the whole
+ * of K inside each workgroup and touches no workspace. Up to 64 rows (decode),
+ * and below under a fixed launch shape, K is split over workgroups; each slice's partial
  * sums go to `workspace` (device memory of at least ftx_fp8_linear_workspace
  * bytes, 16-byte aligned; it may be NULL when that size is 0) and a second
  * kernel adds them in slice order, so results are deterministic for a given
@@ -306,7 +308,7 @@ int ftx_fp8_linear_group(const void *x, int group, const void *const *w, const v
  *   FTX_FP8_EPILOGUE_RESIDUAL group 1: y = bf16(residual + bf16(out))
  *                             (residual + F.linear(...)); residual is bf16
  *                             [m, n] and may be y itself.
- * y is one bf16 [m, n[0]] output. Every call goes through the workspace
+ * y is one bf16 [m, n[0]] output. Split calls go through the workspace
  * (ftx_fp8_linear_fused_workspace, non-zero). More than 64 rows, or an
  * epilogue of the wrong group shape, returns FTX_ERR_UNSUPPORTED or
  * FTX_ERR_INVALID before any operand is touched. */
@@ -317,6 +319,20 @@ int ftx_fp8_linear_fused_workspace(int64_t m, const int64_t *n, int group, int64
 int ftx_fp8_linear_fused(const void *x, int group, const void *const *w, const void *const *scale, void *y,
                          const int64_t *n, int64_t m, int64_t k, int epilogue, const void *residual, void *workspace,
                          size_t workspace_bytes, void *stream);
+
+/* Bytes of workspace a call of this group and epilogue touches under the launch
+ * shape in force: 0 for calls that run in one launch, which then accept a NULL
+ * workspace; otherwise what the queries above return. */
+int ftx_fp8_linear_scratch(int64_t m, const int64_t *n, int group, int64_t k, int epilogue, size_t *bytes);
+
+/* No counterpart in the reference. Decode-sized linears with bf16 weights, m <=
+ * 16, in one launch and without workspace: y[s] = bf16(x @ w[s]^T) for up to
+ * four matrices [n[s], k] that share x [m, k] (k a multiple of 8; x and w
+ * contiguous and 16-byte aligned), fp32 sums. Epilogues and their group shapes
+ * as for ftx_fp8_linear_fused, with y[0] the one output. Each output's sum has
+ * the same order alone and in any group. */
+int ftx_bf16_linear(const void *x, int group, const void *const *w, void *const *y, const int64_t *n, int64_t m,
+                    int64_t k, int epilogue, const void *residual, void *stream);
 
 /* Bytes of the static scratch array behind ftx_fp8_linear_static (64 MiB per GPU). */
 #define FTX_FP8_STATIC_SCRATCH_BYTES ((size_t)64 << 20)

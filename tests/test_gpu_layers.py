@@ -198,6 +198,55 @@ def test_silu_mul_matches_float64(gpu, n):
     assert hip.silu_mul(g[1:], u[1:]) is None
 
 
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("ns,k", [((1,), 8), ((17, 16), 120), ((15, 300, 64), 136), ((257,), 2056), ((4096,), 1024)])
+def test_bf16_linear_matches_float64(gpu, m, ns, k):
+    """One launch for a group; each output has the same bits alone (the sum's order depends on k only), also under
+    the residual epilogue; SwiGLU rounds where the separate operations round."""
+    from flextensor_amd import _native as nat
+    from flextensor_amd import hip
+
+    x = _randn(gpu, m, k)
+    ws = [_randn(gpu, n, k, seed=i + 1) for i, n in enumerate(ns)]
+    assert hip.bf16_linear_eligible(x, *ws)
+    got = hip.bf16_linear(x, ws)
+    for y, w in zip(got, ws):
+        assert _rel(y, x.double() @ w.double().t()) < ONE_ROUNDING
+        assert torch.equal(hip.bf16_linear(x, [w])[0], y)
+        r = _randn(gpu, m, w.shape[0], seed=9)
+        assert torch.equal(hip.bf16_linear(x, [w], nat.FP8_EPILOGUE_RESIDUAL, r)[0], r + y)
+    up = _randn(gpu, ns[0], k, seed=7)
+    act = hip.bf16_linear(x, [ws[0], up], nat.FP8_EPILOGUE_SWIGLU)[0]
+    g, u = got[0].double(), hip.bf16_linear(x, [up])[0].double()
+    assert _rel(act, (g / (1 + torch.exp(-g))).to(torch.bfloat16).double() * u) < TWO_ROUNDINGS
+
+
+def test_bf16_linear_takes_decode_batches_of_plain_modules_only(gpu):
+    from flextensor_amd import _native as nat
+    from flextensor_amd import hip
+    from flextensor_amd import workloads as W
+
+    x, w = _randn(gpu, 16, 64), _randn(gpu, 32, 64)
+    assert not hip.bf16_linear_eligible(_randn(gpu, 17, 64), w)
+    assert not hip.bf16_linear_eligible(x[:, :60].contiguous(), w[:, :60].contiguous())
+    assert not hip.bf16_linear_eligible(x, w[:, :60].contiguous())
+    assert not hip.bf16_linear_eligible(x, _randn(gpu, 64, 64)[:, ::2])
+    assert not hip.bf16_linear_eligible(x.float(), w)
+    with pytest.raises(nat.FtxError, match="up to 16 rows"):
+        hip.bf16_linear(_randn(gpu, 17, 64), [w])
+    lin = W.Linear(64, 32, bias=False, dtype=torch.bfloat16).to(gpu)
+    seen = []
+    with torch.no_grad():
+        alone = lin(x)
+        assert torch.equal(W.linear_group(x, [lin])[0], alone)
+        handle = lin.register_forward_hook(lambda mod, args, out: seen.append(out))
+        assert W.linear_group(x, [lin]) is None and W.linear_residual(x, lin, alone) is None
+        assert torch.equal(lin(x), alone) and len(seen) == 1
+        handle.remove()
+    y = lin(x)  # with autograd, torch's linear
+    assert y.requires_grad and _rel(y.detach(), alone.double()) < TWO_ROUNDINGS
+
+
 def test_operations_that_must_be_seen_run_in_torch(gpu):
     """Autograd, forward-mode differentiation, function and dispatch modes, functorch transforms and autocast get
     torch's operations; a plain call gets the kernel."""
