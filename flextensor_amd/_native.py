@@ -257,7 +257,9 @@ def check(rc: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    rc = getattr(_lib if _lib is not None else load(), name)(*args)
+    if rc != FTX_OK:
+        check(rc)
 
 
 # ---- convenience wrappers ---------------------------------------------------

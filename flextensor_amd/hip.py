@@ -11,7 +11,6 @@ as a CPU ``uint8`` tensor without copying.
 from __future__ import annotations
 
 import ctypes
-import math
 from collections.abc import Iterator
 from contextlib import contextmanager
 from typing import Any
@@ -337,43 +336,57 @@ def checksum(t: torch.Tensor, stream: HipStream | None = None) -> int:
     return nat.checksum64(t.data_ptr(), t.numel() * t.element_size(), s.handle)
 
 
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
 def kernel_call(*tensors: torch.Tensor) -> bool:
     """Whether a call on these tensors may run a library kernel in place of torch operations: bf16 tensors on the
     current GPU, and nothing around the call that has to see torch operations - autograd, forward-mode
     differentiation, a function or dispatch mode (an offload manager's discovery is one), a functorch transform,
     autocast, or a trace."""
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_function_stack()
-            or torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None
+    first = tensors[0]
+    if not first.is_cuda:
+        return False
+    c = torch._C
+    if (torch.compiler.is_compiling() or c._get_tracing_state() is not None or c._len_torch_function_stack()
+            or c._len_torch_dispatch_stack() or c._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda")):
         return False
     grad = torch.is_grad_enabled()
+    device = c._cuda_getDevice()
+    bf16 = torch.bfloat16
     for t in tensors:
-        if type(t) not in _PLAIN_TYPES or t.dtype != torch.bfloat16 or not t.is_cuda or (grad and t.requires_grad):
+        if type(t) not in _PLAIN_TYPES or t.dtype != bf16 or t.get_device() != device or (grad and t.requires_grad):
             return False
-    return tensors[0].get_device() == torch.cuda.current_device() and \
-        all(t.get_device() == tensors[0].get_device() for t in tensors[1:])
-
-
-_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+    return True
 
 
 def _packed(*tensors: torch.Tensor) -> bool:
     """Whether every tensor is contiguous and starts at a 16-byte boundary."""
-    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+    for t in tensors:
+        if t.data_ptr() % 16 or not t.is_contiguous():
+            return False
+    return True
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+def _stream(device: int | None = None) -> int:
+    """The handle of torch's current stream on ``device`` (None: the current device)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if device is None else device)
 
 
-def _strided_heads(t: torch.Tensor) -> bool:
-    """Whether a [batch, position, head, d] tensor can be read 16 bytes at a time: contiguous along d, every
-    other stride (of more than one element) a multiple of 8, a 16-byte aligned start."""
-    return t.stride(3) == 1 and t.data_ptr() % 16 == 0 and all(t.stride(i) % 8 == 0 for i in range(3) if t.shape[i] > 1)
+def _head_strides(t: torch.Tensor) -> tuple[int, int, int] | None:
+    """Batch, position and head strides of a [batch, position, head, d] tensor that can be read 16 bytes at a
+    time, else None: contiguous along d, strides (of more than one element) multiples of 8, an aligned start."""
+    s0, s1, s2, s3 = t.stride()
+    n0, n1, n2, _ = t.shape
+    s0, s1, s2 = s0 if n0 > 1 else 0, s1 if n1 > 1 else 0, s2 if n2 > 1 else 0
+    return (s0, s1, s2) if s3 == 1 and not (s0 | s1 | s2) % 8 and t.data_ptr() % 16 == 0 else None
 
 
-def _strides(t: torch.Tensor) -> tuple[int, int, int]:
-    return tuple(t.stride(i) if t.shape[i] > 1 else 0 for i in range(3))
+def _attention_sizes(b: int, t: int, s: int, h: int, kv: int, d: int, position_stride: int) -> bool:
+    return (d in (64, 128) and b > 0 and t > 0 and s > 0 and kv > 0 and h > 0 and h % kv == 0
+            and max(b, t * (h // kv), s) <= 1 << 24 and h <= 65536 and b * h * t <= 1 << 30
+            and (s + 256) * 2 * position_stride < 1 << 31)
 
 
 def attention_eligible(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
@@ -381,14 +394,31 @@ def attention_eligible(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> boo
     if not kernel_call(q, k, v) or q.dim() != 4 or k.dim() != 4 or k.shape != v.shape:
         return False
     b, t, h, d = q.shape
-    s, kv = k.shape[1], k.shape[2]
-    return (k.shape[0] == b and k.shape[3] == d and d in (64, 128) and b > 0 and t > 0 and s > 0 and kv > 0
-            and h > 0 and h % kv == 0 and max(b, t * (h // kv), s) <= 1 << 24 and h <= 65536 and b * h * t <= 1 << 30
-            and (s + 256) * 2 * max(k.stride(1), v.stride(1)) < 1 << 31
-            and _strided_heads(q) and _strided_heads(k) and _strided_heads(v))
+    return (k.shape[0] == b and k.shape[3] == d
+            and _attention_sizes(b, t, k.shape[1], h, k.shape[2], d, max(k.stride(1), v.stride(1)))
+            and all(_head_strides(x) is not None for x in (q, k, v)))
 
 
 _ATTENTION_WORKSPACE: dict[tuple, int] = {}
+
+
+def _attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, shape: tuple[int, ...], k_strides: tuple[int, ...],
+            v_strides: tuple[int, ...], pos: int | None, stream: int) -> torch.Tensor:
+    """The checked call: ``shape`` is (batch, queries, keys, heads, kv heads, d)."""
+    out = torch.empty_like(q)
+    ws_bytes = _ATTENTION_WORKSPACE.get(shape)
+    if ws_bytes is None:
+        got = ctypes.c_size_t(0)
+        nat.call("ftx_attention_workspace", *shape, ctypes.byref(got))
+        if len(_ATTENTION_WORKSPACE) >= 4096:  # a decode's key count grows by one a step
+            _ATTENTION_WORKSPACE.clear()
+        ws_bytes = _ATTENTION_WORKSPACE[shape] = int(got.value)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    strides = (ctypes.c_int64 * 12)(*_head_strides(q), *k_strides, *v_strides, *_head_strides(out))
+    nat.call("ftx_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *shape, strides,
+             0 if pos is None else 1, pos or 0, shape[5] ** -0.5, ws.data_ptr() if ws is not None else None, ws_bytes,
+             stream)
+    return out
 
 
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: int | None = None) -> torch.Tensor:
@@ -398,22 +428,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: int | None
     out as q is. ``pos``: query t sees the keys up to ``pos + t``; None: every key.
     """
     b, t, h, d = q.shape
-    s, kv = k.shape[1], k.shape[2]
-    out = torch.empty_like(q)
-    key = (b, t, s, h, kv, d)
-    ws_bytes = _ATTENTION_WORKSPACE.get(key)
-    if ws_bytes is None:
-        got = ctypes.c_size_t(0)
-        nat.call("ftx_attention_workspace", b, t, s, h, kv, d, ctypes.byref(got))
-        if len(_ATTENTION_WORKSPACE) >= 4096:  # a decode's key count grows by one a step
-            _ATTENTION_WORKSPACE.clear()
-        ws_bytes = _ATTENTION_WORKSPACE[key] = int(got.value)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
-    strides = (ctypes.c_int64 * 12)(*_strides(q), *_strides(k), *_strides(v), *_strides(out))
-    nat.call("ftx_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, t, s, h, kv, d, strides,
-             int(pos is not None), pos or 0, 1.0 / math.sqrt(d), ws.data_ptr() if ws is not None else None, ws_bytes,
-             _stream())
-    return out
+    return _attend(q, k, v, (b, t, k.shape[1], h, k.shape[2], d), _head_strides(k), _head_strides(v), pos, _stream())
 
 
 NORM_MAX_DIM = 32768
@@ -462,32 +477,61 @@ def residual_norm(x: torch.Tensor, eps: float, delta: torch.Tensor | None = None
     return total, y
 
 
+def _rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: int,
+          cache_k: torch.Tensor, cache_v: torch.Tensor, stream: int):
+    """:func:`rope_cache`, with the caches' strides: ``(rotated q, cache_k strides, cache_v strides)``."""
+    b, t, h, d = q.shape
+    kv = k.shape[2]
+    if (type(pos) is not int or pos < 0 or d % 16 or not q.numel() or k.shape != (b, t, kv, d) or v.shape != k.shape
+            or not _packed(q, k, v)):
+        return None
+    grad = torch.is_grad_enabled()
+    device = q.get_device()
+    for table in (cos, sin):
+        if (type(table) not in _PLAIN_TYPES or table.dtype != torch.float32 or table.dim() != 2
+                or table.shape[1] != d or table.shape[0] < pos + t or table.get_device() != device
+                or (grad and table.requires_grad) or not _packed(table)):
+            return None
+    strides = []
+    for cache in (cache_k, cache_v):
+        if cache.dim() != 4 or cache.shape[0] < b or cache.shape[1] < pos + t or cache.shape[2:] != (kv, d):
+            return None
+        strides.append(_head_strides(cache))
+        if strides[-1] is None or 0 in cache.stride():
+            return None
+    if cache_k.data_ptr() == cache_v.data_ptr():
+        return None
+    out = torch.empty_like(q)
+    nat.call("ftx_rope_cache", q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+             out.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), b, t, h, kv, d, pos,
+             (ctypes.c_int64 * 6)(*strides[0], *strides[1]), stream)
+    return out, *strides
+
+
 def rope_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: int,
                cache_k: torch.Tensor, cache_v: torch.Tensor) -> torch.Tensor | None:
     """The rotated queries of [batch, t, head, d] ``q``; the rotated ``k`` and ``v`` go to positions ``pos ..
     pos + t - 1`` of the caches, in one launch (``ftx_rope_cache``). None when the kernel does not take the
     call."""
+    got = _rope(q, k, v, cos, sin, pos, cache_k, cache_v, _stream()) if kernel_call(q, k, v, cache_k, cache_v) else None
+    return got[0] if got is not None else None
+
+
+def rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: int,
+                   cache_k: torch.Tensor, cache_v: torch.Tensor) -> torch.Tensor | None:
+    """Causal attention of new positions over the KV cache: :func:`rope_cache`, then :func:`attention` of the
+    rotated queries over the first ``pos + t`` cached positions. None, with nothing written, when the kernels do
+    not take the call."""
+    if type(pos) is not int:
+        return None
     b, t, h, d = q.shape
-    kv = k.shape[2]
-    if (type(pos) is not int or pos < 0 or d % 16 or not q.numel() or not kernel_call(q, k, v, cache_k, cache_v)
-            or k.shape != (b, t, kv, d) or v.shape != k.shape or not _packed(q, k, v)):
+    shape = (b, t, pos + t, h, k.shape[2], d)
+    if (not kernel_call(q, k, v, cache_k, cache_v) or cache_k.dim() != 4 or cache_v.dim() != 4
+            or not _attention_sizes(*shape, max(cache_k.stride(1), cache_v.stride(1)))):
         return None
-    for table in (cos, sin):
-        if (type(table) not in _PLAIN_TYPES or table.dtype != torch.float32 or table.dim() != 2
-                or table.shape[1] != d or table.shape[0] < pos + t or table.device != q.device
-                or (table.requires_grad and torch.is_grad_enabled()) or not _packed(table)):
-            return None
-    for cache in (cache_k, cache_v):
-        if (cache.dim() != 4 or cache.shape[0] < b or cache.shape[1] < pos + t or cache.shape[2:] != (kv, d)
-                or not _strided_heads(cache) or 0 in cache.stride()):
-            return None
-    if cache_k.data_ptr() == cache_v.data_ptr():
-        return None
-    out = torch.empty_like(q)
-    strides = (ctypes.c_int64 * 6)(*_strides(cache_k), *_strides(cache_v))
-    nat.call("ftx_rope_cache", q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-             out.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), b, t, h, kv, d, pos, strides, _stream())
-    return out
+    stream = _stream()
+    got = _rope(q, k, v, cos, sin, pos, cache_k, cache_v, stream)
+    return _attend(got[0], cache_k, cache_v, shape, got[1], got[2], pos, stream) if got is not None else None
 
 
 def silu_mul(g: torch.Tensor, u: torch.Tensor) -> torch.Tensor | None:
@@ -563,7 +607,7 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> to
     ws_bytes = _fp8_scratch_bytes(m, (n,), k, nat.FP8_EPILOGUE_NONE)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     nat.call("ftx_fp8_linear", x.data_ptr(), weight.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k,
-             ws.data_ptr() if ws is not None else None, ws_bytes, torch.cuda.current_stream(x.device).cuda_stream)
+             ws.data_ptr() if ws is not None else None, ws_bytes, _stream(x.get_device()))
     return y
 
 
@@ -607,9 +651,8 @@ def fp8_linear_group(x: torch.Tensor, weights: list[torch.Tensor], scales: list[
     ws_bytes = _fp8_scratch_bytes(m, tuple(ns), k, nat.FP8_EPILOGUE_NONE)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     ptrs = [(ctypes.c_void_p * g)(*[t.data_ptr() for t in ts]) for ts in (weights, scales, outs)]
-    nat.call("ftx_fp8_linear_group", x.data_ptr(), g, *(ctypes.cast(a, ctypes.c_void_p) for a in ptrs),
-             ctypes.cast(ns, ctypes.c_void_p), m, k, ws.data_ptr() if ws is not None else None, ws_bytes,
-             torch.cuda.current_stream(x.device).cuda_stream)
+    nat.call("ftx_fp8_linear_group", x.data_ptr(), g, *ptrs, ns, m, k, ws.data_ptr() if ws is not None else None,
+             ws_bytes, _stream(x.get_device()))
     return outs
 
 
@@ -650,10 +693,9 @@ def _fp8_fused(x: torch.Tensor, weights: list[torch.Tensor], scales: list[torch.
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     arrays = [(ctypes.c_void_p * g)(*[t.data_ptr() for t in ts]) for ts in (weights, scales)]
     n_arr = (ctypes.c_int64 * g)(*ns)
-    nat.call("ftx_fp8_linear_fused", x.data_ptr(), g, *(ctypes.cast(a, ctypes.c_void_p) for a in arrays),
-             y.data_ptr(), ctypes.cast(n_arr, ctypes.c_void_p), m, k, epilogue,
+    nat.call("ftx_fp8_linear_fused", x.data_ptr(), g, *arrays, y.data_ptr(), n_arr, m, k, epilogue,
              residual.data_ptr() if residual is not None else None, ws.data_ptr() if ws is not None else None, ws_bytes,
-             torch.cuda.current_stream(x.device).cuda_stream)
+             _stream(x.get_device()))
     return y
 
 

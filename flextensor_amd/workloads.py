@@ -24,6 +24,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules import module as torch_module
 
 from . import hip
 
@@ -171,8 +172,6 @@ def _plain_call(module: nn.Module) -> bool:
     """Whether calling ``module`` would run its class's forward and nothing else: no forward set on the
     instance (an offload manager's enter/exit trap is one) and no forward hooks. Only then may a caller
     compute the module's output from its weights directly, in a grouped or fused launch."""
-    from torch.nn.modules import module as torch_module
-
     return ("forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
             and not torch_module._global_forward_hooks and not torch_module._global_forward_pre_hooks)
 
@@ -295,9 +294,8 @@ class Attention(nn.Module):
         q = q.view(b, t, s.n_heads, s.head_dim)
         k = k.view(b, t, s.n_kv_heads, s.head_dim)
         v = v.view(b, t, s.n_kv_heads, s.head_dim)
-        fused = hip.rope_cache(q, k, v, cos, sin, pos, cache_k, cache_v)
-        if fused is not None and hip.attention_eligible(fused, cache_k[:b, : pos + t], cache_v[:b, : pos + t]):
-            o = hip.attention(fused, cache_k[:b, : pos + t], cache_v[:b, : pos + t], pos)
+        o = hip.rope_attention(q, k, v, cos, sin, pos, cache_k, cache_v)
+        if o is not None:
             return self._output(o.view(b, t, s.n_heads * s.head_dim), residual)
         c = cos[pos: pos + t].view(1, t, 1, -1).to(q.dtype)
         sn = sin[pos: pos + t].view(1, t, 1, -1).to(q.dtype)
