@@ -51,6 +51,8 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// four floats at any 4-byte boundary: vector memory accesses need no more than dword alignment
+typedef float f32x4_dword __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kWave = 64;
 constexpr int kPieceBytes = 16;              // fp8 bytes one lane loads per row and step
@@ -250,10 +252,14 @@ __global__ __launch_bounds__(512) void fp8_linear_kernel(const uint8_t *__restri
   for (int b = 0; b < MB; ++b) {
     const int m = b * 16 + r;
     if (m >= M) continue;
-    float *dst = pseg + (static_cast<size_t>(sp) * M + m) * N;
+    float *dst = pseg + (static_cast<size_t>(sp) * M + m) * N + nb;
+    if (nb + 3 < N) {
+      *reinterpret_cast<f32x4_dword *>(dst) = acc[b];
+    } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (nb + i < N) dst[nb + i] = acc[b][i];
+      for (int i = 0; i < 4; ++i)
+        if (nb + i < N) dst[i] = acc[b][i];
+    }
   }
 }
 
@@ -284,12 +290,12 @@ __device__ __forceinline__ void sum_slices(const float *__restrict__ p, int64_t 
                                            float (&acc)[kReduceVec]) {
 #pragma unroll
   for (int e = 0; e < kReduceVec; ++e) acc[e] = 0.f;
-  if (MN % kReduceVec == 0) {
+  if (i0 + kReduceVec <= MN) {
     for (int p0 = 0; p0 < splits; p0 += kReduceBatch) {
       f32x4 v[kReduceBatch];
 #pragma unroll
       for (int j = 0; j < kReduceBatch; ++j)
-        v[j] = p0 + j < splits ? *reinterpret_cast<const f32x4 *>(p + (p0 + j) * MN + i0)
+        v[j] = p0 + j < splits ? *reinterpret_cast<const f32x4_dword *>(p + (p0 + j) * MN + i0)
                                : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < kReduceBatch; ++j)
@@ -315,6 +321,10 @@ __global__ __launch_bounds__(kReduceThreads) void fp8_linear_reduce_kernel(const
   if (i0 >= MN) return;
   const uint16_t *__restrict__ scale = seg.scale[s];
   uint16_t *__restrict__ y = seg.y[s];
+  int col[kReduceVec];  // the channels of this thread's outputs (M N is at most 2^31)
+  col[0] = static_cast<int>(static_cast<uint32_t>(i0) % static_cast<uint32_t>(N));
+#pragma unroll
+  for (int e = 1; e < kReduceVec; ++e) col[e] = col[e - 1] + 1 == N ? 0 : col[e - 1] + 1;
   float acc[kReduceVec];
   sum_slices(part + seg.part0[s], MN, i0, splits, acc);
   if (epilogue == kFp8EpilogueSwiglu) {  // s is 0: the gate; the up matrix is segment 1, same shape
@@ -325,8 +335,8 @@ __global__ __launch_bounds__(kReduceThreads) void fp8_linear_reduce_kernel(const
     for (int e = 0; e < kReduceVec; ++e) {
       const int64_t i = i0 + e;
       if (i < MN) {
-        const float g = bf16_bits_to_f32(f32_to_bf16_bits(acc[e] * bf16_bits_to_f32(scale[i % N])));
-        const float u = bf16_bits_to_f32(f32_to_bf16_bits(up[e] * bf16_bits_to_f32(scale_up[i % N])));
+        const float g = bf16_bits_to_f32(f32_to_bf16_bits(acc[e] * bf16_bits_to_f32(scale[col[e]])));
+        const float u = bf16_bits_to_f32(f32_to_bf16_bits(up[e] * bf16_bits_to_f32(scale_up[col[e]])));
         const float act = bf16_bits_to_f32(f32_to_bf16_bits(g / (1.0f + expf(-g))));
         y[i] = f32_to_bf16_bits(act * u);
       }
@@ -337,7 +347,7 @@ __global__ __launch_bounds__(kReduceThreads) void fp8_linear_reduce_kernel(const
   for (int e = 0; e < kReduceVec; ++e) {
     const int64_t i = i0 + e;
     if (i < MN) {
-      const uint16_t out = f32_to_bf16_bits(acc[e] * bf16_bits_to_f32(scale[i % N]));
+      const uint16_t out = f32_to_bf16_bits(acc[e] * bf16_bits_to_f32(scale[col[e]]));
       y[i] = epilogue == kFp8EpilogueResidual
                  ? f32_to_bf16_bits(bf16_bits_to_f32(residual[i]) + bf16_bits_to_f32(out))
                  : out;
@@ -603,10 +613,7 @@ SegTable seg_table(const Fp8LinearLaunch &p) {
 // one n-tile get consecutive slots on one XCD, so each weight tile comes from
 // HBM once and from that XCD's L2 for the other m-tiles.
 constexpr int kPTileK = 64;
-constexpr int kPXStage = kPTileM * kPTileK * 2;      // 16 KiB activation tile
 constexpr int kPWStage = kPTileN * kPTileK;          // 8 KiB weight tile
-constexpr int kPStage = kPXStage + kPWStage;
-constexpr int kPLoadsPerWave = 6;                    // load instructions per loading wave and step
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -623,14 +630,11 @@ __device__ __forceinline__ bf16x8 fp8x8_to_bf16(uint32_t w0, uint32_t w1) {
 // Activation-tile swizzle: rotate a row's low three bits (see the layout above).
 __device__ __forceinline__ int rot3(int v) { return ((v & 3) << 1) | ((v >> 2) & 1); }
 
-// s_waitcnt vmcnt(n) (expcnt and lgkmcnt left free); n is a constant at every call.
-__device__ __forceinline__ void wait_vmcnt(int n) {
-  switch (n) {
-    case 0: __builtin_amdgcn_s_waitcnt(0x0f70); break;
-    case 6: __builtin_amdgcn_s_waitcnt(0x0f76); break;
-    case 12: __builtin_amdgcn_s_waitcnt(0x0f7c); break;
-    default: __builtin_amdgcn_s_waitcnt(0x0f70); break;
-  }
+// s_waitcnt vmcnt(N) (expcnt and lgkmcnt left free).
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N < 64, "vmcnt holds six bits");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
 }
 
 // Workgroup barrier that also keeps the compiler from moving memory accesses
@@ -647,44 +651,56 @@ __device__ __forceinline__ void ring_barrier() {
 // takes a scalar base (the matrix plus the step's K offset) and a per-lane
 // 32-bit offset, and the loading wave's LDS address is scalar arithmetic: the
 // per-step address work leaves the vector ALU (about 3% per layer, measured).
-template <int WAVES, int S, bool SADDR>
+//
+// TM is the tile's activation rows: 128, or 64 for the batches between decode and prefill (mid_linear_wins).
+// Those also split K: workgroup sp of a tile takes the steps from sp * split_steps and writes fp32 sums for
+// fp8_linear_reduce_kernel. Four waves of 32 channels x 64 rows, four stages of 16 KB, two workgroups per CU;
+// bound by the weights' bytes (28672 x 8192 at 64 rows: 70.8 us, 3.3 TB/s). Five and eight stages, four steps
+// at least per split and three workgroups per CU were within 5% or slower.
+template <int TM, int WAVES, int S, bool SADDR>
 __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *__restrict__ x, SegTable seg, int M,
-                                                                 int K, int m_tiles, int n_tiles, int xcds) {
-  static_assert(WAVES == 4 || WAVES == 8, "4 or 8 waves");
-  constexpr int JT = 16 / WAVES;             // 16-row activation tiles per wave
-  constexpr int WROWS = 16 * JT;             // activation rows per wave
-  __shared__ __align__(1024) uint8_t lds[S * kPStage];
+                                                                 int K, int m_tiles, int n_tiles, int xcds, int splits,
+                                                                 int split_steps, float *__restrict__ part) {
+  static_assert(TM == 128 ? WAVES == 4 || WAVES == 8 : TM == 64 && WAVES == 4, "4 or 8 waves");
+  constexpr int IT = TM == 128 ? 4 : 2;            // 16-channel weight tiles per wave
+  constexpr int JT = TM == 128 ? 16 / WAVES : 4;   // 16-row activation tiles per wave
+  constexpr int WROWS = 16 * JT;                   // activation rows per wave
+  constexpr int kXStage = TM * kPTileK * 2;
+  constexpr int kStage = kXStage + kPWStage;
+  constexpr int XL = TM / 32;                      // activation loads per loading wave and step, besides 2 weight loads
+  __shared__ __align__(1024) uint8_t lds[S * kStage];
   const int xcd = blockIdx.x % xcds;
   const int slot = blockIdx.x / xcds;
-  const int nt = (slot / m_tiles) * xcds + xcd;
-  const int mt = slot % m_tiles;
+  const int mt = TM == 128 ? slot % m_tiles : 0;
+  const int sp = TM == 128 ? 0 : slot % splits;
+  const int nt = slot / (TM == 128 ? m_tiles : splits) * xcds + xcd;
   if (nt >= n_tiles) return;  // the last round of n-tiles does not fill every XCD
   int s = 0;
   while (s + 1 < seg.count && nt >= seg.rg0[s + 1]) ++s;
   const int N = seg.n[s];
   const uint8_t *__restrict__ w = seg.w[s];
   const int n_base = (nt - seg.rg0[s]) * kPTileN;
-  const int m_base = mt * kPTileM;
+  const int m_base = mt * TM;
 
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int r = lane & 15;
   const int g = lane >> 4;
-  const int wn = wave & 1;
-  const int wm = wave >> 1;
+  const int wn = TM == 128 ? wave & 1 : wave;
+  const int wm = TM == 128 ? wave >> 1 : 0;
   const bool loads = WAVES == 4 || wave < 4;
   const int lw = __builtin_amdgcn_readfirstlane(wave & 3);  // uniform: LDS destinations stay scalar
 
-  // This lane's load sources: activation rows (lw*4 + t)*8 + lane/8, weight
+  // This lane's load sources: activation rows (lw*XL + t)*8 + lane/8, weight
   // rows (lw*2 + t)*16 + lane/4, at the chunk the swizzle assigns.
   const int xc = ((lane & 7) ^ rot3(lane >> 3)) * 8;        // k offset (elements) within a step
   const int wc = ((lane & 3) ^ ((lane >> 3) & 3)) * 16;     // k offset (bytes) within a step
-  const uint8_t *xrow[4];
+  const uint8_t *xrow[4];  // XL of them
   const uint8_t *wrow[2];
   uint32_t xoff[4], woff[2];  // SADDR: byte offsets of this lane's chunk in step 0
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int gm = min(m_base + (lw * 4 + t) * 8 + (lane >> 3), M - 1);
+  for (int t = 0; t < XL; ++t) {
+    const int gm = min(m_base + (lw * XL + t) * 8 + (lane >> 3), M - 1);
     xrow[t] = x + static_cast<size_t>(gm) * K * 2;
     xoff[t] = static_cast<uint32_t>((static_cast<size_t>(gm) * K + xc) * 2);
   }
@@ -696,18 +712,19 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
   }
   const int full = K / kPTileK;                 // whole steps
   const int tail = K % kPTileK;                 // k values of a final partial step, a multiple of 16
-  const int steps = full + (tail ? 1 : 0);
+  const int first = TM == 128 ? 0 : sp * split_steps;
+  const int steps = TM == 128 ? full + (tail ? 1 : 0) : min(full + (tail ? 1 : 0), first + split_steps);
   auto issue = [&](int st) {
-    uint8_t *base = lds + (st % S) * kPStage;
+    uint8_t *base = lds + (st % S) * kStage;
     if (SADDR && st < full) {  // whole step: scalar base, per-lane offsets fixed for the whole kernel
       const uint8_t *xb = x + static_cast<size_t>(st) * kPTileK * 2;
       const uint8_t *wb = w + static_cast<size_t>(st) * kPTileK;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        __builtin_amdgcn_global_load_lds(xb + xoff[t], (lds_void *)(base + (lw * 4 + t) * 1024), 16, 0, 0);
+      for (int t = 0; t < XL; ++t)
+        __builtin_amdgcn_global_load_lds(xb + xoff[t], (lds_void *)(base + (lw * XL + t) * 1024), 16, 0, 0);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
-        __builtin_amdgcn_global_load_lds(wb + woff[t], (lds_void *)(base + kPXStage + (lw * 2 + t) * 1024), 16, 0,
+        __builtin_amdgcn_global_load_lds(wb + woff[t], (lds_void *)(base + kXStage + (lw * 2 + t) * 1024), 16, 0,
                                          0);
       return;
     }
@@ -716,30 +733,30 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
     const int kw = min(st * kPTileK + wc, K - 16);
     if (SADDR) {  // the same 32-bit offsets, moved by the clamped k
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < XL; ++t)
         __builtin_amdgcn_global_load_lds(x + (xoff[t] + static_cast<uint32_t>(kx - xc) * 2),
-                                         (lds_void *)(base + (lw * 4 + t) * 1024), 16, 0, 0);
+                                         (lds_void *)(base + (lw * XL + t) * 1024), 16, 0, 0);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
         __builtin_amdgcn_global_load_lds(w + (woff[t] + static_cast<uint32_t>(kw - wc)),
-                                         (lds_void *)(base + kPXStage + (lw * 2 + t) * 1024), 16, 0, 0);
+                                         (lds_void *)(base + kXStage + (lw * 2 + t) * 1024), 16, 0, 0);
       return;
     }
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < XL; ++t)
       __builtin_amdgcn_global_load_lds(xrow[t] + static_cast<size_t>(kx) * 2,
-                                       (lds_void *)(base + (lw * 4 + t) * 1024), 16, 0, 0);
+                                       (lds_void *)(base + (lw * XL + t) * 1024), 16, 0, 0);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
-      __builtin_amdgcn_global_load_lds(wrow[t] + kw, (lds_void *)(base + kPXStage + (lw * 2 + t) * 1024), 16, 0,
+      __builtin_amdgcn_global_load_lds(wrow[t] + kw, (lds_void *)(base + kXStage + (lw * 2 + t) * 1024), 16, 0,
                                        0);
   };
 
-  int aoff[4], boff0[JT], boff1[JT];
+  int aoff[IT], boff0[JT], boff1[JT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int R = wn * 64 + i * 16 + r;
-    aoff[i] = kPXStage + R * kPTileK + ((g ^ ((R >> 1) & 3)) << 4);
+  for (int i = 0; i < IT; ++i) {
+    const int R = wn * (16 * IT) + i * 16 + r;
+    aoff[i] = kXStage + R * kPTileK + ((g ^ ((R >> 1) & 3)) << 4);
   }
 #pragma unroll
   for (int j = 0; j < JT; ++j) {
@@ -748,16 +765,16 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
     boff1[j] = R * 128 + (((2 * g + 1) ^ rot3(R & 7)) << 4);
   }
 
-  f32x4 acc[4][JT];
+  f32x4 acc[IT][JT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IT; ++i)
 #pragma unroll
     for (int j = 0; j < JT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   if (loads) {
 #pragma unroll
     for (int st = 0; st < S - 1; ++st)
-      if (st < steps) issue(st);
+      if (first + st < steps) issue(first + st);
   }
   // One step: this wave's loads of step st are in LDS once at most the later
   // steps' loads are outstanding; the barrier then covers every loading wave,
@@ -767,16 +784,16 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
   auto step = [&](int st, bool partial) {
     if (loads) {
       if (st + S - 2 < steps)
-        wait_vmcnt((S - 2) * kPLoadsPerWave);
+        wait_vmcnt<(S - 2) * (XL + 2)>();
       else
-        wait_vmcnt(0);
+        wait_vmcnt<0>();
     }
     ring_barrier();
     if (loads && st + S - 1 < steps) issue(st + S - 1);
-    const uint8_t *sb = lds + (st % S) * kPStage;
-    u32x4 A[4], B0[JT], B1[JT];
+    const uint8_t *sb = lds + (st % S) * kStage;
+    u32x4 A[IT], B0[JT], B1[JT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) A[i] = *reinterpret_cast<const u32x4 *>(sb + aoff[i]);
+    for (int i = 0; i < IT; ++i) A[i] = *reinterpret_cast<const u32x4 *>(sb + aoff[i]);
 #pragma unroll
     for (int j = 0; j < JT; ++j) {
       B0[j] = *reinterpret_cast<const u32x4 *>(sb + boff0[j]);
@@ -784,12 +801,12 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
     }
     if (partial && 16 * g >= tail) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) A[i] = u32x4{0u, 0u, 0u, 0u};
+      for (int i = 0; i < IT; ++i) A[i] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
       for (int j = 0; j < JT; ++j) B0[j] = B1[j] = u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < IT; ++i) {
       const bf16x8 a0 = fp8x8_to_bf16(A[i][0], A[i][1]);
       const bf16x8 a1 = fp8x8_to_bf16(A[i][2], A[i][3]);
 #pragma unroll
@@ -799,16 +816,37 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
       }
     }
   };
-  for (int st = 0; st < full; ++st) step(st, false);
-  if (tail) step(full, true);
+  for (int st = first; st < min(full, steps); ++st) step(st, false);
+  if (tail && steps > full) step(full, true);
 
   // lane holds D rows (output channels) 4g..4g+3 of column (activation row) r of every tile
+  if (TM != 128 && part != nullptr) {
+    float *__restrict__ pseg = part + seg.part0[s] + static_cast<size_t>(sp) * M * N;
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      const int nb = n_base + wn * (16 * IT) + i * 16 + 4 * g;
+#pragma unroll
+      for (int j = 0; j < JT; ++j) {
+        const int m = j * 16 + r;
+        if (m >= M) continue;
+        float *dst = pseg + static_cast<size_t>(m) * N + nb;
+        if (nb + 3 < N) {
+          *reinterpret_cast<f32x4_dword *>(dst) = acc[i][j];
+        } else {
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            if (nb + v < N) dst[v] = acc[i][j][v];
+        }
+      }
+    }
+    return;
+  }
   const uint16_t *__restrict__ scale = seg.scale[s];
   uint16_t *__restrict__ y = seg.y[s];
   const bool vec = (N & 3) == 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int nb = n_base + wn * 64 + i * 16 + 4 * g;
+  for (int i = 0; i < IT; ++i) {
+    const int nb = n_base + wn * (16 * IT) + i * 16 + 4 * g;
     float sc[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) sc[v] = nb + v < N ? __uint_as_float(static_cast<uint32_t>(scale[nb + v]) << 16) : 0.f;
@@ -919,22 +957,38 @@ __global__ __launch_bounds__(256) void mfma_probe_32x32_kernel(float *sink, int 
   if (sum == 1234.5f) sink[0] = sum;
 }
 
-template <int MB>
-hipError_t launch_mb(const Fp8LinearLaunch &p, hipStream_t stream) {
-  const SegTable seg = seg_table(p);
-  const bool reduce = p.workspace_bytes > 0;  // split K, or an epilogue: partials, then the reduce kernel
-  hipLaunchKernelGGL((fp8_linear_kernel<MB>), dim3(static_cast<unsigned>(p.grid)), dim3(p.waves * kWave),
-                     p.lds_bytes, stream, static_cast<const uint8_t *>(p.x), seg,
-                     reduce ? static_cast<float *>(p.workspace) : nullptr, static_cast<int>(p.m), static_cast<int>(p.k),
-                     static_cast<int>(p.kc), p.splits);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess || !reduce) return err;
+hipError_t launch_reduce(const Fp8LinearLaunch &p, const SegTable &seg, hipStream_t stream) {
   // the SwiGLU epilogue writes one output per gate/up pair: the gate's blocks only
   const int blocks = p.epilogue == kFp8EpilogueSwiglu ? seg.rb0[1] : seg.rb0[p.group];
   hipLaunchKernelGGL(fp8_linear_reduce_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kReduceThreads),
                      kReduceLdsToken, stream, static_cast<const float *>(p.workspace), seg, static_cast<int>(p.m),
                      p.splits, p.epilogue, static_cast<const uint16_t *>(p.residual));
   return hipGetLastError();
+}
+
+template <int MB>
+hipError_t launch_mb(const Fp8LinearLaunch &p, hipStream_t stream) {
+  const SegTable seg = seg_table(p);
+  const bool reduce = p.scratch_bytes > 0;  // split K, or an epilogue: partials, then the reduce kernel
+  hipLaunchKernelGGL((fp8_linear_kernel<MB>), dim3(static_cast<unsigned>(p.grid)), dim3(p.waves * kWave),
+                     p.lds_bytes, stream, static_cast<const uint8_t *>(p.x), seg,
+                     reduce ? static_cast<float *>(p.workspace) : nullptr, static_cast<int>(p.m), static_cast<int>(p.k),
+                     static_cast<int>(p.kc), p.splits);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || !reduce) return err;
+  return launch_reduce(p, seg, stream);
+}
+
+}  // namespace
+
+namespace {
+
+// Whether 32-bit load offsets reach every byte of x and of each weight matrix (kept under 2^31, so they read
+// the same whether the hardware widens the offset as signed or unsigned).
+bool offsets_fit(const Fp8LinearLaunch &p) {
+  bool fit = static_cast<uint64_t>(p.m) * p.k * 2 < (uint64_t(1) << 31);
+  for (int s = 0; s < p.group; ++s) fit = fit && static_cast<uint64_t>(p.n[s]) * p.k < (uint64_t(1) << 31);
+  return fit;
 }
 
 }  // namespace
@@ -965,9 +1019,10 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
     // at most one tile per CU: 8 waves (two per SIMD) and 4 LDS stages in one
     // workgroup; more tiles: 4 waves and 2 stages, three workgroups per CU
     p.waves = (waves == 4 || waves == 8) ? waves : (m_tiles * n_tiles <= cus ? 8 : 4);
+    p.small = offsets_fit(p);
     return p;
   }
-  p.batch_blocks = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
+  p.batch_blocks = static_cast<int>((m + 15) / 16);
   // LDS: m activation rows of (2*Kc + 16) bytes plus one weight tile per
   // wave, within kFp8LinearMaxLds (less a margin for the kernel's own flag).
   const int64_t budget = static_cast<int64_t>(kFp8LinearMaxLds) - 256;
@@ -1009,6 +1064,7 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
   p.workspace_bytes = p.splits > 1 || epilogue != kFp8EpilogueNone
                           ? static_cast<size_t>(p.splits) * m * p.n_total * sizeof(float)
                           : 0;
+  p.scratch_bytes = p.workspace_bytes;
   return p;
 }
 
@@ -1023,6 +1079,38 @@ bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k) {
   return m <= 8 ? k <= 16384 : m <= kDirectMaxRows && n_total * k <= int64_t(48) << 20;
 }
 
+// Where tiles of 64 rows beat the split-K decode kernel, whose workgroups hold all rows of x for their slice of
+// K in LDS: from 33 rows that leaves slices of 256 to 512 values and as many partial sums as weights. us,
+// decode kernel and tiles: 64 rows of 28672 x 8192 152 and 70.8, of 4096 x 4096 23.7 and 15.8, of 1024 x 8192
+// 16.1 and 12.5, of 512 x 1024 8.3 and 9.3; 33 rows of 8192 x 8192 36.1 and 26.0; 24 rows of 11008 x 4096 25.5
+// and 22.4, of 5003 x 4080 15.1 and 17.0.
+bool mid_linear_wins(int64_t m, int64_t n_total, int64_t k) {
+  return m > 16 && n_total * k >= (m <= 32 ? int64_t(1) << 25 : int64_t(1) << 23);
+}
+
+void plan_mid_linear(Fp8LinearLaunch *p, int cus, int xcds) {
+  const int64_t steps = (p->k + kPTileK - 1) / kPTileK;
+  int64_t n_tiles = 0;
+  for (int s = 0; s < p->group; ++s) n_tiles += (p->n[s] + kPTileN - 1) / kPTileN;
+  // two workgroups per CU (their LDS fits), at least eight steps each, and no more partial sums than the
+  // split-K plan's, whose size callers are told to allocate
+  int64_t splits = std::min<int64_t>((2 * cus + n_tiles - 1) / n_tiles, std::max<int64_t>(1, steps / 8));
+  splits = std::max<int64_t>(1, std::min<int64_t>(splits, p->splits));
+  const int64_t split_steps = std::max<int64_t>(1, (steps + splits - 1) / splits);
+  p->prefill = p->mid = true;
+  p->small = offsets_fit(*p);
+  p->xcds = std::max(1, xcds);
+  p->waves = 4;
+  p->splits = static_cast<int>(std::max<int64_t>(1, (steps + split_steps - 1) / split_steps));
+  p->kc = split_steps * kPTileK;
+  p->m_tiles = 1;
+  p->row_groups = n_tiles;
+  p->grid = p->xcds * p->splits * ((n_tiles + p->xcds - 1) / p->xcds);
+  p->scratch_bytes = p->splits > 1 || p->epilogue != kFp8EpilogueNone
+                         ? static_cast<size_t>(p->splits) * p->m * p->n_total * sizeof(float)
+                         : 0;
+}
+
 void plan_direct_linear(Fp8LinearLaunch *p) {
   p->direct = true;
   p->splits = 1;
@@ -1030,6 +1118,7 @@ void plan_direct_linear(Fp8LinearLaunch *p) {
   p->row_groups = 0;
   for (int s = 0; s < p->group; ++s) p->row_groups += (p->n[s] + 15) / 16;
   p->grid = p->row_groups;
+  p->scratch_bytes = 0;
 }
 
 hipError_t launch_mfma_probe(int shape, int workgroups, int iters, float *sink, hipStream_t stream) {
@@ -1041,6 +1130,8 @@ hipError_t launch_mfma_probe(int shape, int workgroups, int iters, float *sink, 
                        iters);
   return hipGetLastError();
 }
+
+namespace {
 
 template <bool FP8, int XL>
 hipError_t launch_direct_rows(const Fp8LinearLaunch &p, hipStream_t stream) {
@@ -1067,38 +1158,43 @@ hipError_t launch_direct(const Fp8LinearLaunch &p, hipStream_t stream) {
   return p.m <= 8 ? launch_direct_rows<true, 4>(p, stream) : launch_direct_rows<true, 8>(p, stream);
 }
 
+template <int TM, int WAVES, int S>
+void launch_tiled(const Fp8LinearLaunch &p, const SegTable &seg, float *part, hipStream_t stream) {
+  const auto *x = static_cast<const uint8_t *>(p.x);
+  const int m = static_cast<int>(p.m), k = static_cast<int>(p.k), mt = static_cast<int>(p.m_tiles),
+            nt = static_cast<int>(p.row_groups);
+  const int split_steps = static_cast<int>(p.kc / kPTileK);
+  const dim3 grid(static_cast<unsigned>(p.grid)), block(WAVES * kWave);
+  if (p.small)
+    hipLaunchKernelGGL((fp8_prefill_kernel<TM, WAVES, S, true>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
+                       p.splits, split_steps, part);
+  else
+    hipLaunchKernelGGL((fp8_prefill_kernel<TM, WAVES, S, false>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
+                       p.splits, split_steps, part);
+}
+
+}  // namespace
+
 hipError_t launch_fp8_linear(const Fp8LinearLaunch &p, hipStream_t stream) {
   if (p.direct) return launch_direct(p, stream);
   if (p.prefill) {
     const SegTable seg = seg_table(p);
-    // 32-bit load offsets reach every byte of x and of each weight matrix (kept under 2^31, so they read
-    // the same whether the hardware widens the offset as signed or unsigned)
-    bool small = static_cast<uint64_t>(p.m) * p.k * 2 < (uint64_t(1) << 31);
-    for (int s = 0; s < p.group; ++s) small = small && static_cast<uint64_t>(p.n[s]) * p.k < (uint64_t(1) << 31);
-    const auto *x = static_cast<const uint8_t *>(p.x);
-    const int m = static_cast<int>(p.m), k = static_cast<int>(p.k), mt = static_cast<int>(p.m_tiles),
-              nt = static_cast<int>(p.row_groups);
-    const dim3 grid(static_cast<unsigned>(p.grid));
-    if (p.waves == 8) {
-      if (small)
-        hipLaunchKernelGGL((fp8_prefill_kernel<8, 4, true>), grid, dim3(8 * kWave), 0, stream, x, seg, m, k, mt, nt,
-                           p.xcds);
-      else
-        hipLaunchKernelGGL((fp8_prefill_kernel<8, 4, false>), grid, dim3(8 * kWave), 0, stream, x, seg, m, k, mt, nt,
-                           p.xcds);
-    } else {
-      if (small)
-        hipLaunchKernelGGL((fp8_prefill_kernel<4, 2, true>), grid, dim3(4 * kWave), 0, stream, x, seg, m, k, mt, nt,
-                           p.xcds);
-      else
-        hipLaunchKernelGGL((fp8_prefill_kernel<4, 2, false>), grid, dim3(4 * kWave), 0, stream, x, seg, m, k, mt, nt,
-                           p.xcds);
+    if (p.mid) {
+      const bool reduce = p.scratch_bytes > 0;
+      launch_tiled<64, 4, 4>(p, seg, reduce ? static_cast<float *>(p.workspace) : nullptr, stream);
+      const hipError_t err = hipGetLastError();
+      return err != hipSuccess || !reduce ? err : launch_reduce(p, seg, stream);
     }
+    if (p.waves == 8)
+      launch_tiled<128, 8, 4>(p, seg, nullptr, stream);
+    else
+      launch_tiled<128, 4, 2>(p, seg, nullptr, stream);
     return hipGetLastError();
   }
   switch (p.batch_blocks) {
     case 1: return launch_mb<1>(p, stream);
     case 2: return launch_mb<2>(p, stream);
+    case 3: return launch_mb<3>(p, stream);
     default: return launch_mb<4>(p, stream);
   }
 }

@@ -75,19 +75,22 @@ struct Fp8LinearLaunch {
   int64_t n_total;                     // sum of n
   void *workspace;    // fp32 partial sums [splits, m, n_s] per segment, back to back, when splits > 1
   int64_t m, k;
-  int batch_blocks;   // 16-column batch blocks: 1, 2 or 4 (m <= 16 * batch_blocks)
+  int batch_blocks;   // 16-column batch blocks, 1 to 4 (m <= 16 * batch_blocks)
   int waves;          // wavefronts per workgroup, 16 output rows each
   int splits;         // K slices, one workgroup each per row group
   int64_t kc;         // K values per slice (multiple of 256)
   int64_t row_groups; // groups of 16 * waves output rows, summed over segments
   int64_t grid;       // workgroups = row_groups * splits
   size_t lds_bytes;   // activation slice + one weight tile per wave
-  size_t workspace_bytes;
+  size_t workspace_bytes; // what callers are told to allocate
+  size_t scratch_bytes;   // what the launch touches: at most workspace_bytes
   int epilogue;         // kFp8Epilogue*: what the reduce kernel applies to the outputs
   const void *residual; // bf16 [m, n[0]] for kFp8EpilogueResidual
   bool prefill;       // more than kFp8LinearMaxRows rows: the tiled prefill kernel (no split, no workspace)
   int64_t m_tiles;    // prefill: tiles of 128 activation rows (row_groups then counts tiles of 128 channels)
   int xcds;           // prefill: L2 domains the block order is arranged for
+  bool small;         // prefill: 32-bit load offsets reach every operand
+  bool mid;           // prefill with 64-row tiles and K split over workgroups, for batches between decode and prefill
   bool direct;        // the one-launch decode kernel: no workspace, a workgroup per 16 channels
   bool bf16;          // direct only: bf16 weights without scales
 };
@@ -95,6 +98,9 @@ struct Fp8LinearLaunch {
 constexpr int kDirectMaxRows = 16;
 bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k);
 void plan_direct_linear(Fp8LinearLaunch *p);
+// Tiles of 64 rows for the batches between decode and prefill: whether they are faster, and their plan.
+bool mid_linear_wins(int64_t m, int64_t n_total, int64_t k);
+void plan_mid_linear(Fp8LinearLaunch *p, int cus, int xcds);
 constexpr int kFp8LinearMaxRows = 64;
 constexpr size_t kFp8LinearMaxLds = 64 * 1024;
 Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t k, int cus, int xcds, int waves,

@@ -972,7 +972,12 @@ int plan_fp8(int64_t m, const int64_t *n, int group, int64_t k, ftx::Fp8LinearLa
   }
   *p = ftx::plan_fp8_linear(m, n, group, k, cus, xcds, waves, slice_k, epilogue);
   if (p->grid > (int64_t(1) << 31) - 1) return ftx::fail(FTX_ERR_INVALID, "fp8 linear grid too large");
-  if (!waves && !slice_k && ftx::direct_linear_wins(m, p->n_total, k)) ftx::plan_direct_linear(p);
+  if (!waves && !slice_k && m <= ftx::kFp8LinearMaxRows) {  // no fixed launch shape
+    if (ftx::direct_linear_wins(m, p->n_total, k))
+      ftx::plan_direct_linear(p);
+    else if (ftx::mid_linear_wins(m, p->n_total, k))
+      ftx::plan_mid_linear(p, cus, xcds);
+  }
   return FTX_OK;
 }
 
@@ -983,7 +988,7 @@ int ftx_fp8_linear_scratch(int64_t m, const int64_t *n, int group, int64_t k, in
   ftx::Fp8LinearLaunch p;
   int rc = plan_fp8(m, n, group, k, &p, epilogue);
   if (rc != FTX_OK) return rc;
-  *bytes = p.direct ? 0 : p.workspace_bytes;
+  *bytes = p.scratch_bytes;
   return FTX_OK;
 }
 
@@ -1041,13 +1046,13 @@ int run_fp8(ftx::Fp8LinearLaunch &p, const void *x, const void *const *w, const 
     int rc = ftx::check_device_range(p.residual, static_cast<size_t>(m * p.n[0] * 2), "fp8 linear residual");
     if (rc != FTX_OK) return rc;
   }
-  if (p.workspace_bytes > 0 && !static_workspace && !p.direct) {
-    if (!workspace || workspace_bytes < p.workspace_bytes)
-      return ftx::fail(FTX_ERR_INVALID, "fp8 linear needs a workspace of " + std::to_string(p.workspace_bytes) +
+  if (p.scratch_bytes > 0 && !static_workspace) {
+    if (!workspace || workspace_bytes < p.scratch_bytes)
+      return ftx::fail(FTX_ERR_INVALID, "fp8 linear needs a workspace of " + std::to_string(p.scratch_bytes) +
                                             " bytes (ftx_fp8_linear_workspace)");
     if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
       return ftx::fail(FTX_ERR_INVALID, "workspace needs 16-byte alignment");
-    int rc = ftx::check_device_range(workspace, p.workspace_bytes, "fp8 linear workspace");
+    int rc = ftx::check_device_range(workspace, p.scratch_bytes, "fp8 linear workspace");
     if (rc != FTX_OK) return rc;
   }
   p.x = x;

@@ -267,8 +267,8 @@ int ftx_scatter(const void *chunk, const ftx_desc *descs, int n_desc, void *stre
  * k a multiple of 16. The weights are widened to bf16 in registers and
  * multiplied on the MFMA units in fp32; no bf16 copy of them is written.
  * A few rows (up to 16 on small matrices) run in one launch that sums the whole
- * of K inside each workgroup and touches no workspace. Up to 64 rows (decode),
- * and below under a fixed launch shape, K is split over workgroups; each slice's partial
+ * of K inside each workgroup and touches no workspace. Otherwise up to 64 rows
+ * (decode) K is split over workgroups; each slice's partial
  * sums go to `workspace` (device memory of at least ftx_fp8_linear_workspace
  * bytes, 16-byte aligned; it may be NULL when that size is 0) and a second
  * kernel adds them in slice order, so results are deterministic for a given

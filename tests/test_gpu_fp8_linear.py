@@ -732,3 +732,24 @@ def test_decoder_layer_fused_path_against_the_separate_operations(gpu, default_c
     assert len(seen) == 1 and torch.equal(hooked, fused)
     del model
     torch.cuda.empty_cache()
+
+
+# Both sides of the lines where the one-launch, 64-row-tile and split-K kernels meet, with ragged n and k.
+@pytest.mark.parametrize("m,n,k", [(4, 300, 16400), (5, 300, 16400), (9, 5003, 10064), (9, 5003, 10000),
+                                   (17, 8201, 4112), (32, 8201, 4080), (33, 2049, 4112), (33, 2049, 4080),
+                                   (48, 2177, 8176), (64, 5003, 4080), (64, 65600, 144)])
+def test_kernel_choice_matches_the_oracle_on_both_sides(gpu, default_config, m, n, k):
+    """Exact products equal the oracle bit for bit through whichever kernel the shape picks, alone, grouped and
+    under the residual epilogue."""
+    from flextensor_amd import hip
+
+    print(f"kernel choice m={m} n={n} k={k}", flush=True)
+    x, w_raw, scale = _exact_case(m, n, k, seed=m + n + k)
+    xt, wt, st = _to_device(x, w_raw, scale, gpu)
+    want = torch.from_numpy(ofp8.fp8_linear(x, w_raw, scale)).to(torch.bfloat16)
+    assert _same_values(hip.fp8_linear(xt, wt, st), want)
+    small = wt[:33].contiguous(), st[:33].contiguous()
+    for got, ref in zip(hip.fp8_linear_group(xt, [small[0], wt], [small[1], st]), (want[:, :33], want)):
+        assert _same_values(got, ref)
+    resid = torch.randn(m, n, device=gpu).to(torch.bfloat16)
+    assert torch.equal(hip.fp8_linear_residual(xt, wt, st, resid), resid + want.to(gpu))
