@@ -609,11 +609,13 @@ SegTable seg_table(const Fp8LinearLaunch &p) {
 // step: its loads past K are clamped into the row and both operands are
 // zeroed for the lane groups past K.
 //
-// Block order: the hardware hands workgroup b to XCD b % xcds. The m-tiles of
-// one n-tile get consecutive slots on one XCD, so each weight tile comes from
-// HBM once and from that XCD's L2 for the other m-tiles.
+// Block order: the hardware hands workgroup b to XCD b % xcds. Up to kPBand
+// m-tiles of one n-tile get consecutive slots on one XCD, then the same m-tiles
+// of its next n-tile, so weight tiles come from that XCD's L2 for the band's
+// other m-tiles and the band's activations for its other n-tiles.
 constexpr int kPTileK = 64;
 constexpr int kPWStage = kPTileN * kPTileK;          // 8 KiB weight tile
+constexpr int kPBand = 8;                            // m-tiles an XCD walks before the next n-tile
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -671,9 +673,18 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
   __shared__ __align__(1024) uint8_t lds[S * kStage];
   const int xcd = blockIdx.x % xcds;
   const int slot = blockIdx.x / xcds;
-  const int mt = TM == 128 ? slot % m_tiles : 0;
-  const int sp = TM == 128 ? 0 : slot % splits;
-  const int nt = slot / (TM == 128 ? m_tiles : splits) * xcds + xcd;
+  int mt = 0, sp = 0, nt;
+  if (TM == 128) {
+    const int n_per_xcd = (n_tiles + xcds - 1) / xcds;
+    const int band = slot / (kPBand * n_per_xcd);
+    const int at = slot - band * kPBand * n_per_xcd;
+    const int rows = min(kPBand, m_tiles - band * kPBand);
+    mt = band * kPBand + at % rows;
+    nt = at / rows * xcds + xcd;
+  } else {
+    sp = slot % splits;
+    nt = slot / splits * xcds + xcd;
+  }
   if (nt >= n_tiles) return;  // the last round of n-tiles does not fill every XCD
   int s = 0;
   while (s + 1 < seg.count && nt >= seg.rg0[s + 1]) ++s;
