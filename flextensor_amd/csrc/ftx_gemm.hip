@@ -549,7 +549,7 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void direct_linear_kernel(con
 SegTable seg_table(const Fp8LinearLaunch &p) {
   SegTable t{};
   t.count = p.group;
-  const int64_t rows = p.prefill ? kPTileN : 16 * static_cast<int64_t>(p.waves);  // of one workgroup
+  const int64_t rows = p.prefill ? p.tile_n : 16 * static_cast<int64_t>(p.waves);  // of one workgroup
   int rg = 0, rb = 0;
   int64_t off = 0;
   for (int s = 0; s < p.group; ++s) {
@@ -593,7 +593,7 @@ SegTable seg_table(const Fp8LinearLaunch &p) {
 // same sum): lane group g feeds k = 16g + 8kb + (0..7) to the kb-th of the
 // step's two MFMAs, so one 16-byte weight read per lane covers both MFMAs.
 //
-// Two launch shapes, chosen by the planner (measured on the 70B projection
+// Two launch shapes of 128 x 128 tiles, chosen by the planner (measured on the 70B projection
 // shapes at 512 rows):
 //   * more tiles than CUs: 4 waves (2 x 2, 64 x 64 each), 2 stages (48 KB
 //     LDS, three workgroups per CU);
@@ -614,7 +614,6 @@ SegTable seg_table(const Fp8LinearLaunch &p) {
 // of its next n-tile, so weight tiles come from that XCD's L2 for the band's
 // other m-tiles and the band's activations for its other n-tiles.
 constexpr int kPTileK = 64;
-constexpr int kPWStage = kPTileN * kPTileK;          // 8 KiB weight tile
 constexpr int kPBand = 8;                            // m-tiles an XCD walks before the next n-tile
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -654,60 +653,58 @@ __device__ __forceinline__ void ring_barrier() {
 // 32-bit offset, and the loading wave's LDS address is scalar arithmetic: the
 // per-step address work leaves the vector ALU (about 3% per layer, measured).
 //
-// TM is the tile's activation rows: 128, or 64 for the batches between decode and prefill (mid_linear_wins).
-// Those also split K: workgroup sp of a tile takes the steps from sp * split_steps and writes fp32 sums for
-// fp8_linear_reduce_kernel. Four waves of 32 channels x 64 rows, four stages of 16 KB, two workgroups per CU;
+// Tiles are TM activation rows x TN channels. The smaller ones serve calls that leave the chip idle otherwise
+// (plan_fp8_linear) and the batches between decode and prefill (mid_linear_wins); those also split K: workgroup sp of a tile takes the steps from sp * split_steps and writes fp32 sums for
+// fp8_linear_reduce_kernel. At 64 x 128 four waves of 32 channels x 64 rows, four stages of 16 KB, two
+// workgroups per CU;
 // bound by the weights' bytes (28672 x 8192 at 64 rows: 70.8 us, 3.3 TB/s). Five and eight stages, four steps
 // at least per split and three workgroups per CU were within 5% or slower.
-template <int TM, int WAVES, int S, bool SADDR>
+template <int TM, int TN, int WAVES, int S, bool SADDR>
 __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *__restrict__ x, SegTable seg, int M,
                                                                  int K, int m_tiles, int n_tiles, int xcds, int splits,
                                                                  int split_steps, float *__restrict__ part) {
-  static_assert(TM == 128 ? WAVES == 4 || WAVES == 8 : TM == 64 && WAVES == 4, "4 or 8 waves");
-  constexpr int IT = TM == 128 ? 4 : 2;            // 16-channel weight tiles per wave
-  constexpr int JT = TM == 128 ? 16 / WAVES : 4;   // 16-row activation tiles per wave
+  static_assert(TM == 128 ? TN == 128 && (WAVES == 4 || WAVES == 8) : TM == 64 && WAVES == 4, "4 or 8 waves");
+  constexpr int WN = TM == 64 && TN == 128 ? 4 : 2;       // waves side by side along the channels
+  constexpr int IT = TN / WN / 16;                        // 16-channel weight tiles per wave
+  constexpr int JT = TM / (WAVES / WN) / 16;              // 16-row activation tiles per wave
   constexpr int WROWS = 16 * JT;                   // activation rows per wave
   constexpr int kXStage = TM * kPTileK * 2;
-  constexpr int kStage = kXStage + kPWStage;
-  constexpr int XL = TM / 32;                      // activation loads per loading wave and step, besides 2 weight loads
+  constexpr int kStage = kXStage + TN * kPTileK;
+  constexpr int XL = TM / 32, WL = TN / 64;        // activation and weight loads per loading wave and step
   __shared__ __align__(1024) uint8_t lds[S * kStage];
   const int xcd = blockIdx.x % xcds;
   const int slot = blockIdx.x / xcds;
-  int mt = 0, sp = 0, nt;
-  if (TM == 128) {
-    const int n_per_xcd = (n_tiles + xcds - 1) / xcds;
-    const int band = slot / (kPBand * n_per_xcd);
-    const int at = slot - band * kPBand * n_per_xcd;
-    const int rows = min(kPBand, m_tiles - band * kPBand);
-    mt = band * kPBand + at % rows;
-    nt = at / rows * xcds + xcd;
-  } else {
-    sp = slot % splits;
-    nt = slot / splits * xcds + xcd;
-  }
+  const int sp = TM == 128 ? 0 : slot % splits;
+  const int tile = TM == 128 ? slot : slot / splits;
+  const int n_per_xcd = (n_tiles + xcds - 1) / xcds;
+  const int band = tile / (kPBand * n_per_xcd);
+  const int at = tile - band * kPBand * n_per_xcd;
+  const int rows = min(kPBand, m_tiles - band * kPBand);
+  const int mt = band * kPBand + at % rows;
+  const int nt = at / rows * xcds + xcd;
   if (nt >= n_tiles) return;  // the last round of n-tiles does not fill every XCD
   int s = 0;
   while (s + 1 < seg.count && nt >= seg.rg0[s + 1]) ++s;
   const int N = seg.n[s];
   const uint8_t *__restrict__ w = seg.w[s];
-  const int n_base = (nt - seg.rg0[s]) * kPTileN;
+  const int n_base = (nt - seg.rg0[s]) * TN;
   const int m_base = mt * TM;
 
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int r = lane & 15;
   const int g = lane >> 4;
-  const int wn = TM == 128 ? wave & 1 : wave;
-  const int wm = TM == 128 ? wave >> 1 : 0;
+  const int wn = wave % WN;
+  const int wm = wave / WN;
   const bool loads = WAVES == 4 || wave < 4;
   const int lw = __builtin_amdgcn_readfirstlane(wave & 3);  // uniform: LDS destinations stay scalar
 
   // This lane's load sources: activation rows (lw*XL + t)*8 + lane/8, weight
-  // rows (lw*2 + t)*16 + lane/4, at the chunk the swizzle assigns.
+  // rows (lw*WL + t)*16 + lane/4, at the chunk the swizzle assigns.
   const int xc = ((lane & 7) ^ rot3(lane >> 3)) * 8;        // k offset (elements) within a step
   const int wc = ((lane & 3) ^ ((lane >> 3) & 3)) * 16;     // k offset (bytes) within a step
   const uint8_t *xrow[4];  // XL of them
-  const uint8_t *wrow[2];
+  const uint8_t *wrow[2];  // WL of them
   uint32_t xoff[4], woff[2];  // SADDR: byte offsets of this lane's chunk in step 0
 #pragma unroll
   for (int t = 0; t < XL; ++t) {
@@ -716,8 +713,8 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
     xoff[t] = static_cast<uint32_t>((static_cast<size_t>(gm) * K + xc) * 2);
   }
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int gn = min(n_base + (lw * 2 + t) * 16 + (lane >> 2), N - 1);
+  for (int t = 0; t < WL; ++t) {
+    const int gn = min(n_base + (lw * WL + t) * 16 + (lane >> 2), N - 1);
     wrow[t] = w + static_cast<size_t>(gn) * K;
     woff[t] = static_cast<uint32_t>(static_cast<size_t>(gn) * K + wc);
   }
@@ -734,8 +731,8 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
       for (int t = 0; t < XL; ++t)
         __builtin_amdgcn_global_load_lds(xb + xoff[t], (lds_void *)(base + (lw * XL + t) * 1024), 16, 0, 0);
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
-        __builtin_amdgcn_global_load_lds(wb + woff[t], (lds_void *)(base + kXStage + (lw * 2 + t) * 1024), 16, 0,
+      for (int t = 0; t < WL; ++t)
+        __builtin_amdgcn_global_load_lds(wb + woff[t], (lds_void *)(base + kXStage + (lw * WL + t) * 1024), 16, 0,
                                          0);
       return;
     }
@@ -748,9 +745,9 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
         __builtin_amdgcn_global_load_lds(x + (xoff[t] + static_cast<uint32_t>(kx - xc) * 2),
                                          (lds_void *)(base + (lw * XL + t) * 1024), 16, 0, 0);
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < WL; ++t)
         __builtin_amdgcn_global_load_lds(w + (woff[t] + static_cast<uint32_t>(kw - wc)),
-                                         (lds_void *)(base + kXStage + (lw * 2 + t) * 1024), 16, 0, 0);
+                                         (lds_void *)(base + kXStage + (lw * WL + t) * 1024), 16, 0, 0);
       return;
     }
 #pragma unroll
@@ -758,8 +755,8 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
       __builtin_amdgcn_global_load_lds(xrow[t] + static_cast<size_t>(kx) * 2,
                                        (lds_void *)(base + (lw * XL + t) * 1024), 16, 0, 0);
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-      __builtin_amdgcn_global_load_lds(wrow[t] + kw, (lds_void *)(base + kXStage + (lw * 2 + t) * 1024), 16, 0,
+    for (int t = 0; t < WL; ++t)
+      __builtin_amdgcn_global_load_lds(wrow[t] + kw, (lds_void *)(base + kXStage + (lw * WL + t) * 1024), 16, 0,
                                        0);
   };
 
@@ -795,7 +792,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
   auto step = [&](int st, bool partial) {
     if (loads) {
       if (st + S - 2 < steps)
-        wait_vmcnt<(S - 2) * (XL + 2)>();
+        wait_vmcnt<(S - 2) * (XL + WL)>();
       else
         wait_vmcnt<0>();
     }
@@ -838,7 +835,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
       const int nb = n_base + wn * (16 * IT) + i * 16 + 4 * g;
 #pragma unroll
       for (int j = 0; j < JT; ++j) {
-        const int m = j * 16 + r;
+        const int m = wm * WROWS + j * 16 + r;
         if (m >= M) continue;
         float *dst = pseg + static_cast<size_t>(m) * N + nb;
         if (nb + 3 < N) {
@@ -1031,6 +1028,22 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
     // workgroup; more tiles: 4 waves and 2 stages, three workgroups per CU
     p.waves = (waves == 4 || waves == 8) ? waves : (m_tiles * n_tiles <= cus ? 8 : 4);
     p.small = offsets_fit(p);
+    p.tile_n = kPTileN;
+    // Half of the chip or more would be idle: 64 x 128 tiles, and 64 x 64 while those leave half idle too. A
+    // tile's time is its steps of K one after the other, so smaller tiles end sooner as well. us, 128 x 128
+    // tiles, 64 x 128 and 64 x 64 at k = 8192: 100 rows x 8192 64.6, 58.3, 48.0; 512 x 1024 62.3, 54.8, 44.3;
+    // 200 x 8192 67.2, 60.4, (58.3); with more tiles than that, 512 x 8192 (256 of 128 x 128) 73.2 and 75.8.
+    // Eight stages instead of four: 49.2 against 48.0.
+    if (!waves && m_tiles * n_tiles * 2 <= cus) {
+      p.mid = true;
+      p.waves = 4;
+      p.kc = (k + kPTileK - 1) / kPTileK * kPTileK;
+      p.m_tiles = (m + 63) / 64;
+      p.tile_n = p.m_tiles * n_tiles * 2 <= cus ? 64 : 128;
+      p.row_groups = 0;
+      for (int s = 0; s < group; ++s) p.row_groups += (n[s] + p.tile_n - 1) / p.tile_n;
+      p.grid = p.xcds * p.m_tiles * ((p.row_groups + p.xcds - 1) / p.xcds);
+    }
     return p;
   }
   p.batch_blocks = static_cast<int>((m + 15) / 16);
@@ -1114,6 +1127,7 @@ void plan_mid_linear(Fp8LinearLaunch *p, int cus, int xcds) {
   p->waves = 4;
   p->splits = static_cast<int>(std::max<int64_t>(1, (steps + split_steps - 1) / split_steps));
   p->kc = split_steps * kPTileK;
+  p->tile_n = kPTileN;
   p->m_tiles = 1;
   p->row_groups = n_tiles;
   p->grid = p->xcds * p->splits * ((n_tiles + p->xcds - 1) / p->xcds);
@@ -1169,7 +1183,7 @@ hipError_t launch_direct(const Fp8LinearLaunch &p, hipStream_t stream) {
   return p.m <= 8 ? launch_direct_rows<true, 4>(p, stream) : launch_direct_rows<true, 8>(p, stream);
 }
 
-template <int TM, int WAVES, int S>
+template <int TM, int TN, int WAVES, int S>
 void launch_tiled(const Fp8LinearLaunch &p, const SegTable &seg, float *part, hipStream_t stream) {
   const auto *x = static_cast<const uint8_t *>(p.x);
   const int m = static_cast<int>(p.m), k = static_cast<int>(p.k), mt = static_cast<int>(p.m_tiles),
@@ -1177,10 +1191,10 @@ void launch_tiled(const Fp8LinearLaunch &p, const SegTable &seg, float *part, hi
   const int split_steps = static_cast<int>(p.kc / kPTileK);
   const dim3 grid(static_cast<unsigned>(p.grid)), block(WAVES * kWave);
   if (p.small)
-    hipLaunchKernelGGL((fp8_prefill_kernel<TM, WAVES, S, true>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
+    hipLaunchKernelGGL((fp8_prefill_kernel<TM, TN, WAVES, S, true>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
                        p.splits, split_steps, part);
   else
-    hipLaunchKernelGGL((fp8_prefill_kernel<TM, WAVES, S, false>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
+    hipLaunchKernelGGL((fp8_prefill_kernel<TM, TN, WAVES, S, false>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
                        p.splits, split_steps, part);
 }
 
@@ -1192,14 +1206,14 @@ hipError_t launch_fp8_linear(const Fp8LinearLaunch &p, hipStream_t stream) {
     const SegTable seg = seg_table(p);
     if (p.mid) {
       const bool reduce = p.scratch_bytes > 0;
-      launch_tiled<64, 4, 4>(p, seg, reduce ? static_cast<float *>(p.workspace) : nullptr, stream);
+      (p.tile_n == 64 ? launch_tiled<64, 64, 4, 4> : launch_tiled<64, 128, 4, 4>)(p, seg, reduce ? static_cast<float *>(p.workspace) : nullptr, stream);
       const hipError_t err = hipGetLastError();
       return err != hipSuccess || !reduce ? err : launch_reduce(p, seg, stream);
     }
     if (p.waves == 8)
-      launch_tiled<128, 8, 4>(p, seg, nullptr, stream);
+      launch_tiled<128, 128, 8, 4>(p, seg, nullptr, stream);
     else
-      launch_tiled<128, 4, 2>(p, seg, nullptr, stream);
+      launch_tiled<128, 128, 4, 2>(p, seg, nullptr, stream);
     return hipGetLastError();
   }
   switch (p.batch_blocks) {

@@ -87,10 +87,11 @@ struct Fp8LinearLaunch {
   int epilogue;         // kFp8Epilogue*: what the reduce kernel applies to the outputs
   const void *residual; // bf16 [m, n[0]] for kFp8EpilogueResidual
   bool prefill;       // more than kFp8LinearMaxRows rows: the tiled prefill kernel (no split, no workspace)
-  int64_t m_tiles;    // prefill: tiles of 128 activation rows (row_groups then counts tiles of 128 channels)
+  int64_t m_tiles;    // prefill: tiles of 128 or 64 activation rows (row_groups then counts tiles of tile_n channels)
+  int tile_n;         // prefill: channels of a tile
   int xcds;           // prefill: L2 domains the block order is arranged for
   bool small;         // prefill: 32-bit load offsets reach every operand
-  bool mid;           // prefill with 64-row tiles and K split over workgroups, for batches between decode and prefill
+  bool mid;           // prefill kernel with 64-row tiles; up to 64 rows K may be split over workgroups
   bool direct;        // the one-launch decode kernel: no workspace, a workgroup per 16 channels
   bool bf16;          // direct only: bf16 weights without scales
 };

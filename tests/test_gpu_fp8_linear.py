@@ -753,3 +753,18 @@ def test_kernel_choice_matches_the_oracle_on_both_sides(gpu, default_config, m, 
         assert _same_values(got, ref)
     resid = torch.randn(m, n, device=gpu).to(torch.bfloat16)
     assert torch.equal(hip.fp8_linear_residual(xt, wt, st, resid), resid + want.to(gpu))
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 1000, 1040), (130, 4160, 528), (300, 5003, 208), (1100, 200, 272), (2100, 129, 80)])
+def test_small_prefill_tiles_agree_bitwise_with_the_large_ones(gpu, default_config, m, n, k):
+    """Calls that leave the chip idle run 64 x 128 or 64 x 64 tiles, long ones walk the rows in bands: the same
+    sums in the same order as the fixed 128 x 128 launch shapes, also in a group."""
+    from flextensor_amd import hip
+
+    xt, wt, st = _to_device(*_random_case(m, n, k, seed=m + n), gpu)
+    auto = hip.fp8_linear(xt, wt, st)
+    grouped = hip.fp8_linear_group(xt, [wt[:100].contiguous(), wt], [st[:100].contiguous(), st])
+    for waves in (4, 8):
+        hip.set_fp8_linear_config(waves, 0)
+        assert torch.equal(hip.fp8_linear(xt, wt, st), auto)
+    assert torch.equal(grouped[1], auto) and torch.equal(grouped[0], auto[:, :100])
