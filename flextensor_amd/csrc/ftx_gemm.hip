@@ -40,6 +40,7 @@
 // k values g*16..g*16+15 of a 64-byte piece: the first eight go to one MFMA,
 // the last eight to a second one.
 #include <algorithm>
+#include <type_traits>
 
 #include "ftx_internal.h"
 
@@ -660,7 +661,7 @@ __device__ __forceinline__ void ring_barrier() {
 // bound by the weights' bytes (28672 x 8192 at 64 rows: 70.8 us, 3.3 TB/s). Five and eight stages, four steps
 // at least per split and three workgroups per CU were within 5% or slower.
 template <int TM, int TN, int WAVES, int S, bool SADDR>
-__global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *__restrict__ x, SegTable seg, int M,
+__global__ __launch_bounds__(WAVES * 64, TM == 128 && WAVES == 4 ? 3 : 2) void fp8_prefill_kernel(const uint8_t *__restrict__ x, SegTable seg, int M,
                                                                  int K, int m_tiles, int n_tiles, int xcds, int splits,
                                                                  int split_steps, float *__restrict__ part) {
   static_assert(TM == 128 ? TN == 128 && (WAVES == 4 || WAVES == 8) : TM == 64 && WAVES == 4, "4 or 8 waves");
@@ -778,6 +779,8 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
   for (int i = 0; i < IT; ++i)
 #pragma unroll
     for (int j = 0; j < JT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // 16-row blocks of this wave that hold a row below M
+  const int live = __builtin_amdgcn_readfirstlane(min(JT, max(0, (M - m_base - wm * WROWS + 15) / 16)));
 
   if (loads) {
 #pragma unroll
@@ -789,7 +792,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
   // and every wave has finished reading the buffer the next loads overwrite.
   // `partial` (the final step of a K that is not a multiple of 64) zeroes both
   // operands of the lane groups past K.
-  auto step = [&](int st, bool partial) {
+  auto step = [&](auto blocks, int st, bool partial) {
     if (loads) {
       if (st + S - 2 < steps)
         wait_vmcnt<(S - 2) * (XL + WL)>();
@@ -799,11 +802,13 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
     ring_barrier();
     if (loads && st + S - 1 < steps) issue(st + S - 1);
     const uint8_t *sb = lds + (st % S) * kStage;
-    u32x4 A[IT], B0[JT], B1[JT];
+    constexpr int J = decltype(blocks)::value;
+    if constexpr (J == 0) return;
+    u32x4 A[IT], B0[J + 1], B1[J + 1];  // one spare: J may be 0
 #pragma unroll
     for (int i = 0; i < IT; ++i) A[i] = *reinterpret_cast<const u32x4 *>(sb + aoff[i]);
 #pragma unroll
-    for (int j = 0; j < JT; ++j) {
+    for (int j = 0; j < J; ++j) {
       B0[j] = *reinterpret_cast<const u32x4 *>(sb + boff0[j]);
       B1[j] = *reinterpret_cast<const u32x4 *>(sb + boff1[j]);
     }
@@ -811,23 +816,34 @@ __global__ __launch_bounds__(WAVES * 64) void fp8_prefill_kernel(const uint8_t *
 #pragma unroll
       for (int i = 0; i < IT; ++i) A[i] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int j = 0; j < JT; ++j) B0[j] = B1[j] = u32x4{0u, 0u, 0u, 0u};
+      for (int j = 0; j < J; ++j) B0[j] = B1[j] = u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const bf16x8 a0 = fp8x8_to_bf16(A[i][0], A[i][1]);
       const bf16x8 a1 = fp8x8_to_bf16(A[i][2], A[i][3]);
 #pragma unroll
-      for (int j = 0; j < JT; ++j) {
+      for (int j = 0; j < J; ++j) {
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, as_bf16x8(B0[j]), acc[i][j], 0, 0, 0);
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, as_bf16x8(B1[j]), acc[i][j], 0, 0, 0);
       }
     }
   };
-  for (int st = first; st < min(full, steps); ++st) step(st, false);
-  if (tail && steps > full) step(full, true);
+  // The walk along K for J blocks of 16 rows: fewer than JT in the last tile of the rows, whose blocks past M
+  // hold nothing. Each count has a loop of its own (a choice inside the loop costs 70 registers), and every
+  // loop meets the same barriers.
+  auto walk = [&](auto blocks) {
+    for (int st = first; st < min(full, steps); ++st) step(blocks, st, false);
+    if (tail && steps > full) step(blocks, full, true);
+  };
+  switch (live) {
+    case 0: walk(std::integral_constant<int, 0>{}); break;
+    case 1: walk(std::integral_constant<int, 1>{}); break;
+    case 2: walk(std::integral_constant<int, JT < 2 ? JT : 2>{}); break;
+    case 3: walk(std::integral_constant<int, JT < 3 ? JT : 3>{}); break;
+    default: walk(std::integral_constant<int, JT>{}); break;
+  }
 
-  // lane holds D rows (output channels) 4g..4g+3 of column (activation row) r of every tile
   if (TM != 128 && part != nullptr) {
     float *__restrict__ pseg = part + seg.part0[s] + static_cast<size_t>(sp) * M * N;
 #pragma unroll
