@@ -394,20 +394,27 @@ void plan_attention(AttentionLaunch *p, int cus, int xcds) {
   p->rep = p->heads / p->kv_heads;
   p->rows = p->t * p->rep;
   const int64_t heads = static_cast<int64_t>(p->batch) * p->kv_heads;
-  // The most rows a workgroup can share its K/V tiles over while every CU still gets a workgroup.
+  // Rows per workgroup: as many as share a K/V tile well, as few as fill the chip. A CU's time is about its
+  // workgroups, rounded up, times their rows; half the rows are taken where that makes it 1.4 times shorter.
+  // 12 heads of 2000 x 2000 in workgroups of 128 rows (192 of them) 60.7 us, of 64 rows (384) 75.8, of 32 62.3;
+  // 32 heads of 512 x 512, causal, of 64 rows (256) 19.2 us, of 128 19.8.
+  const auto cost = [&](int waves) {
+    const int64_t groups = heads * ((p->rows + kRowsPerWave * waves - 1) / (kRowsPerWave * waves));
+    return (groups + cus - 1) / cus * waves;
+  };
   p->waves = 8;
-  while (p->waves > 1 && (p->rows <= kRowsPerWave * p->waves / 2 ||
-                          heads * ((p->rows + kRowsPerWave * p->waves - 1) / (kRowsPerWave * p->waves)) < cus))
-    p->waves /= 2;
+  for (int w = 4; w >= 1; w /= 2)
+    if (p->rows <= kRowsPerWave * w || cost(p->waves) * 10 >= cost(w) * 14) p->waves = w;
   p->row_tiles = (p->rows + kRowsPerWave * p->waves - 1) / (kRowsPerWave * p->waves);
   const int kt = p->waves == 8 ? 64 : 32;
   const int tiles = (p->s + kt - 1) / kt;
-  // One-wave workgroups (a decode token, a handful of rows): split the keys until three workgroups per CU
-  // have work, with at least two tiles each.
+  // One-wave workgroups (a decode token, a handful of rows): split the keys until two workgroups per CU have
+  // work, with at least two tiles each. Up to four tiles the combine launch costs more than it saves: 16 heads
+  // over 101 keys 6.7 us, split in two 7.9; over 528 keys of 32 heads 9 splits 10.0 us.
   const int64_t groups = heads * p->row_tiles;
   p->splits = 1;
-  if (p->waves == 1 && groups < cus && tiles > 2) {
-    const int64_t want = std::min<int64_t>((3 * cus + groups - 1) / groups, (tiles + 1) / 2);
+  if (p->waves == 1 && groups < cus && tiles > 4) {
+    const int64_t want = std::min<int64_t>((2 * cus + groups - 1) / groups, (tiles + 1) / 2);
     p->split_tiles = static_cast<int>((tiles + want - 1) / want);
     p->splits = (tiles + p->split_tiles - 1) / p->split_tiles;
   }
