@@ -178,3 +178,22 @@ def test_refusals_happen_on_the_host(gpu, dense):
     assert code(dst.data_ptr(), bad.arena.ptr, bad.nbytes, None, s) == nat.FTX_ERR_INVALID
     torch.cuda.synchronize()
     assert torch.count_nonzero(dst).item() == 0  # nothing ran
+
+
+@pytest.mark.parametrize("maker", [_bf16_bytes, _specials,
+                                   lambda n, s: np.random.default_rng(s).integers(0, 256, n, dtype=np.uint8),
+                                   lambda n, s: np.zeros(n, dtype=np.uint8)])
+@pytest.mark.parametrize("n", [1, 2047, 4097, (1 << 20) + 1, (3 << 20) + 2050])
+def test_dense_decode_from_hbm_at_every_escape_density(gpu, maker, n):
+    """Blocks with no escapes, a few, and more than the 256-byte window of nibbles that a wave holds."""
+    from flextensor_amd import _native as nat
+    from flextensor_amd import expcode
+
+    raw = _raw_tensor(maker(n, 23))
+    block = expcode.DeviceEncodedBlock.from_raw(raw, expcode.encoded_size(raw, dense=True), torch.device(gpu), dense=True)
+    for grid in (0, 3):
+        out = torch.full((n + 16,), 0xA5, dtype=torch.uint8, device=gpu)
+        nat.call("ftx_expcode_decode_dense_d2d", out.data_ptr(), block.dev.data_ptr(), block.nbytes, n, grid,
+                 torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(out[:n].cpu(), raw) and bool((out[n:] == 0xA5).all())
