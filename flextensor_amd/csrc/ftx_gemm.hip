@@ -3,9 +3,11 @@
 //   y[m, n] = bf16( scale[n] * sum_k x[m, k] * w[n, k] )
 //
 // x is bf16 [M, K], w is float8 e4m3fn [N, K] (row-major, K contiguous),
-// scale is one bf16 per output channel, y is bf16 [M, N]. Up to 64 rows
-// (decode) run fp8_linear_kernel below; more rows (prefill) run the tiled
-// fp8_prefill_kernel further down.
+// scale is one bf16 per output channel, y is bf16 [M, N]. A few rows run
+// direct_linear_kernel (which takes bf16 weights too), up to 64 rows (decode)
+// fp8_linear_kernel or 64-row tiles, more rows (prefill) the tiled
+// fp8_prefill_kernel; the rules are at direct_linear_wins, mid_linear_wins and
+// plan_fp8_linear.
 //
 // Decode multiplies a few activation rows by a large weight matrix, so the
 // kernel is bound by reading the fp8 weights from HBM once (1 byte per

@@ -125,9 +125,9 @@ class Fp8Linear(nn.Module):
     """y = x @ (W_fp8 * scale[:, None])^T with W in float8_e4m3fn and a bf16 scale per output channel.
 
     On the GPU (K a multiple of 16) the library's fp8-weight MFMA kernels run:
-    up to 64 rows (decode) a split-K kernel that reads each fp8 weight once,
-    more rows (prefill) a tiled GEMM; both widen the weights to bf16 in
-    registers. The decoder groups its q/k/v and gate/up projections into one
+    a few rows in one launch, up to 64 rows (decode) a split-K kernel or
+    64-row tiles, more rows (prefill) a tiled GEMM; all widen the weights to
+    bf16 in registers. The decoder groups its q/k/v and gate/up projections into one
     launch each (:func:`fp8_group`). CPU inputs dequantise to bf16 and run a
     bf16 GEMM. Every e4m3 value is exactly
     representable in bf16, so both compute the same products; they differ in
