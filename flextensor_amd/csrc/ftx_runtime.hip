@@ -1199,7 +1199,8 @@ int64_t view_extent(const int64_t *stride, int64_t n0, int64_t n1, int64_t n2, i
   const int64_t n[3] = {n0, n1, n2};
   int64_t extent = d;
   for (int i = 0; i < 3; ++i) {
-    if (stride[i] < 0 || stride[i] % 8 != 0 || stride[i] > (int64_t(1) << 40)) return -1;
+    if (stride[i] < 0 || stride[i] % 8 != 0) return -1;
+    if (n[i] > 1 && stride[i] > (int64_t(1) << 40) / (n[i] - 1)) return -1;
     extent += (n[i] - 1) * stride[i];
   }
   return extent;

@@ -190,3 +190,34 @@ def test_event_flags_are_checked_before_the_runtime():
         assert lib.ftx_event_create(bad, ctypes.byref(ev)) == _native.FTX_ERR_INVALID
         assert b"unknown event flags" in lib.ftx_last_error()
     assert (_native.EVENT_TIMING, _native.EVENT_DEVICE_ONLY) == (1, 2)
+
+
+def test_layer_entry_points_refuse_bad_shapes_before_any_device_call():
+    """Head dimensions, head groups, empty keys, alignment of sizes and strides beyond any memory are refused on
+    the host, with no device present."""
+    import ctypes
+
+    from flextensor_amd import _native as nat
+
+    lib = nat.load()
+    b = ctypes.c_size_t(0)
+    for shape, code in (((1, 1, 8, 4, 4, 96), nat.FTX_ERR_UNSUPPORTED), ((1, 1, 8, 4, 3, 64), nat.FTX_ERR_INVALID),
+                        ((1, 1, 0, 4, 4, 64), nat.FTX_ERR_INVALID), ((-1, 1, 8, 4, 4, 64), nat.FTX_ERR_INVALID)):
+        assert lib.ftx_attention_workspace(*shape, ctypes.byref(b)) == code
+    assert lib.ftx_attention_workspace(0, 1, 8, 4, 4, 64, ctypes.byref(b)) == nat.FTX_OK and b.value == 0
+    big = (ctypes.c_int64 * 12)(*[1 << 62] * 12)
+    assert lib.ftx_attention(None, None, None, None, 2, 2, 8, 4, 4, 64, big, 0, 0, 1.0, None, 0, None) == \
+        nat.FTX_ERR_INVALID
+    assert lib.ftx_attention(None, None, None, None, 2, 2, 8, 4, 4, 64, big, 0, 0, 0.0, None, 0, None) == \
+        nat.FTX_ERR_INVALID
+    assert lib.ftx_rope_cache(None, None, None, None, None, None, None, None, 1, 1, 4, 4, 24, 0, big, None) == \
+        nat.FTX_ERR_UNSUPPORTED
+    assert lib.ftx_rope_cache(None, None, None, None, None, None, None, None, 2, 2, 4, 4, 64, 1 << 29, big, None) == \
+        nat.FTX_ERR_INVALID
+    assert lib.ftx_norm(None, None, None, None, 4, 12, nat.NORM_RMS, None, None, None, None, 1, -1, -1, -1, 1e-5,
+                        None) == nat.FTX_ERR_UNSUPPORTED
+    assert lib.ftx_silu_mul(None, None, None, 12, None) == nat.FTX_ERR_UNSUPPORTED
+    n = (ctypes.c_int64 * 1)(64)
+    ptr = (ctypes.c_void_p * 1)(None)
+    assert lib.ftx_bf16_linear(None, 1, ptr, ptr, n, 17, 64, 0, None, None) == nat.FTX_ERR_UNSUPPORTED
+    assert lib.ftx_bf16_linear(None, 1, ptr, ptr, n, 4, 12, 0, None, None) == nat.FTX_ERR_INVALID
