@@ -233,8 +233,9 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : 1) void attention_kernel(
     mx = half_max(mx) * a.scale_log2;
     if (__any(mx > m + kSlack)) {
       const float m_new = fmaxf(m, mx);
-      // a split may hold no key of a row that others of the wave can see: its maximum stays -inf, its sum 0
-      const float alpha = __builtin_amdgcn_exp2f(m - (SPLIT && m_new == -INFINITY ? 0.f : m_new));
+      // the maximum stays -inf and the sum 0 while no key of the row counts: every score so far is -inf, or the
+      // split holds no key of a row that others of the wave can see
+      const float alpha = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));
       m = m_new;
       l *= alpha;
 #pragma unroll
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : 1) void attention_kernel(
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[d][e] *= alpha;
     }
-    const float ref = SPLIT && m == -INFINITY ? 0.f : m;
+    const float ref = m == -INFINITY ? 0.f : m;
     bf16x8 p[2 * kSub];  // 16 keys each, in the order the V reads share
     float sum = 0.f;
 #pragma unroll

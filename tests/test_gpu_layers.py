@@ -100,6 +100,26 @@ def test_attention_passes_nan_and_infinite_scores_on(gpu):
     assert torch.equal(hip.attention(q, k, v)[0, :, 0].isnan().all(-1), s.isnan().any(-1))
 
 
+@pytest.mark.parametrize("blank", [32, 64, 96])
+@pytest.mark.parametrize("b,t,s,h,kv,d,pos", [
+    (1, 1, 100, 4, 4, 128, None), (1, 3, 528, 2, 1, 64, 525),  # one wave: unsplit, split over the keys
+    (2, 64, 128, 256, 32, 128, None), (4, 127, 127, 64, 64, 128, 0), (1, 257, 257, 128, 64, 64, 0),  # 2, 4, 8 waves
+])
+def test_attention_after_keys_that_all_score_minus_infinity(gpu, blank, b, t, s, h, kv, d, pos):
+    """Whole tiles of -inf scores ahead of finite ones weigh nothing, on split and unsplit plans; a causal row that
+    sees only such keys is NaN, as softmax gives."""
+    from flextensor_amd import hip
+
+    print(f"attention blank={blank} b={b} t={t} s={s} h={h}/{kv} d={d} pos={pos}", flush=True)
+    q, k, v = _randn(gpu, b, t, h, d), _randn(gpu, b, s, kv, d, seed=1), _randn(gpu, b, s, kv, d, seed=2)
+    q[..., 0] = q[..., 0].abs() + 1
+    k[:, :blank, :, 0] = float("-inf")
+    want, got = _attend64(q, k, v, pos), hip.attention(q, k, v, pos).cpu()
+    nan = want.isnan()
+    assert bool(nan.any()) == (pos == 0) and torch.equal(got.isnan(), nan)
+    assert _rel(got[~nan], want[~nan]) < TWO_ROUNDINGS
+
+
 def test_attention_refuses_what_the_kernel_cannot_address(gpu):
     from flextensor_amd import _native as nat
     from flextensor_amd import hip
