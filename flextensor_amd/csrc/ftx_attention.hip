@@ -20,10 +20,13 @@
 //
 // K and V go from memory into LDS by buffer loads (no register staging). Their descriptors end with the
 // last key's row, so rows past it read as zero: a ragged end needs no clamped addresses, and a zero weight
-// never meets a value from outside the tensor. Each load writes 1 KB, lane l at +16 l; the layout is chosen
-// by which 16-byte chunk a lane fetches. Chunk c of row R lies at slot c ^ f(R), with f spreading the rows
-// one read touches over all 64 banks: for K (16 bytes of 32 rows a read) f = R % 16 at 256-byte rows and
-// (R / 2) % 8 at 128-byte rows; for V (four rows of 32 bytes a transposed read) 4 (R % 4) and 4 (R / 2 % 2).
+// never meets a value from outside the tensor. Rows that overlap (TIGHT: a position stride below a row, 0 for
+// expanded values) would lie inside the descriptor past the last key too, so V's loads of those rows are sent
+// past its end by row number (in every kernel this cost 1 to 7%); K's need not, their scores are masked by
+// position. Each load writes 1 KB, lane l at +16 l; the layout is chosen by which 16-byte chunk a lane fetches.
+// Chunk c of row R lies at slot c ^ f(R), with f spreading the rows one read touches over all 64 banks: for K
+// (16 bytes of 32 rows a read) f = R % 16 at 256-byte rows and (R / 2) % 8 at 128-byte rows; for V (four rows
+// of 32 bytes a transposed read) 4 (R % 4) and 4 (R / 2 % 2).
 //
 // The maximum is only raised when a score exceeds it by more than 2^kSlack: the probabilities stay below
 // 2^kSlack, keep their relative precision, and the accumulators are rescaled a few times per row instead
@@ -93,7 +96,7 @@ __device__ __forceinline__ void ring_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <int D, int NW, int KT, int STAGES, bool SPLIT>
+template <int D, int NW, int KT, int STAGES, bool SPLIT, bool TIGHT = false>
 __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : 1) void attention_kernel(AttentionLaunch a) {
   constexpr int kRowBytes = 2 * D;
   constexpr int kRowChunks = D / 8;
@@ -161,8 +164,12 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : 1) void attention_kernel(
     for (int i = 0; i < kPerWave; ++i)
       load_to_lds(kb, k_bytes, koff[i] + kt, base + i * 1024);
 #pragma unroll
-    for (int i = 0; i < kPerWave; ++i)
-      load_to_lds(vb, v_bytes, voff[i] + vt, base + kTileBytes + i * 1024);
+    for (int i = 0; i < kPerWave; ++i) {
+      uint32_t offset = voff[i] + vt;
+      if constexpr (TIGHT)
+        if ((wave * kPerWave + i) * kRowsPerLoad + lane / kRowChunks >= a.s - t * KT) offset = v_bytes;
+      load_to_lds(vb, v_bytes, offset, base + kTileBytes + i * 1024);
+    }
   };
 
   // Queries: lane (r, g) holds elements 16 ks + 8 g .. + 7 of its row for every step ks.
@@ -373,6 +380,10 @@ hipError_t launch_shape(const AttentionLaunch &p, hipStream_t stream) {
                          stream, p);
       return hipGetLastError();
     }
+    if (p.tight) {
+      hipLaunchKernelGGL((attention_kernel<D, NW, KT, STAGES, false, true>), grid, dim3(NW * kWave), 0, stream, p);
+      return hipGetLastError();
+    }
   }
   hipLaunchKernelGGL((attention_kernel<D, NW, KT, STAGES, false>), grid, dim3(NW * kWave), 0, stream, p);
   return hipGetLastError();
@@ -403,8 +414,9 @@ void plan_attention(AttentionLaunch *p, int cus, int xcds) {
     const int64_t groups = heads * ((p->rows + kRowsPerWave * waves - 1) / (kRowsPerWave * waves));
     return (groups + cus - 1) / cus * waves;
   };
-  p->waves = 8;
-  for (int w = 4; w >= 1; w /= 2)
+  // Overlapping values run unsplit one-wave workgroups, the only ones built for them.
+  p->waves = p->tight ? 1 : 8;
+  for (int w = 4; w >= 1 && !p->tight; w /= 2)
     if (p->rows <= kRowsPerWave * w || cost(p->waves) * 10 >= cost(w) * 14) p->waves = w;
   p->row_tiles = (p->rows + kRowsPerWave * p->waves - 1) / (kRowsPerWave * p->waves);
   const int kt = p->waves == 8 ? 64 : 32;
@@ -414,7 +426,7 @@ void plan_attention(AttentionLaunch *p, int cus, int xcds) {
   // over 101 keys 6.7 us, split in two 7.9; over 528 keys of 32 heads 9 splits 10.0 us.
   const int64_t groups = heads * p->row_tiles;
   p->splits = 1;
-  if (p->waves == 1 && groups < cus && tiles > 4) {
+  if (p->waves == 1 && groups < cus && tiles > 4 && !p->tight) {
     const int64_t want = std::min<int64_t>((2 * cus + groups - 1) / groups, (tiles + 1) / 2);
     p->split_tiles = static_cast<int>((tiles + want - 1) / want);
     p->splits = (tiles + p->split_tiles - 1) / p->split_tiles;

@@ -125,6 +125,7 @@ struct AttentionLaunch {
   int rep, rows, waves, row_tiles, splits, split_tiles, xcds;
   int64_t items;
   size_t part_bytes;
+  bool tight;                 // given: values overlap, a position stride below a row
 };
 // Fills the planned members from the shapes.
 void plan_attention(AttentionLaunch *p, int cus, int xcds);

@@ -1249,6 +1249,7 @@ int ftx_attention(const void *q, const void *k, const void *v, void *o, int64_t 
                   size_t workspace_bytes, void *stream) {
   FTX_REQUIRE_LIVE();
   ftx::AttentionLaunch p{};
+  p.tight = strides && s > 1 && strides[7] < d;
   int rc = plan_attention_call(batch, t, s, heads, kv_heads, d, &p);
   if (rc != FTX_OK) return rc;
   if (batch == 0 || t == 0) return FTX_OK;
@@ -1288,6 +1289,7 @@ int ftx_attention(const void *q, const void *k, const void *v, void *o, int64_t 
     p.v_stride[i] = strides[6 + i];
     p.o_stride[i] = strides[9 + i];
   }
+  if (s == 1) p.k_stride[1] = p.v_stride[1] = d;  // the rows that fill up its tile end up past the descriptors
   p.causal = causal != 0;
   p.pos = causal ? static_cast<int>(pos) : 0;
   p.scale_log2 = scale * 1.44269504088896340736f;

@@ -120,6 +120,23 @@ def test_attention_after_keys_that_all_score_minus_infinity(gpu, blank, b, t, s,
     assert _rel(got[~nan], want[~nan]) < TWO_ROUNDINGS
 
 
+@pytest.mark.parametrize("s,stride", [(1, 0), (1, 128), (5, 0), (33, 8), (40, 64), (600, 0)])
+@pytest.mark.parametrize("t", [1, 70])
+def test_attention_reads_no_value_past_the_last_key(gpu, s, stride, t):
+    """Keys and values whose rows overlap (a single one, expanded ones, a stride below a row) and hold infinities:
+    the rows that fill up the last tile stay out of the sum."""
+    from flextensor_amd import hip
+
+    print(f"attention s={s} stride={stride} t={t}", flush=True)
+    q, k, v = _randn(gpu, 1, t, 2, 128), _randn(gpu, 2 * (s + 2) * 128, seed=1), _randn(gpu, 2 * (s + 2) * 128, seed=2)
+    v[(s - 1) * stride + 127] = float("inf")  # the end of the last row: inside the rows that would follow it
+    k, v = (x.as_strided((1, s, 2, 128), (0, stride, (s + 2) * 128, 1)) for x in (k, v))
+    want, got = _attend64(q, k, v, None), hip.attention(q, k, v).cpu()
+    inf = want.isinf()
+    assert bool(inf.any()) and torch.equal(got.isinf(), inf) and not bool(got.isnan().any())
+    assert _rel(got[~inf], want[~inf]) < TWO_ROUNDINGS
+
+
 def test_attention_refuses_what_the_kernel_cannot_address(gpu):
     from flextensor_amd import _native as nat
     from flextensor_amd import hip
