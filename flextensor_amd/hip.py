@@ -461,6 +461,8 @@ def residual_norm(x: torch.Tensor, eps: float, delta: torch.Tensor | None = None
     if x.dim() != 3 or not x.numel():
         return None
     b, n, dim = x.shape
+    if affine is not None and (affine[0] is None or affine[1] is None):  # a LayerNorm without a weight or a bias
+        return None
     tensors = [t for t in (x, delta, *(affine or ()), *(adaln or ())) if t is not None]
     if (dim % 8 or dim > NORM_MAX_DIM or b * n >= 1 << 31 or not kernel_call(*tensors) or not _packed(*tensors)
             or (delta is not None and delta.shape != x.shape)

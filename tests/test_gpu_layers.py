@@ -198,6 +198,23 @@ def test_residual_norm_matches_float64(gpu, b, n, dim, residual, norm):
     assert hip.residual_norm(x, 1e-6, delta[:, :, : dim // 2], adaln=(mod, e)) is None
 
 
+@pytest.mark.parametrize("options", [{}, {"bias": False}, {"elementwise_affine": False}])
+def test_dit_block_with_any_layer_norm(gpu, options):
+    """A norm3 without a bias, or without weight and bias, runs as torch's module between the kernels."""
+    from flextensor_amd import workloads as W
+
+    s = W.DiTShape(n_blocks=1, dim=128, n_heads=2, ffn=256)
+    block = W.build_dit(s, seed=3).blocks[0]
+    block.norm3 = torch.nn.LayerNorm(s.dim, eps=s.eps, dtype=torch.bfloat16, **options)
+    x, e, ctx = W.dit_inputs(s, 40, 8, seed=3)
+    with torch.no_grad():
+        for p in block.norm3.parameters():
+            p.uniform_(0.5, 1.5)
+        want = block.float()(x.float(), e.float(), ctx.float())
+        got = block.to(gpu, torch.bfloat16)(x.to(gpu), e.to(gpu), ctx.to(gpu))
+    assert _rel(got.cpu(), want.double()) < 1e-2  # a bf16 block
+
+
 @pytest.mark.parametrize("b,t,h,kv,d,pos", [(1, 1, 1, 1, 16, 0), (2, 3, 8, 2, 64, 5), (1, 65, 5, 5, 128, 0), (3, 1, 64, 8, 128, 40)])
 def test_rope_cache_matches_float64(gpu, b, t, h, kv, d, pos):
     """Rotated queries, and keys and values at their positions; the rest of the caches is left alone."""

@@ -122,6 +122,17 @@ def _ref_dit_block(blk: W.DiTBlock, x, e, ctx):
     return x + (y + f["fc2.bias"]) * m[5]
 
 
+def test_residual_norm_leaves_a_layer_norm_without_weight_or_bias_to_torch(monkeypatch):
+    """With the kernel path open, LayerNorms without a weight or a bias are not the kernel's; nothing is called."""
+    from flextensor_amd import hip
+
+    monkeypatch.setattr(hip, "kernel_call", lambda *ts: True)
+    x = torch.zeros(1, 3, 16, dtype=torch.bfloat16)
+    w = torch.ones(16, dtype=torch.bfloat16)
+    for affine in ((w, None), (None, None)):
+        assert hip.residual_norm(x, 1e-6, x, affine=affine) is None
+
+
 def test_dit_block_matches_float32_restatement():
     shape = W.DiTShape(n_blocks=2, dim=64, n_heads=4, ffn=160)
     model = W.build_dit(shape, seed=7)
