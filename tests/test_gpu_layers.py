@@ -215,6 +215,24 @@ def test_dit_block_with_any_layer_norm(gpu, options):
     assert _rel(got.cpu(), want.double()) < 1e-2  # a bf16 block
 
 
+@pytest.mark.parametrize("dim,n", [(5120, 8000), (256, 40)])
+def test_dit_block_has_the_same_bits_with_its_norm_called_as_a_module(gpu, dim, n):
+    """A hook (as a streamed unit's trap does) makes the block call norm3 instead of folding it into the add."""
+    from flextensor_amd import workloads as W
+
+    s = W.DiTShape(n_blocks=1, dim=dim, n_heads=dim // 128, ffn=256)
+    block = W.build_dit(s, seed=3).blocks[0].to(gpu)
+    x, e, ctx = (t.to(gpu) for t in W.dit_inputs(s, n, 64, seed=3))
+    with torch.no_grad():
+        block.modulation.copy_(_randn(gpu, 1, 6, dim) * 0.3)
+        block.norm3.weight.copy_(_randn(gpu, dim, seed=1) * 0.1 + 1)
+        block.norm3.bias.copy_(_randn(gpu, dim, seed=2))
+        want = block(x, e, ctx)
+        seen = []
+        block.norm3.register_forward_hook(lambda mod, args, out: seen.append(out))
+        assert torch.equal(block(x, e, ctx), want) and len(seen) == 1
+
+
 @pytest.mark.parametrize("b,t,h,kv,d,pos", [(1, 1, 1, 1, 16, 0), (2, 3, 8, 2, 64, 5), (1, 65, 5, 5, 128, 0), (3, 1, 64, 8, 128, 40)])
 def test_rope_cache_matches_float64(gpu, b, t, h, kv, d, pos):
     """Rotated queries, and keys and values at their positions; the rest of the caches is left alone."""
