@@ -437,6 +437,8 @@ NORM_MAX_DIM = 32768
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor | None:
     """``bf16(x * rsqrt(mean(x^2) + eps) * weight)`` over the last dimension in one launch (``ftx_norm``), or
     None when the kernel does not take the call."""
+    if type(x) not in _PLAIN_TYPES:  # a subclass, or a proxy of a symbolic trace
+        return None
     dim = x.shape[-1] if x.dim() else 0
     if (not dim or dim % 8 or dim > NORM_MAX_DIM or not x.numel() or x.numel() // dim >= 1 << 31
             or not kernel_call(x, weight) or weight.shape != (dim,) or not _packed(x, weight)):
@@ -458,7 +460,7 @@ def residual_norm(x: torch.Tensor, eps: float, delta: torch.Tensor | None = None
     are its LayerNorm with ``affine`` (weight, bias), or ``LayerNorm(sum) * (1 + m[scale]) + m[shift]`` for a
     ``scale`` that is not negative. ``m = modulation + e`` from ``adaln``: [1, 6, dim] and [batch, 6, dim].
     """
-    if x.dim() != 3 or not x.numel():
+    if type(x) not in _PLAIN_TYPES or x.dim() != 3 or not x.numel():
         return None
     b, n, dim = x.shape
     if affine is not None and (affine[0] is None or affine[1] is None):  # a LayerNorm without a weight or a bias
@@ -725,6 +727,8 @@ BF16_LINEAR_MAX_ROWS = 16
 
 def bf16_linear_eligible(x: torch.Tensor, *weights: torch.Tensor) -> bool:
     """Whether :func:`bf16_linear` takes ``x`` [..., k] and these weights [n, k]."""
+    if type(x) not in _PLAIN_TYPES:  # a subclass, or a proxy of a symbolic trace
+        return False
     k = x.shape[-1] if x.dim() else 0
     return (k > 0 and 0 < x.numel() <= BF16_LINEAR_MAX_ROWS * k and k % 8 == 0 and kernel_call(x, *weights)
             and all(w.dim() == 2 and w.shape[1] == k and w.shape[0] > 0 for w in weights)

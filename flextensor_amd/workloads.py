@@ -163,9 +163,10 @@ class Linear(nn.Linear):
     """``nn.Linear`` whose forward on a few bf16 GPU rows (a decode batch) is the library's one-launch kernel."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if self.bias is None and hip.bf16_linear_eligible(x, self.weight):
-            return hip.bf16_linear(x, [self.weight])[0]
-        return super().forward(x)
+        if not torch.jit.is_scripting():  # a scripted module holds torch's operation alone
+            if self.bias is None and hip.bf16_linear_eligible(x, self.weight):
+                return hip.bf16_linear(x, [self.weight])[0]
+        return F.linear(x, self.weight, self.bias)
 
 
 def _plain_call(module: nn.Module) -> bool:
@@ -259,9 +260,10 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim, dtype=dtype))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        fused = hip.rms_norm(x, self.weight, self.eps)
-        if fused is not None:
-            return fused
+        if not torch.jit.is_scripting():
+            fused = hip.rms_norm(x, self.weight, self.eps)
+            if fused is not None:
+                return fused
         xf = x.float()
         y = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)
         return (y * self.weight.float()).to(x.dtype)
@@ -474,8 +476,11 @@ class LayerNorm(nn.LayerNorm):
     folds the norm into the residual add before it, also where the module is called on its own (as a streamed unit)."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        fused = hip.residual_norm(x, self.eps, affine=(self.weight, self.bias))
-        return fused[1] if fused is not None else super().forward(x)
+        if not torch.jit.is_scripting():
+            fused = hip.residual_norm(x, self.eps, affine=(self.weight, self.bias))
+            if fused is not None:
+                return fused[1]
+        return F.layer_norm(x, self.normalized_shape, self.weight, self.bias, self.eps)
 
 
 class _DiTAttention(nn.Module):

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import math
 
+import pytest
 import torch
 
 from flextensor_amd import workloads as W
@@ -120,6 +121,20 @@ def _ref_dit_block(blk: W.DiTBlock, x, e, ctx):
     h = ln(x) * (1 + m[4]) + m[3]
     y = torch.nn.functional.gelu(h @ f["fc1.weight"].T + f["fc1.bias"], approximate="tanh") @ f["fc2.weight"].T
     return x + (y + f["fc2.bias"]) * m[5]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_norms_and_projections_trace_symbolically_and_script(dtype):
+    """``torch.fx.symbolic_trace`` and ``torch.jit.script`` of the modules that may run a kernel, with torch's
+    operations in the graph: the results of the module itself."""
+    mods = [W.RMSNorm(32, 1e-5, dtype), W.LayerNorm(32, eps=1e-5, dtype=dtype), W.Linear(32, 16, bias=False, dtype=dtype),
+            W.Linear(32, 16, dtype=dtype)]
+    x = torch.randn(2, 3, 32, generator=torch.Generator().manual_seed(1)).to(dtype)
+    with torch.no_grad():
+        for mod in mods:
+            want = mod(x)
+            assert torch.equal(torch.fx.symbolic_trace(mod)(x), want)
+            assert torch.equal(torch.jit.script(mod)(x), want)
 
 
 def test_residual_norm_leaves_a_layer_norm_without_weight_or_bias_to_torch(monkeypatch):
