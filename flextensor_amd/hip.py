@@ -421,12 +421,47 @@ def _attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, shape: tuple[int,
     return out
 
 
+def _check_operands(what: str, **tensors: torch.Tensor) -> None:
+    """Refuses what a kernel must not read as plain bf16 memory of the current device, or would answer without
+    the derivative that the caller asks for."""
+    for name, t in tensors.items():
+        if type(t) not in _PLAIN_TYPES:
+            raise TypeError(f"{what} takes plain tensors, {name} is a {type(t).__name__}")
+        if t.dtype != torch.bfloat16:
+            raise TypeError(f"{what} takes bf16 tensors, {name} is {t.dtype}")
+    for name, t in tensors.items():
+        if not t.is_cuda or t.get_device() != torch._C._cuda_getDevice():
+            raise ValueError(f"{what} runs on the current GPU, {name} is on {t.device}")
+        if torch.is_grad_enabled() and t.requires_grad:
+            raise ValueError(f"{what} has no backward and {name} requires a gradient")
+        if torch.autograd.forward_ad._current_level >= 0 and torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+            raise ValueError(f"{what} has no forward-mode derivative and {name} carries a tangent")
+
+
 def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: int | None = None) -> torch.Tensor:
     """``softmax(q k^T / sqrt(d)) v`` over bf16 [batch, position, head, d] tensors (``ftx_attention``).
 
     ``k`` and ``v`` may have fewer heads than ``q`` (each shared by a group) and any strides; the result is laid
-    out as q is. ``pos``: query t sees the keys up to ``pos + t``; None: every key.
+    out as q is. ``pos``: query t sees the keys up to ``pos + t``; None: every key. The tensors are on the current
+    device, start at 16-byte boundaries and are contiguous along d, with strides that are multiples of 8; the
+    kernel has no backward.
     """
+    if not q.dim() == k.dim() == v.dim() == 4:
+        raise ValueError(f"attention takes [batch, position, head, d] tensors, got {q.dim()}, {k.dim()} and {v.dim()} "
+                         "dimensions")
+    if k.shape != v.shape or k.shape[0] != q.shape[0] or k.shape[3] != q.shape[3]:
+        raise ValueError(f"attention operands differ in batch, keys or head dimension: q {tuple(q.shape)}, "
+                         f"k {tuple(k.shape)}, v {tuple(v.shape)}")
+    _check_operands("attention", q=q, k=k, v=v)
+    for name, t in (("q", q), ("k", k), ("v", v)):
+        if _head_strides(t) is None:
+            raise ValueError(f"attention reads {name} 16 bytes at a time: it must be contiguous along d and 16-byte "
+                             f"aligned, with strides that are multiples of 8, not {t.stride()}")
+    return attention_unchecked(q, k, v, pos)
+
+
+def attention_unchecked(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: int | None = None) -> torch.Tensor:
+    """:func:`attention` for callers that have asked :func:`attention_eligible`."""
     b, t, h, d = q.shape
     return _attend(q, k, v, (b, t, k.shape[1], h, k.shape[2], d), _head_strides(k), _head_strides(v), pos, _stream())
 
@@ -738,7 +773,29 @@ def bf16_linear_eligible(x: torch.Tensor, *weights: torch.Tensor) -> bool:
 def bf16_linear(x: torch.Tensor, weights: list[torch.Tensor], epilogue: int = nat.FP8_EPILOGUE_NONE,
                 residual: torch.Tensor | None = None) -> list[torch.Tensor]:
     """``[x @ w.T for w in weights]`` for up to 16 bf16 rows in one launch (``ftx_bf16_linear``); under an
-    epilogue one output: ``silu(g) * u`` of two weights, or ``residual + x @ w.T`` of one."""
+    epilogue one output: ``silu(g) * u`` of two weights, or ``residual + x @ w.T`` of one. ``x`` [..., k] and the
+    weights [n, k] are contiguous, 16-byte aligned and on the current device; the kernel has no backward."""
+    k = x.shape[-1] if x.dim() else 0
+    if k == 0:
+        raise ValueError(f"bf16_linear takes x [..., k], got {tuple(x.shape)}")
+    named = {"x": x, **{f"weights[{i}]": w for i, w in enumerate(weights)}}
+    for name, t in named.items():
+        if t is not x and (t.dim() != 2 or t.shape[1] != k):
+            raise ValueError(f"bf16_linear: {name} must be [n, {k}], got {tuple(t.shape)}")
+        if not _packed(t):
+            raise ValueError(f"bf16_linear needs a contiguous, 16-byte aligned {name}")
+    if epilogue == nat.FP8_EPILOGUE_RESIDUAL and residual is not None and weights:
+        shape = (*x.shape[:-1], weights[0].shape[0])
+        if residual.shape != shape or not residual.is_contiguous():
+            raise ValueError(f"residual must be a contiguous {shape} tensor, got {tuple(residual.shape)}")
+        named["residual"] = residual
+    _check_operands("bf16_linear", **named)
+    return bf16_linear_unchecked(x, weights, epilogue, residual)
+
+
+def bf16_linear_unchecked(x: torch.Tensor, weights: list[torch.Tensor], epilogue: int = nat.FP8_EPILOGUE_NONE,
+                          residual: torch.Tensor | None = None) -> list[torch.Tensor]:
+    """:func:`bf16_linear` for callers that have asked :func:`bf16_linear_eligible`."""
     k = x.shape[-1]
     m, g = x.numel() // k, len(weights)
     n_out = 1 if epilogue == nat.FP8_EPILOGUE_SWIGLU else g

@@ -165,7 +165,7 @@ class Linear(nn.Linear):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not torch.jit.is_scripting():  # a scripted module holds torch's operation alone
             if self.bias is None and hip.bf16_linear_eligible(x, self.weight):
-                return hip.bf16_linear(x, [self.weight])[0]
+                return hip.bf16_linear_unchecked(x, [self.weight])[0]
         return F.linear(x, self.weight, self.bias)
 
 
@@ -230,14 +230,14 @@ def _bf16_fusable(x: torch.Tensor, layers: list[nn.Module]) -> bool:
 def linear_group(x: torch.Tensor, layers: list[nn.Module]) -> list[torch.Tensor] | None:
     """The outputs of several linear layers on one input in one launch, or None when no kernel takes the group."""
     if _bf16_fusable(x, layers):
-        return hip.bf16_linear(x, [lin.weight for lin in layers])
+        return hip.bf16_linear_unchecked(x, [lin.weight for lin in layers])
     return fp8_group(x, layers)
 
 
 def linear_swiglu(x: torch.Tensor, gate: nn.Module, up: nn.Module) -> torch.Tensor | None:
     """``F.silu(gate(x)) * up(x)`` in one launch, or None when no kernel takes the call."""
     if _bf16_fusable(x, [gate, up]) and gate.weight.shape == up.weight.shape:
-        return hip.bf16_linear(x, [gate.weight, up.weight], hip.nat.FP8_EPILOGUE_SWIGLU)[0]
+        return hip.bf16_linear_unchecked(x, [gate.weight, up.weight], hip.nat.FP8_EPILOGUE_SWIGLU)[0]
     return fp8_swiglu(x, gate, up)
 
 
@@ -245,7 +245,7 @@ def linear_residual(x: torch.Tensor, lin: nn.Module, residual: torch.Tensor) -> 
     """``residual + lin(x)`` in one launch, or None when no kernel takes the call."""
     if _bf16_fusable(x, [lin]) and hip.kernel_call(residual) and residual.is_contiguous() and \
             residual.shape == (*x.shape[:-1], lin.weight.shape[0]):
-        return hip.bf16_linear(x, [lin.weight], hip.nat.FP8_EPILOGUE_RESIDUAL, residual)[0]
+        return hip.bf16_linear_unchecked(x, [lin.weight], hip.nat.FP8_EPILOGUE_RESIDUAL, residual)[0]
     return fp8_residual(x, lin, residual)
 
 
@@ -463,7 +463,7 @@ def sdpa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
     if q.device.type == "cuda":
         heads = [t.transpose(1, 2) for t in (q, k, v)] if q.dim() == k.dim() == v.dim() == 4 else None
         if heads is not None and q.shape[1] == k.shape[1] and hip.attention_eligible(*heads):
-            return hip.attention(*heads).transpose(1, 2)
+            return hip.attention_unchecked(*heads).transpose(1, 2)
         from torch.nn.attention import SDPBackend, sdpa_kernel
 
         with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):

@@ -319,6 +319,32 @@ def test_bf16_linear_takes_decode_batches_of_plain_modules_only(gpu):
     assert y.requires_grad and _rel(y.detach(), alone.double()) < TWO_ROUNDINGS
 
 
+def test_public_kernel_functions_refuse_what_has_no_answer(gpu):
+    """Host operands, layouts that cannot be read in place and calls that ask for a derivative are refused; the same
+    call on plain operands runs."""
+    import torch.autograd.forward_ad as fwd
+
+    from flextensor_amd import hip
+
+    q, x, w = _randn(gpu, 1, 8, 4, 128), _randn(gpu, 4, 64), _randn(gpu, 32, 64)
+    hip.attention(q, q, q)
+    hip.bf16_linear(x, [w])
+    shifted = torch.empty(q.numel() + 4, dtype=torch.bfloat16, device=gpu)[4:].view_as(q)
+    for args in ((q, q.cpu(), q.cpu()), (shifted, q, q), (q, shifted, q), (q, q, q.transpose(2, 3).contiguous().transpose(2, 3))):
+        with pytest.raises(ValueError):
+            hip.attention(*args)
+    for args in ((x, [w.cpu()]), (x[:, ::2], [w[:, :32].contiguous()]), (x, [w[:, :32].contiguous()]), (x.view(-1)[1:65], [w])):
+        with pytest.raises(ValueError):
+            hip.bf16_linear(*args)
+    for call in (lambda t: hip.attention(t(q), q, q), lambda t: hip.bf16_linear(x, [t(w)])):
+        with pytest.raises(ValueError, match="no backward"):
+            call(lambda a: a.clone().requires_grad_())
+        with fwd.dual_level(), pytest.raises(ValueError, match="forward-mode"):
+            call(lambda a: fwd.make_dual(a, torch.ones_like(a)))
+        with torch.no_grad():
+            call(lambda a: a.clone().requires_grad_())
+
+
 def test_operations_that_must_be_seen_run_in_torch(gpu):
     """Autograd, forward-mode differentiation, function and dispatch modes, functorch transforms and autocast get
     torch's operations; a plain call gets the kernel."""
