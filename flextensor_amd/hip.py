@@ -536,10 +536,11 @@ def _rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, 
         if cache.dim() != 4 or cache.shape[0] < b or cache.shape[1] < pos + t or cache.shape[2:] != (kv, d):
             return None
         strides.append(_head_strides(cache))
-        if strides[-1] is None or 0 in cache.stride():
+        if strides[-1] is None or 0 in cache.stride() or (cache.is_inference() and not torch.is_inference_mode_enabled()):
             return None
     if cache_k.data_ptr() == cache_v.data_ptr():
         return None
+    torch.autograd.graph.increment_version((cache_k, cache_v))  # as an in-place operation, for what autograd saved
     out = torch.empty_like(q)
     nat.call("ftx_rope_cache", q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
              out.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), b, t, h, kv, d, pos,

@@ -148,6 +148,33 @@ def test_public_kernel_functions_refuse_operands_the_kernel_would_misread():
             hip.bf16_linear(*args)
 
 
+def test_cache_writes_are_in_place_operations_to_autograd(monkeypatch):
+    """The kernel's cache writes move the version counters, so a backward that needs the old values is refused, and
+    inference tensors are left to torch (which refuses them) outside inference mode."""
+    from flextensor_amd import hip
+
+    calls = []
+    monkeypatch.setattr(hip, "kernel_call", lambda *ts: True)
+    monkeypatch.setattr(hip, "_stream", lambda device=None: 0)
+    monkeypatch.setattr(hip.nat, "call", lambda name, *args: calls.append(name))
+    q, kv = torch.zeros(1, 2, 4, 16, dtype=torch.bfloat16), torch.zeros(1, 2, 2, 16, dtype=torch.bfloat16)
+    table = torch.zeros(8, 16)
+    caches = [torch.ones(1, 8, 2, 16, dtype=torch.bfloat16) for _ in range(2)]
+    w = torch.ones(16, dtype=torch.bfloat16, requires_grad=True)
+    y = (w * caches[1][:, :4]).sum()
+    with torch.no_grad():
+        assert hip.rope_cache(q, kv, kv, table, table, 2, *caches) is not None and calls == ["ftx_rope_cache"]
+    assert [c._version for c in caches] == [1, 1]
+    with pytest.raises(RuntimeError, match="inplace"):
+        y.backward()
+    with torch.inference_mode():
+        inference = [torch.zeros(1, 8, 2, 16, dtype=torch.bfloat16) for _ in range(2)]
+        assert hip.rope_cache(q, kv, kv, table, table, 2, *inference) is not None
+    with torch.no_grad():
+        assert hip.rope_cache(q, kv, kv, table, table, 2, *inference) is None
+    assert len(calls) == 2
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_norms_and_projections_trace_symbolically_and_script(dtype):
     """``torch.fx.symbolic_trace`` and ``torch.jit.script`` of the modules that may run a kernel, with torch's
