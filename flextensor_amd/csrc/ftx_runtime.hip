@@ -1214,7 +1214,7 @@ int plan_attention_call(int64_t batch, int64_t t, int64_t s, int heads, int kv_h
   if (d != 64 && d != 128) return ftx::fail(FTX_ERR_UNSUPPORTED, "attention runs at head dimensions 64 and 128");
   if (s == 0) return ftx::fail(FTX_ERR_INVALID, "attention over no keys");
   if (batch > kMax || t > kMax || s > kMax || heads > 65536 || t * (heads / kv_heads) > kMax ||
-      batch * heads * std::max<int64_t>(t, 1) > (int64_t(1) << 30))
+      batch * heads > (int64_t(1) << 30) / std::max<int64_t>(t, 1))  // batch * heads * t may not fit 64 bits
     return ftx::fail(FTX_ERR_INVALID, "attention dimensions too large");
   p->batch = static_cast<int>(batch);
   p->t = static_cast<int>(t);
@@ -1353,7 +1353,7 @@ int ftx_rope_cache(const void *q, const void *k, const void *v, const void *cos,
   if (d % 16 != 0 || d > 4096 || heads > 65536 || kv_heads > 65536 || pos > (int64_t(1) << 30))
     return ftx::fail(FTX_ERR_UNSUPPORTED, "rope heads hold a multiple of 16 values, at most 4096");
   if (batch > (int64_t(1) << 24) || t > (int64_t(1) << 24) ||
-      batch * t * (heads + 2 * static_cast<int64_t>(kv_heads)) * d > int64_t(1) << 35)
+      batch * t > (int64_t(1) << 35) / ((heads + 2 * static_cast<int64_t>(kv_heads)) * d))
     return ftx::fail(FTX_ERR_INVALID, "rope dimensions too large");
   if (batch == 0 || t == 0) return FTX_OK;
   if (!cache_strides) return ftx::fail(FTX_ERR_INVALID, "cache_strides is null");

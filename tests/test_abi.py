@@ -221,3 +221,20 @@ def test_layer_entry_points_refuse_bad_shapes_before_any_device_call():
     ptr = (ctypes.c_void_p * 1)(None)
     assert lib.ftx_bf16_linear(None, 1, ptr, ptr, n, 17, 64, 0, None, None) == nat.FTX_ERR_UNSUPPORTED
     assert lib.ftx_bf16_linear(None, 1, ptr, ptr, n, 4, 12, 0, None, None) == nat.FTX_ERR_INVALID
+
+
+def test_layer_size_limits_hold_where_the_product_of_sizes_wraps():
+    """Sizes within each limit whose product is 2^64 are refused as the smaller ones beyond the limit are."""
+    import ctypes
+
+    from flextensor_amd import _native as nat
+
+    lib = nat.load()
+    b = ctypes.c_size_t(0)
+    for t in (1 << 10, 1 << 24):
+        assert lib.ftx_attention_workspace(1 << 24, t, 8, 65536, 65536, 64, ctypes.byref(b)) == nat.FTX_ERR_INVALID
+        assert b"too large" in lib.ftx_last_error()
+    for t in (1 << 12, 1 << 24):  # batch * t * (heads + 2 kv_heads) * d is a multiple of 2^64 for the second
+        assert lib.ftx_rope_cache(None, None, None, None, None, None, None, None, 1 << 24, t, 32768, 16384, 1 << 12, 0,
+                                  None, None) == nat.FTX_ERR_INVALID
+        assert b"too large" in lib.ftx_last_error()
