@@ -1127,6 +1127,7 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
 // rows 4096 x 11008 in 15.6 against 20.0, 11008 x 4096 in 19.6 against 19.8, 8192 x 28672 in 64 against 62.
 // bf16 weights are twice the bytes for the same x, and the library's GEMM takes longer at every size.
 bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k) {
+  if (n_total > kDirectMaxChannels) return false;
   if (m <= 4) return true;
   return m <= 8 ? k <= 16384 : m <= kDirectMaxRows && n_total * k <= int64_t(48) << 20;
 }

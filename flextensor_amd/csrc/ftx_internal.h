@@ -30,6 +30,9 @@ bool is_shut_down();
       return ::ftx::fail(FTX_ERR_UNSUPPORTED, "the library has been shut down (ftx_shutdown)"); \
   } while (0)
 
+// Threads one launch can hold: the runtime refuses grids of 2^32 and more.
+constexpr int64_t kMaxThreads = (int64_t(1) << 32) - 1;
+
 // Default bytes per wave tile of the scatter kernel: one round of 8 loads and
 // 8 non-temporal stores of 16 bytes per lane (fastest of 8/16/32 KiB on the
 // 2000-tensor set's 512 MiB chunks: 5.94 TB/s against 5.78 and 5.77).
@@ -97,6 +100,7 @@ struct Fp8LinearLaunch {
 };
 // The one-launch decode kernel: its most rows, whether it is the faster one for an fp8 call, and its plan.
 constexpr int kDirectMaxRows = 16;
+constexpr int64_t kDirectMaxChannels = (int64_t(1) << 27) - 128;  // 512 threads for 16 of them, within kMaxThreads
 bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k);
 void plan_direct_linear(Fp8LinearLaunch *p);
 // Tiles of 64 rows for the batches between decode and prefill: whether they are faster, and their plan.
@@ -133,6 +137,7 @@ hipError_t launch_attention(const AttentionLaunch &p, hipStream_t stream);
 
 // The operations between a layer's matrix products (ftx_layers.hip). dim is a multiple of 8.
 constexpr int kNormMaxDim = 32768;
+int64_t norm_max_rows(int64_t dim);  // of a launch within kMaxThreads
 constexpr int kNormNone = FTX_NORM_NONE, kNormRms = FTX_NORM_RMS, kNormAffine = FTX_NORM_LAYER,
               kNormAdaln = FTX_NORM_ADALN;
 constexpr int kNormNoResidual = 0, kNormResidual = 1, kNormGatedResidual = 2;
@@ -161,6 +166,7 @@ struct RopeLaunch {
   int batch, t, heads, kv_heads, d;  // d a multiple of 16
 };
 hipError_t launch_rope_cache(const RopeLaunch &p, hipStream_t stream);
+constexpr int64_t kSiluMulMax = (int64_t(1) << 35) - 4096;  // a thread for 8 values, within kMaxThreads
 hipError_t launch_silu_mul(const uint16_t *g, const uint16_t *u, uint16_t *y, int64_t n, hipStream_t stream);
 
 // Staged copies from pageable host memory and the parallel host memcpy

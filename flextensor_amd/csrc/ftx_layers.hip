@@ -243,11 +243,17 @@ hipError_t launch_norm_waves(const NormLaunch &p, hipStream_t stream) {
 
 }  // namespace
 
+int64_t norm_max_rows(int64_t dim) {
+  const int64_t threads = dim <= 2048 ? 64 : dim <= 8192 ? 256 : 1024;  // of a row: launch_norm
+  return kMaxThreads / threads - 3;                                     // workgroups of four rows round up
+}
+
 // A row takes the fewest wavefronts whose registers hold it: one up to 2048 values (64 lanes x 4 vectors of
 // 8), four up to 8192, sixteen up to 32768.
 hipError_t launch_norm(const NormLaunch &p, hipStream_t stream) {
   constexpr int kPerWave = kWave * kVec * kNormVecs;
   static_assert(16 * kPerWave == kNormMaxDim, "the largest row the wavefronts of one workgroup hold");
+  static_assert(kPerWave == 2048, "norm_max_rows counts the same wavefronts");
   if (p.dim <= kPerWave) return launch_norm_waves<1>(p, stream);
   if (p.dim <= 4 * kPerWave) return launch_norm_waves<4>(p, stream);
   return launch_norm_waves<16>(p, stream);

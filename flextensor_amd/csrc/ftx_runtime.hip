@@ -1124,6 +1124,9 @@ int ftx_bf16_linear(const void *x, int group, const void *const *w, void *const 
   }
   if (p.n_total > (int64_t(1) << 30) || k > (int64_t(1) << 29))
     return ftx::fail(FTX_ERR_INVALID, "linear dimensions too large");
+  if (p.n_total > ftx::kDirectMaxChannels)
+    return ftx::fail(FTX_ERR_UNSUPPORTED, "the bf16 linear runs up to " + std::to_string(ftx::kDirectMaxChannels) +
+                                              " channels");
   if (epilogue == ftx::kFp8EpilogueSwiglu) {
     if (group != 2 || n[0] != n[1])
       return ftx::fail(FTX_ERR_INVALID, "the SwiGLU epilogue takes two matrices (gate, up) with the same n");
@@ -1230,6 +1233,8 @@ int plan_attention_call(int64_t batch, int64_t t, int64_t s, int heads, int kv_h
     xcds = st->xcd_count;
   }
   ftx::plan_attention(p, cus, xcds);
+  if (p->items + p->xcds > ftx::kMaxThreads / (64 * p->waves))  // the grid is a multiple of xcds
+    return ftx::fail(FTX_ERR_UNSUPPORTED, "attention: more workgroups than one launch holds");
   return FTX_OK;
 }
 
@@ -1308,6 +1313,7 @@ int ftx_norm(const void *x, const void *delta, void *x_out, void *y, int64_t row
   if (gate > 5 || (gate >= 0 && !delta)) return ftx::fail(FTX_ERR_INVALID, "the gate is one of six terms on a delta");
   if (norm == FTX_NORM_ADALN && (scale < 0 || scale > 5 || shift < 0 || shift > 5))
     return ftx::fail(FTX_ERR_INVALID, "scale and shift are each one of six terms");
+  if (rows > ftx::norm_max_rows(dim)) return ftx::fail(FTX_ERR_UNSUPPORTED, "norm: more rows than one launch holds");
   if (rows == 0) return FTX_OK;
   const int64_t n = rows * dim;
   int rc = check_operand(x, n, 2, "norm input");
@@ -1398,6 +1404,7 @@ int ftx_silu_mul(const void *g, const void *u, void *y, int64_t n, void *stream)
   FTX_REQUIRE_LIVE();
   if (n < 0 || n > (int64_t(1) << 40)) return ftx::fail(FTX_ERR_INVALID, "silu_mul size");
   if (n % 8 != 0) return ftx::fail(FTX_ERR_UNSUPPORTED, "silu_mul takes a multiple of 8 values");
+  if (n > ftx::kSiluMulMax) return ftx::fail(FTX_ERR_UNSUPPORTED, "silu_mul: more values than one launch holds");
   if (n == 0) return FTX_OK;
   int rc = check_operand(g, n, 2, "silu_mul gate");
   if (rc == FTX_OK) rc = check_operand(u, n, 2, "silu_mul up");

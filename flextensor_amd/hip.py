@@ -386,6 +386,7 @@ def _head_strides(t: torch.Tensor) -> tuple[int, int, int] | None:
 def _attention_sizes(b: int, t: int, s: int, h: int, kv: int, d: int, position_stride: int) -> bool:
     return (d in (64, 128) and b > 0 and t > 0 and s > 0 and kv > 0 and h > 0 and h % kv == 0
             and max(b, t * (h // kv), s) <= 1 << 24 and h <= 65536 and b * h * t <= 1 << 30
+            and b * kv * ((t * (h // kv) + 31) // 32) < (1 << 26) - 64  # workgroups of one wave in one launch
             and (s + 256) * 2 * position_stride < 1 << 31)
 
 
@@ -469,13 +470,18 @@ def attention_unchecked(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: 
 NORM_MAX_DIM = 32768
 
 
+def _norm_rows_fit(rows: int, dim: int) -> bool:
+    """Whether one launch (fewer than 2^32 threads) holds these rows of 1, 4 or 16 waves."""
+    return rows * (64 if dim <= 2048 else 256 if dim <= 8192 else 1024) <= (1 << 32) - 4096
+
+
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor | None:
     """``bf16(x * rsqrt(mean(x^2) + eps) * weight)`` over the last dimension in one launch (``ftx_norm``), or
     None when the kernel does not take the call."""
     if type(x) not in _PLAIN_TYPES:  # a subclass, or a proxy of a symbolic trace
         return None
     dim = x.shape[-1] if x.dim() else 0
-    if (not dim or dim % 8 or dim > NORM_MAX_DIM or not x.numel() or x.numel() // dim >= 1 << 31
+    if (not dim or dim % 8 or dim > NORM_MAX_DIM or not x.numel() or not _norm_rows_fit(x.numel() // dim, dim)
             or not kernel_call(x, weight) or weight.shape != (dim,) or not _packed(x, weight)):
         return None
     y = torch.empty_like(x)
@@ -501,8 +507,8 @@ def residual_norm(x: torch.Tensor, eps: float, delta: torch.Tensor | None = None
     if affine is not None and (affine[0] is None or affine[1] is None):  # a LayerNorm without a weight or a bias
         return None
     tensors = [t for t in (x, delta, *(affine or ()), *(adaln or ())) if t is not None]
-    if (dim % 8 or dim > NORM_MAX_DIM or b * n >= 1 << 31 or not kernel_call(*tensors) or not _packed(*tensors)
-            or (delta is not None and delta.shape != x.shape)
+    if (dim % 8 or dim > NORM_MAX_DIM or not _norm_rows_fit(b * n, dim) or not kernel_call(*tensors)
+            or not _packed(*tensors) or (delta is not None and delta.shape != x.shape)
             or (affine is not None and not affine[0].shape == affine[1].shape == (dim,))
             or (adaln is not None and (adaln[0].shape != (1, 6, dim) or adaln[1].shape != (b, 6, dim)))):
         return None
@@ -521,8 +527,9 @@ def _rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, 
     """:func:`rope_cache`, with the caches' strides: ``(rotated q, cache_k strides, cache_v strides)``."""
     b, t, h, d = q.shape
     kv = k.shape[2]
-    if (type(pos) is not int or pos < 0 or d % 16 or not q.numel() or k.shape != (b, t, kv, d) or v.shape != k.shape
-            or not _packed(q, k, v)):
+    if (type(pos) is not int or pos < 0 or d % 16 or d > 4096 or max(b, t) > 1 << 24 or max(h, kv) > 65536
+            or pos > 1 << 30 or b * t * (h + 2 * kv) * d > 1 << 35 or not q.numel() or k.shape != (b, t, kv, d)
+            or v.shape != k.shape or not _packed(q, k, v)):
         return None
     grad = torch.is_grad_enabled()
     device = q.get_device()
@@ -577,10 +584,11 @@ def rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch
 def silu_mul(g: torch.Tensor, u: torch.Tensor) -> torch.Tensor | None:
     """``bf16(bf16(silu(g)) * u)`` in one launch (``ftx_silu_mul``), or None when the kernel does not take the
     call."""
-    if g.shape != u.shape or not g.numel() or g.numel() % 8 or not kernel_call(g, u) or not _packed(g, u):
+    n = g.numel()
+    if g.shape != u.shape or not n or n % 8 or n > (1 << 35) - 4096 or not kernel_call(g, u) or not _packed(g, u):
         return None
     y = torch.empty_like(g)
-    nat.call("ftx_silu_mul", g.data_ptr(), u.data_ptr(), y.data_ptr(), g.numel(), _stream())
+    nat.call("ftx_silu_mul", g.data_ptr(), u.data_ptr(), y.data_ptr(), n, _stream())
     return y
 
 
@@ -766,8 +774,9 @@ def bf16_linear_eligible(x: torch.Tensor, *weights: torch.Tensor) -> bool:
     if type(x) not in _PLAIN_TYPES:  # a subclass, or a proxy of a symbolic trace
         return False
     k = x.shape[-1] if x.dim() else 0
-    return (k > 0 and 0 < x.numel() <= BF16_LINEAR_MAX_ROWS * k and k % 8 == 0 and kernel_call(x, *weights)
+    return (0 < k <= 1 << 29 and 0 < x.numel() <= BF16_LINEAR_MAX_ROWS * k and k % 8 == 0 and kernel_call(x, *weights)
             and all(w.dim() == 2 and w.shape[1] == k and w.shape[0] > 0 for w in weights)
+            and sum(w.shape[0] for w in weights) <= (1 << 27) - 128  # channels of one launch
             and _packed(x, *weights))
 
 

@@ -328,9 +328,9 @@ int ftx_fp8_linear_scratch(int64_t m, const int64_t *n, int group, int64_t k, in
 /* No counterpart in the reference. Decode-sized linears with bf16 weights, m <=
  * 16, in one launch and without workspace: y[s] = bf16(x @ w[s]^T) for up to
  * four matrices [n[s], k] that share x [m, k] (k a multiple of 8; x and w
- * contiguous and 16-byte aligned), fp32 sums. Epilogues and their group shapes
- * as for ftx_fp8_linear_fused, with y[0] the one output. Each output's sum has
- * the same order alone and in any group. */
+ * contiguous and 16-byte aligned; fewer than 2^27 channels in all), fp32 sums.
+ * Epilogues and their group shapes as for ftx_fp8_linear_fused, with y[0] the one
+ * output. Each output's sum has the same order alone and in any group. */
 int ftx_bf16_linear(const void *x, int group, const void *const *w, void *const *y, const int64_t *n, int64_t m,
                     int64_t k, int epilogue, const void *residual, void *stream);
 

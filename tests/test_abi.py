@@ -238,3 +238,26 @@ def test_layer_size_limits_hold_where_the_product_of_sizes_wraps():
         assert lib.ftx_rope_cache(None, None, None, None, None, None, None, None, 1 << 24, t, 32768, 16384, 1 << 12, 0,
                                   None, None) == nat.FTX_ERR_INVALID
         assert b"too large" in lib.ftx_last_error()
+
+
+def test_launches_beyond_the_threads_of_a_grid_are_refused_or_planned_otherwise():
+    """A launch holds fewer than 2^32 threads: the layer entry points refuse more before any operand is looked at,
+    and an fp8 linear of that many channels keeps the split-K kernel (whose workspace shows it)."""
+    import ctypes
+
+    from flextensor_amd import _native as nat
+
+    lib = nat.load()
+    b = ctypes.c_size_t(0)
+    assert lib.ftx_attention_workspace(1 << 24, 1, 8, 64, 64, 64, ctypes.byref(b)) == nat.FTX_ERR_UNSUPPORTED
+    assert lib.ftx_attention_workspace(1 << 19, 1, 8, 64, 64, 64, ctypes.byref(b)) == nat.FTX_OK
+    for rows, dim in ((1 << 26, 2048), (1 << 24, 8192), (1 << 22, 32768)):
+        assert lib.ftx_norm(None, None, None, None, rows, dim, nat.NORM_RMS, None, None, None, None, 1, -1, -1, -1, 1e-5,
+                            None) == nat.FTX_ERR_UNSUPPORTED
+    assert lib.ftx_silu_mul(None, None, None, 1 << 35, None) == nat.FTX_ERR_UNSUPPORTED
+    ptr = (ctypes.c_void_p * 1)(None)
+    n = (ctypes.c_int64 * 1)(1 << 27)
+    assert lib.ftx_bf16_linear(None, 1, ptr, ptr, n, 4, 64, 0, None, None) == nat.FTX_ERR_UNSUPPORTED
+    for channels, split in ((1 << 26, False), (1 << 28, True)):
+        n[0] = channels
+        assert lib.ftx_fp8_linear_scratch(4, n, 1, 4096, 0, ctypes.byref(b)) == nat.FTX_OK and (b.value > 0) == split

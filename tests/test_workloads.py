@@ -175,6 +175,33 @@ def test_cache_writes_are_in_place_operations_to_autograd(monkeypatch):
     assert len(calls) == 2
 
 
+def test_calls_beyond_one_launch_are_left_to_torch(monkeypatch):
+    """Sizes whose launch would hold 2^32 threads or more are not the kernels', the ones just below are."""
+    from flextensor_amd import hip
+
+    calls = []
+    monkeypatch.setattr(hip, "kernel_call", lambda *ts: True)
+    monkeypatch.setattr(hip, "_stream", lambda device=None: 0)
+    monkeypatch.setattr(hip.nat, "call", lambda name, *args: calls.append(name))
+
+    def meta(*shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device="meta")
+
+    for dim, rows in ((64, 1 << 26), (2056, 1 << 24), (8200, 1 << 22)):
+        for count, takes in ((rows, False), (rows - 64, True)):
+            calls.clear()
+            assert (hip.rms_norm(meta(count, dim), meta(dim), 1e-5) is not None) == takes == bool(calls)
+            calls.clear()
+            x = meta(2, count // 2, dim)
+            assert (hip.residual_norm(x, 1e-6, x) is not None) == takes == bool(calls)
+    assert hip.silu_mul(meta(1 << 35), meta(1 << 35)) is None and hip.silu_mul(meta(1 << 34), meta(1 << 34)) is not None
+    for tokens, takes in ((1 << 20, False), (1 << 19, True)):
+        q = meta(tokens, 1, 64, 64)
+        assert hip.attention_eligible(q, q, q) == takes
+    for channels, takes in ((1 << 27, False), (1 << 26, True)):
+        assert hip.bf16_linear_eligible(meta(1, 8), meta(channels, 8)) == takes
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_norms_and_projections_trace_symbolically_and_script(dtype):
     """``torch.fx.symbolic_trace`` and ``torch.jit.script`` of the modules that may run a kernel, with torch's
