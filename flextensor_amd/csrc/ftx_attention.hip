@@ -376,8 +376,8 @@ hipError_t launch_shape(const AttentionLaunch &p, hipStream_t stream) {
       hipError_t err = hipGetLastError();
       if (err != hipSuccess) return err;
       const int64_t lanes = static_cast<int64_t>(p.batch) * p.kv_heads * p.rows * (D / 4);
-      hipLaunchKernelGGL((attention_combine_kernel<D>), dim3(static_cast<unsigned>((lanes + 255) / 256)), dim3(256), 0,
-                         stream, p);
+      hipLaunchKernelGGL((attention_combine_kernel<D>), dim3(static_cast<unsigned>((lanes + 255) / 256)), dim3(256),
+                         kLdsToken, stream, p);
       return hipGetLastError();
     }
     if (p.tight) {

@@ -280,13 +280,8 @@ __global__ __launch_bounds__(512) void fp8_linear_kernel(const uint8_t *__restri
 constexpr int kReduceVec = 4;
 constexpr int kReduceBatch = 8;
 constexpr int kReduceThreads = 256;
-// LDS the reduce asks for and never touches: one allocation granule. A ring
-// copy running beside a streamed decode holds its CUs' whole LDS (a small
-// zero-copy grid), so with any LDS request the reduce's workgroups stay off
-// those CUs. A workgroup that does share a CU with the copy queues behind the
-// copy's outstanding host reads: in a streamed 70B decode the SwiGLU reduce
-// took 45 us (median) against 5 us alone, the q/k/v reduce 26 against 5.
-constexpr unsigned kReduceLdsToken = 512;
+// The reduce asks for kLdsToken bytes of LDS: in a streamed 70B decode, where it shared CUs with the ring copy,
+// the SwiGLU reduce took 45 us (median) against 5 us alone, the q/k/v reduce 26 against 5.
 
 // Sum over slices of kReduceVec consecutive partials starting at i0 (fewer at the end of MN).
 __device__ __forceinline__ void sum_slices(const float *__restrict__ p, int64_t MN, int64_t i0, int splits,
@@ -996,7 +991,7 @@ hipError_t launch_reduce(const Fp8LinearLaunch &p, const SegTable &seg, hipStrea
   // the SwiGLU epilogue writes one output per gate/up pair: the gate's blocks only
   const int blocks = p.epilogue == kFp8EpilogueSwiglu ? seg.rb0[1] : seg.rb0[p.group];
   hipLaunchKernelGGL(fp8_linear_reduce_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kReduceThreads),
-                     kReduceLdsToken, stream, static_cast<const float *>(p.workspace), seg, static_cast<int>(p.m),
+                     kLdsToken, stream, static_cast<const float *>(p.workspace), seg, static_cast<int>(p.m),
                      p.splits, p.epilogue, static_cast<const uint16_t *>(p.residual));
   return hipGetLastError();
 }

@@ -43,6 +43,11 @@ constexpr int kZeroCopyDefaultGrid = 64;
 // A zero-copy launch of at most this many workgroups takes each CU it runs on
 // whole (its workgroups reserve the CU's LDS).
 constexpr int kZeroCopyReserveMaxGrid = 16;
+// LDS that kernels without LDS of their own ask for and never touch when they run between a layer's products:
+// one allocation granule. A ring copy beside a streamed pass holds its CUs' whole LDS (a small zero-copy grid),
+// so with any LDS request a workgroup stays off those CUs; one that shares a CU with the copy queues behind the
+// copy's outstanding host reads.
+constexpr unsigned kLdsToken = 512;
 // Wave tiles handled by one workgroup (one tile per wavefront).
 constexpr int kScatterWavesPerGroup = 4;
 // Checksum block: 64 lanes x 8 bytes x 8 steps.

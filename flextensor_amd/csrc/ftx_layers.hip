@@ -8,6 +8,11 @@
 //                       to their place in the KV cache.
 //  * silu_mul_kernel  - silu(gate) * up.
 //
+// All ask for some LDS (kLdsToken), which keeps their workgroups off the CUs that a streamed pass's copy holds.
+// Traced beside that copy, us (median) without and with it: silu_mul of 64 x 5504 12.2 and 3.8, of 128 x 28672
+// 18.8 and 8.5; the rotary kernel for 64 tokens of 32 heads 12.1 and 5.3; the combine of 64 heads (attention)
+// 26.3 and 6.3.
+//
 // All are bound by the bytes they read and write (for a decode token by the launch itself). Arithmetic is
 // fp32; values round to bf16 where they are stored. As separate elementwise operations an RMSNorm is six
 // launches that move each value 12 times (17 us for 8 rows of 8192 and 55 us for 512 rows), the rotary
@@ -223,11 +228,12 @@ template <int WAVES, int RESIDUAL>
 hipError_t launch_norm_residual(const NormLaunch &p, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(WAVES == 1 ? (p.rows + 3) / 4 : p.rows));
   const dim3 block(WAVES == 1 ? 256 : WAVES * kWave);
+  constexpr unsigned lds = kLdsToken;  // a row within one wave, or without a norm, has none of its own
   switch (p.norm) {
-    case kNormNone: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormNone>), grid, block, 0, stream, p); break;
-    case kNormRms: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormRms>), grid, block, 0, stream, p); break;
-    case kNormAffine: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormAffine>), grid, block, 0, stream, p); break;
-    default: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormAdaln>), grid, block, 0, stream, p); break;
+    case kNormNone: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormNone>), grid, block, lds, stream, p); break;
+    case kNormRms: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormRms>), grid, block, lds, stream, p); break;
+    case kNormAffine: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormAffine>), grid, block, lds, stream, p); break;
+    default: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormAdaln>), grid, block, lds, stream, p); break;
   }
   return hipGetLastError();
 }
@@ -261,14 +267,15 @@ hipError_t launch_norm(const NormLaunch &p, hipStream_t stream) {
 
 hipError_t launch_rope_cache(const RopeLaunch &p, hipStream_t stream) {
   const int64_t lanes = static_cast<int64_t>(p.batch) * p.t * (p.heads + 2 * p.kv_heads) * (p.d / 2 / kVec);
-  hipLaunchKernelGGL(rope_cache_kernel, dim3(static_cast<unsigned>((lanes + 255) / 256)), dim3(256), 0, stream, p);
+  hipLaunchKernelGGL(rope_cache_kernel, dim3(static_cast<unsigned>((lanes + 255) / 256)), dim3(256), kLdsToken,
+                     stream, p);
   return hipGetLastError();
 }
 
 hipError_t launch_silu_mul(const uint16_t *g, const uint16_t *u, uint16_t *y, int64_t n, hipStream_t stream) {
   const int64_t per_block = 256 * kVec;
-  hipLaunchKernelGGL(silu_mul_kernel, dim3(static_cast<unsigned>((n + per_block - 1) / per_block)), dim3(256), 0,
-                     stream, g, u, y, n);
+  hipLaunchKernelGGL(silu_mul_kernel, dim3(static_cast<unsigned>((n + per_block - 1) / per_block)), dim3(256),
+                     kLdsToken, stream, g, u, y, n);
   return hipGetLastError();
 }
 

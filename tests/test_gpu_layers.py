@@ -270,6 +270,40 @@ def test_silu_mul_matches_float64(gpu, n):
     assert hip.silu_mul(g[1:], u[1:]) is None
 
 
+def test_small_kernels_stay_off_the_cus_of_a_ring_copy(gpu):
+    """Beside a copy that holds its 16 CUs, a silu_mul or rotary launch takes 11 us (2.1 and 2.6 alone); where their
+    workgroups may share those CUs and queue behind the copy's host reads, 26."""
+    from flextensor_amd import _native as nat
+    from flextensor_amd import hip
+
+    g, q, kv = _randn(gpu, 64, 5504), _randn(gpu, 1, 64, 32, 128), _randn(gpu, 1, 64, 32, 128, seed=1)
+    table, caches = torch.ones(64, 128, device=gpu), [torch.empty_like(kv) for _ in range(2)]
+    host = torch.empty(256 << 20, dtype=torch.uint8, pin_memory=True)
+    dst, side, policy = torch.empty_like(host, device=gpu), torch.cuda.Stream(), nat.copy_policy(0, 2**63 - 1, 1, 16)
+    for name, call in (("silu_mul", lambda: hip.silu_mul(g, g)),
+                       ("rope_cache", lambda: hip.rope_cache(q, kv, kv, table, table, 0, *caches))):
+        graph = torch.cuda.CUDAGraph()
+        call()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+            for _ in range(50):
+                call()
+        best = {}
+        for beside in (False, True) * 4:
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            if beside:
+                nat.copy_h2d(dst.data_ptr(), host.data_ptr(), dst.numel(), nat.COPY_MODES["kernel"], side.cuda_stream,
+                             policy)
+            start.record()
+            graph.replay()
+            end.record()
+            torch.cuda.synchronize()
+            best[beside] = min(best.get(beside, math.inf), start.elapsed_time(end) * 20)
+        print(f"{name}: {best[False]:.2f} us alone, {best[True]:.2f} beside the copy", flush=True)
+        assert best[True] < 7 * best[False]
+        del graph
+
+
 @pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("ns,k", [((1,), 8), ((17, 16), 120), ((15, 300, 64), 136), ((257,), 2056), ((4096,), 1024)])
 def test_bf16_linear_matches_float64(gpu, m, ns, k):
