@@ -528,8 +528,12 @@ class DiTBlock(nn.Module):
         adaln = (self.modulation, e)
         eps = self.s.eps
 
-        def m() -> torch.Tensor:
-            return self.modulation.float() + e.float()
+        terms = []
+
+        def m() -> torch.Tensor:  # made once, by the first operation that no kernel takes
+            if not terms:
+                terms.append(self.modulation.float() + e.float())
+            return terms[0]
 
         fused = hip.residual_norm(x, eps, adaln=adaln, scale=1, shift=0)
         h = fused[1] if fused is not None else self._modulate(x, m(), 1, 0)

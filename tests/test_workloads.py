@@ -216,6 +216,26 @@ def test_norms_and_projections_trace_symbolically_and_script(dtype):
             assert torch.equal(torch.jit.script(mod)(x), want)
 
 
+def test_dit_block_adds_its_modulation_once():
+    """The six AdaLN terms of a block are made once when torch's operations run, as for training."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    sums = []
+
+    class Sums(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            if func is torch.ops.aten.add.Tensor and out.shape == (1, 6, 64):
+                sums.append(func)
+            return out
+
+    s = W.DiTShape(n_blocks=1, dim=64, n_heads=4, ffn=160)
+    model = W.build_dit(s, seed=7)
+    with Sums():
+        model(*W.dit_inputs(s, 24, 8, seed=7))
+    assert len(sums) == 1
+
+
 def test_residual_norm_leaves_a_layer_norm_without_weight_or_bias_to_torch(monkeypatch):
     """With the kernel path open, LayerNorms without a weight or a bias are not the kernel's; nothing is called."""
     from flextensor_amd import hip
