@@ -111,13 +111,27 @@ def test_split_calls_in_a_row_stay_exact(gpu, default_config):
             assert _same_values(got, want)
 
 
-def test_graph_replays_match_eager(gpu, default_config):
-    """Captured split-K calls (main kernel + reduce) replay exactly, with eager calls between replays."""
+def _scratch(m, ns, k, epilogue=0) -> int:
+    """Bytes of partial sums a call touches: 0 where it runs in one launch."""
+    import ctypes
+
+    from flextensor_amd import _native as nat
+
+    b = ctypes.c_size_t(0)
+    nat.call("ftx_fp8_linear_scratch", m, (ctypes.c_int64 * len(ns))(*ns), len(ns), k, epilogue, ctypes.byref(b))
+    return b.value
+
+
+# Fixed launch shapes run the split-K kernel; chosen ones run one launch at 8 rows here and 64-row tiles at 33.
+@pytest.mark.parametrize("m,config,split", [(8, (8, 1024), True), (8, (0, 0), False), (33, (0, 0), True)])
+def test_graph_replays_match_eager(gpu, default_config, m, config, split):
+    """Captured calls (main kernel + reduce, or one launch) replay exactly, with eager calls between replays."""
     from flextensor_amd import hip
 
-    x, w_raw, scale = _random_case(8, 4096, 8192, seed=11)
+    hip.set_fp8_linear_config(*config)
+    x, w_raw, scale = _random_case(m, 4096, 8192, seed=11)
     xt, wt, st = _to_device(x, w_raw, scale, gpu)
-    assert hip.fp8_linear_workspace_bytes(8, 4096, 8192) > 0
+    assert (_scratch(m, [4096], 8192) > 0) == split
     eager = hip.fp8_linear(xt, wt, st)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
@@ -368,9 +382,12 @@ def test_group_70b_projections_match_float64_oracle(gpu, default_config, ns):
         assert float((got - one.double().cpu()).norm() / want.norm()) < 1e-3
 
 
-def test_group_graph_replays_match_eager(gpu, default_config):
+@pytest.mark.parametrize("config,split", [((4, 1024), True), ((0, 0), False)])
+def test_group_graph_replays_match_eager(gpu, default_config, config, split):
     from flextensor_amd import hip
 
+    hip.set_fp8_linear_config(*config)
+    assert (_scratch(8, [2048, 512, 512], 4096) > 0) == split
     cases = [_random_case(8, n, 4096, seed=n) for n in (2048, 512, 512)]
     xt = _to_device(*cases[0], gpu)[0]
     dev = [_to_device(cases[0][0], w_raw, scale, gpu)[1:] for _, w_raw, scale in cases]
@@ -532,7 +549,7 @@ def test_prefill_weight_over_2gib_takes_the_wide_address_path(gpu, default_confi
 # ---- fused epilogues: SwiGLU after gate/up, the residual add after o and down ---------------------------
 
 _FUSED_SHAPES = [(1, 16, 16), (8, 1024, 8192), (5, 100, 48), (3, 300, 256), (17, 96, 1040), (64, 512, 256),
-                 (8, 8192, 28672)]
+                 (8, 8192, 28672), (24, 8200, 2064), (33, 2050, 2064), (64, 4100, 2064)]  # three of 64-row tiles under SwiGLU
 
 
 def _fused_call(nat, x, ws, ss, epilogue, residual=None, out=None):
@@ -626,17 +643,24 @@ def test_swiglu_epilogue_matches_the_oracle_and_the_separate_operations(gpu, def
                                                   f"{int((differ & ~near).sum())} away from a midpoint"
 
 
-def test_fused_epilogues_with_one_k_slice_and_in_graphs(gpu, default_config):
-    """A call with one K slice still goes through the partials (the reduce applies the epilogue), and a
+# One K slice of the split-K kernel, the one-launch kernel, and 64-row tiles whose K is split.
+@pytest.mark.parametrize("m,n,k,config,scratch", [(4, 64, 256, (4, 256), 4 * 4 * 64), (4, 64, 256, (0, 0), 0),
+                                                  (33, 4100, 2064, (0, 0), None)])
+def test_fused_epilogues_with_one_k_slice_and_in_graphs(gpu, default_config, m, n, k, config, scratch):
+    """A split-K call with one K slice still goes through the partials (the reduce applies the epilogue), and a
     captured graph of fused calls replays to the eager results."""
+    from flextensor_amd import _native as nat
     from flextensor_amd import hip
 
-    x, wg, sg = _random_case(4, 64, 256, seed=1)
-    _, wu, su = _random_case(4, 64, 256, seed=2)
+    hip.set_fp8_linear_config(*config)
+    x, wg, sg = _random_case(m, n, k, seed=1)
+    _, wu, su = _random_case(m, n, k, seed=2)
     xt, wgt, sgt = _to_device(x, wg, sg, gpu)
     _, wut, sut = _to_device(x, wu, su, gpu)
-    resid = torch.randn(4, 64, device=gpu).to(torch.bfloat16)
-    assert hip.fp8_linear_fused_workspace_bytes(4, [64], 256, 2) > 0
+    resid = torch.randn(m, n, device=gpu).to(torch.bfloat16)
+    for epilogue, ns in ((nat.FP8_EPILOGUE_RESIDUAL, [n]), (nat.FP8_EPILOGUE_SWIGLU, [n, n])):
+        got = _scratch(m, ns, k, epilogue)
+        assert got > 4 * m * sum(ns) if scratch is None else got == scratch * len(ns)
     assert torch.equal(hip.fp8_linear_residual(xt, wgt, sgt, resid), resid + hip.fp8_linear(xt, wgt, sgt))
     eager = (hip.fp8_linear_swiglu(xt, wgt, sgt, wut, sut), hip.fp8_linear_residual(xt, wgt, sgt, resid))
     side = torch.cuda.Stream()
@@ -649,6 +673,8 @@ def test_fused_epilogues_with_one_k_slice_and_in_graphs(gpu, default_config):
             static = (hip.fp8_linear_swiglu(xt, wgt, sgt, wut, sut), hip.fp8_linear_residual(xt, wgt, sgt, resid))
     torch.cuda.current_stream().wait_stream(side)
     for _ in range(3):
+        for out in static:
+            out.zero_()
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(static[0], eager[0]) and torch.equal(static[1], eager[1])

@@ -42,12 +42,15 @@ def test_static_scratch_entry_point_matches_the_workspace_one(gpu):
 
     stream = torch.cuda.current_stream(gpu).cuda_stream
     gen = torch.Generator(device=gpu).manual_seed(11)
-    # a 70B down projection at batch 8 (16 K slices), then a smaller call that uses less of the scratch
-    for m, n, k in ((8, 8192, 28672), (3, 1024, 4096), (8, 8192, 28672)):
+    # a 70B down projection at batch 8 (split K), a smaller call that uses less of the scratch, 64-row tiles with K
+    # split, then the first again
+    for m, n, k in ((8, 8192, 28672), (8, 1024, 20480), (33, 2048, 8192), (8, 8192, 28672)):
         print(f"fp8 linear static: m={m} n={n} k={k}", flush=True)
         x, w, sc = _operands(gen, m, n, k, gpu)
         want, ws_bytes = _with_workspace(nat, x, w, sc, stream)
-        assert ws_bytes > 0  # the call does use split-K partials
+        touched = ctypes.c_size_t(0)
+        nat.call("ftx_fp8_linear_scratch", m, (ctypes.c_int64 * 1)(n), 1, k, 0, ctypes.byref(touched))
+        assert ws_bytes >= touched.value > 0  # the call does use partial sums
         got = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu)
         nat.call("ftx_fp8_linear_static", x.data_ptr(), w.data_ptr(), sc.data_ptr(), got.data_ptr(), m, n, k, stream)
         torch.cuda.synchronize()
