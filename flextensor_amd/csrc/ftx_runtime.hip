@@ -1182,12 +1182,12 @@ int ftx_fp8_linear_static(const void *x, const void *w, const void *scale, void 
   if (m == 0 || n == 0) return FTX_OK;
   if (p.workspace_bytes > FTX_FP8_STATIC_SCRATCH_BYTES)
     return ftx::fail(FTX_ERR_UNSUPPORTED,
-                     "fp8 linear of " + std::to_string(m) + " x " + std::to_string(n) + " x " + std::to_string(k) +
-                         " needs " + std::to_string(p.workspace_bytes) + " bytes of split-K partial sums, more than "
-                         "the static scratch's " + std::to_string(FTX_FP8_STATIC_SCRATCH_BYTES) +
+                     "the workspace of an fp8 linear of " + std::to_string(m) + " x " + std::to_string(n) + " x " +
+                         std::to_string(k) + " (ftx_fp8_linear_workspace, " + std::to_string(p.workspace_bytes) +
+                         " bytes) exceeds the static scratch's " + std::to_string(FTX_FP8_STATIC_SCRATCH_BYTES) +
                          " bytes; call ftx_fp8_linear with a workspace instead");
   void *ws = nullptr;
-  if (p.workspace_bytes > 0) {
+  if (p.scratch_bytes > 0) {
     rc = ftx::static_scratch(&ws);
     if (rc != FTX_OK) return rc;
   }

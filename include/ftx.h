@@ -273,7 +273,7 @@ int ftx_scatter(const void *chunk, const ftx_desc *descs, int n_desc, void *stre
  * bytes, 16-byte aligned; it may be NULL when that size is 0) and a second
  * kernel adds them in slice order, so results are deterministic for a given
  * launch shape. More rows (prefill) run a tiled GEMM (128 x 128 output tiles,
- * whole K per tile) that needs no workspace.
+ * smaller ones for calls of few tiles, whole K per tile) that needs no workspace.
  * Calls that share a workspace must be ordered on one stream.
  * ftx_set_fp8_linear_config fixes the decode launch shape (0 = chosen per
  * call): waves (wavefronts per workgroup, 16 output rows each, 1..8) and
@@ -321,8 +321,9 @@ int ftx_fp8_linear_fused(const void *x, int group, const void *const *w, const v
                          size_t workspace_bytes, void *stream);
 
 /* Bytes of workspace a call of this group and epilogue touches under the launch
- * shape in force: 0 for calls that run in one launch, which then accept a NULL
- * workspace; otherwise what the queries above return. */
+ * shape in force, never more than the queries above return: 0 for calls that run
+ * in one launch, which then accept a NULL workspace, and less than the queries
+ * where 64-row tiles split K less often. A workspace of this size is enough. */
 int ftx_fp8_linear_scratch(int64_t m, const int64_t *n, int group, int64_t k, int epilogue, size_t *bytes);
 
 /* No counterpart in the reference. Decode-sized linears with bf16 weights, m <=
@@ -343,7 +344,8 @@ int ftx_bf16_linear(const void *x, int group, const void *const *w, void *const 
  * on holds until the process ends. Same operands, results and launch shape as
  * ftx_fp8_linear; allocates nothing (no hipMalloc, hipFree or allocating
  * library call). Returns FTX_ERR_UNSUPPORTED, before touching any operand,
- * when the call's partial sums (ftx_fp8_linear_workspace) exceed the array.
+ * when the call's ftx_fp8_linear_workspace exceeds the array, also where the
+ * kernel that would run touches less (ftx_fp8_linear_scratch).
  * Every call on one GPU shares that GPU's array: calls that may overlap on one
  * GPU (unordered streams, other host threads) race and must be ordered, e.g.
  * on one stream. Every partial sum a call reads is written by that call

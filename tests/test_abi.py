@@ -261,3 +261,18 @@ def test_launches_beyond_the_threads_of_a_grid_are_refused_or_planned_otherwise(
     for channels, split in ((1 << 26, False), (1 << 28, True)):
         n[0] = channels
         assert lib.ftx_fp8_linear_scratch(4, n, 1, 4096, 0, ctypes.byref(b)) == nat.FTX_OK and (b.value > 0) == split
+
+
+def test_static_scratch_refusal_names_the_workspace_it_is_measured_by():
+    import ctypes
+
+    from flextensor_amd import _native as nat
+
+    lib = nat.load()
+    b, touched = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    m, n, k = 64, 28672, 8192
+    assert lib.ftx_fp8_linear_workspace(m, n, k, ctypes.byref(b)) == nat.FTX_OK
+    assert lib.ftx_fp8_linear_scratch(m, (ctypes.c_int64 * 1)(n), 1, k, 0, ctypes.byref(touched)) == nat.FTX_OK
+    assert touched.value < 64 << 20 < b.value
+    assert lib.ftx_fp8_linear_static(None, None, None, None, m, n, k, None) == nat.FTX_ERR_UNSUPPORTED
+    assert f"ftx_fp8_linear_workspace, {b.value} bytes" in lib.ftx_last_error().decode()

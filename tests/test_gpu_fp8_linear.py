@@ -548,8 +548,9 @@ def test_prefill_weight_over_2gib_takes_the_wide_address_path(gpu, default_confi
 
 # ---- fused epilogues: SwiGLU after gate/up, the residual add after o and down ---------------------------
 
+# The last three run 64-row tiles under SwiGLU.
 _FUSED_SHAPES = [(1, 16, 16), (8, 1024, 8192), (5, 100, 48), (3, 300, 256), (17, 96, 1040), (64, 512, 256),
-                 (8, 8192, 28672), (24, 8200, 2064), (33, 2050, 2064), (64, 4100, 2064)]  # three of 64-row tiles under SwiGLU
+                 (8, 8192, 28672), (24, 8200, 2064), (33, 2050, 2064), (64, 4100, 2064)]
 
 
 def _fused_call(nat, x, ws, ss, epilogue, residual=None, out=None):
