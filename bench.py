@@ -829,8 +829,8 @@ def bench_fp8_linear(batch: int = 8, reps: int = 20) -> dict:
     Every projection has its own weights (858 MB per layer, more than the
     256 MB Infinity Cache, so no call finds the previous call's weights
     cached). The layer runs as the decoder runs it: grouped calls for q/k/v
-    and for gate/up, single calls for o and down, each the main kernel plus,
-    when K is split, one reduce launch. Algorithmic bytes per call = fp8
+    and for gate/up, single calls for o and down, each one launch, or the main
+    kernel and one reduce launch where K is split. Algorithmic bytes per call = fp8
     weights (n*k) + bf16 activations (m*k*2) + bf16 outputs (m*n*2) + bf16
     scales (n*2). GPU time: ``reps`` layers captured in one HIP graph (two
     layers' weights alternated), one replay timed with HIP events on the
@@ -899,7 +899,7 @@ def bench_fp8_linear(batch: int = 8, reps: int = 20) -> dict:
     layer_ms = graph_ms(lambda i: [run_call(layers[i % n_layers], names, k) for _, names, k in calls], reps)
     # The same projections with the operations that consume their outputs, as the decoder runs them: the
     # residual add after o and after down, SiLU(gate) * up before down (whose input it is). Separately
-    # (torch's bf16 ops after each call), then with those ops folded into the calls' reduce kernels.
+    # (torch's bf16 ops after each call), then with those ops folded into the calls' last launch.
     resid = torch.randn(batch, h, device=dev, generator=gen).to(torch.bfloat16)
 
     def path_separate(i):
@@ -923,10 +923,11 @@ def bench_fp8_linear(batch: int = 8, reps: int = 20) -> dict:
     for label, names, k in calls:
         ms = graph_ms(lambda i, names=names, k=k: run_call(layers[i % n_layers], names, k), reps)
         nb = nbytes(names, k)
-        ws = hip.fp8_linear_group_workspace_bytes(batch, [rows[nm] for nm in names], k)
+        ws = hip.fp8_linear_scratch_bytes(batch, tuple(rows[nm] for nm in names), k)
         per_call.append({"call": label, "matrices": list(names), "k": k, "us": round(ms * 1e3, 2),
                          "GBps": round(nb / ms / 1e6, 1), "algorithmic_bytes": nb,
-                         "k_slices": ws // (4 * batch * sum(rows[nm] for nm in names)) or 1})
+                         "k_slices": ws // (4 * batch * sum(rows[nm] for nm in names)) or 1,
+                         "kernel": "fp8_linear_kernel + fp8_linear_reduce_kernel" if ws else "direct_linear_kernel"})
     ungrouped_ms = graph_ms(lambda i: [hip.fp8_linear(xs[k], *layers[i % n_layers][nm]) for nm, _, k in projections], reps)
     # accuracy of every output against float32, and the dequantize-then-GEMM forward it replaces
     errs = {}
@@ -979,7 +980,7 @@ def bench_fp8_linear(batch: int = 8, reps: int = 20) -> dict:
             "frac_of_plain_read": round(read_ms / layer_ms, 4),
             "layer_ungrouped_us": round(ungrouped_ms * 1e3, 2), "layer_dequant_gemm_us": round(dq_ms * 1e3, 2),
             "rel_err_vs_fp32": errs, "timing": f"HIP graph of {reps} layers (two layers' weights alternated), one replay",
-            "roofline": {"kernel": "fp8_linear_kernel + fp8_linear_reduce_kernel (grouped q/k/v and gate/up)",
+            "roofline": {"kernel": ", ".join(f"{c['call']}: {c['kernel']}" for c in per_call),
                          "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                          "frac": round(achieved / HBM_PEAK_GBPS, 4), "algorithmic_bytes_per_layer": int(layer_bytes),
                          "per": "decoder layer (4 calls)"},

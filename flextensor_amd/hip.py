@@ -607,8 +607,8 @@ def fp8_linear_workspace_bytes(m: int, n: int, k: int) -> int:
     return got
 
 
-def _fp8_scratch_bytes(m: int, ns: tuple[int, ...], k: int, epilogue: int) -> int:
-    """Bytes of workspace a call touches under the launch shape in force (cached per shape)."""
+def fp8_linear_scratch_bytes(m: int, ns: tuple[int, ...], k: int, epilogue: int = nat.FP8_EPILOGUE_NONE) -> int:
+    """Bytes of workspace a call touches under the launch shape in force, 0 for one launch (cached per shape)."""
     key = ("scratch", epilogue, m, k) + ns
     got = _FP8_WORKSPACE.get(key)
     if got is None:
@@ -652,7 +652,7 @@ def fp8_linear(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> to
     if not scale.is_contiguous():
         scale = scale.contiguous()
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    ws_bytes = _fp8_scratch_bytes(m, (n,), k, nat.FP8_EPILOGUE_NONE)
+    ws_bytes = fp8_linear_scratch_bytes(m, (n,), k, nat.FP8_EPILOGUE_NONE)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     nat.call("ftx_fp8_linear", x.data_ptr(), weight.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n, k,
              ws.data_ptr() if ws is not None else None, ws_bytes, _stream(x.get_device()))
@@ -696,7 +696,7 @@ def fp8_linear_group(x: torch.Tensor, weights: list[torch.Tensor], scales: list[
     g = len(weights)
     ns = (ctypes.c_int64 * g)(*[w.shape[0] for w in weights])
     outs = [torch.empty((m, w.shape[0]), dtype=torch.bfloat16, device=x.device) for w in weights]
-    ws_bytes = _fp8_scratch_bytes(m, tuple(ns), k, nat.FP8_EPILOGUE_NONE)
+    ws_bytes = fp8_linear_scratch_bytes(m, tuple(ns), k, nat.FP8_EPILOGUE_NONE)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     ptrs = [(ctypes.c_void_p * g)(*[t.data_ptr() for t in ts]) for ts in (weights, scales, outs)]
     nat.call("ftx_fp8_linear_group", x.data_ptr(), g, *ptrs, ns, m, k, ws.data_ptr() if ws is not None else None,
@@ -737,7 +737,7 @@ def _fp8_fused(x: torch.Tensor, weights: list[torch.Tensor], scales: list[torch.
     g = len(weights)
     ns = [w.shape[0] for w in weights]
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    ws_bytes = _fp8_scratch_bytes(m, tuple(ns), k, epilogue)
+    ws_bytes = fp8_linear_scratch_bytes(m, tuple(ns), k, epilogue)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
     arrays = [(ctypes.c_void_p * g)(*[t.data_ptr() for t in ts]) for ts in (weights, scales)]
     n_arr = (ctypes.c_int64 * g)(*ns)
