@@ -364,12 +364,12 @@ __global__ __launch_bounds__(kReduceThreads) void fp8_linear_reduce_kernel(const
 // Weights and the window of x that meets them go through per-wave LDS tiles, as the weights do in
 // fp8_linear_kernel: loads cover whole rows and MFMA operands are read back in their layout. Weights are e4m3
 // (with a scale per channel) or bf16 (without): a 256-byte window is 256 or 128 values of k, a 64-byte step
-// two MFMAs or one. Two windows are in flight per wave and two workgroups fit a CU; 32 channels per
-// workgroup read x half as often but need 140 registers, one workgroup per CU (28672 x 8192 fp8 in 57
-// against 41 us).
+// two MFMAs or one. Two windows are in flight per wave and two workgroups fit a CU (one at 9 to 16 fp8 rows, whose
+// tiles take 100 KB of LDS); 32 channels per workgroup read x half as often but need 140 registers, one workgroup
+// per CU (28672 x 8192 fp8 in 57 against 41 us).
 //
 // The sum's order depends on K alone, not on the grouping or on M: a projection gives the same bits on its
-// own and in a group.
+// own and in a group that also runs this kernel (direct_linear_wins looks at an fp8 group's channels together).
 //
 // Bound by the weight bytes. Measured in a row on distinct weights, us: fp8 at 1 / 8 rows, before (split-K
 // and reduce) and here: 1024 x 8192 7.7 / 8.6 and 6.6 / 8.2, 4096 x 4096 8.8 / 10.0 and 6.7 / 7.2,
@@ -1115,16 +1115,42 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
   return p;
 }
 
-// Where the one-launch kernel is the faster one. Its workgroups read all of x from L2, M / 8 bytes per fp8
-// weight, which the split-K kernel's 128-channel workgroups do not. Up to 4 rows it always wins (above). Of
-// 5 to 8 rows it loses where K is long and N does not make up for it: 8192 x 28672 at 8 rows in 48.1 us
-// against 45.1, 4096 x 11008 in 13.5 against 15.9. From 9 to 16 rows it wins on small matrices only: at 16
-// rows 4096 x 11008 in 15.6 against 20.0, 11008 x 4096 in 19.6 against 19.8, 8192 x 28672 in 64 against 62.
-// bf16 weights are twice the bytes for the same x, and the library's GEMM takes longer at every size.
-bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k) {
-  if (n_total > kDirectMaxChannels) return false;
-  if (m <= 4) return true;
-  return m <= 8 ? k <= 16384 : m <= kDirectMaxRows && n_total * k <= int64_t(48) << 20;
+// Where the one-launch kernel is the faster one: both it and the plan of plan_fp8_linear measured at 1, 3, 4, 8, 9
+// and 16 rows of K = 512 .. 28672 and 512 .. 131072 channels, plain and under SwiGLU (1580 calls, graph replays on
+// distinct weights). Ratios below are its time by the other's; its line is crossed by 6% at most at 9 of them.
+//
+//  * Short K, many channels: a workgroup's 16 channels give its eight waves K / 2048 windows each (twice that under
+//    SwiGLU, hence `depth`), so launching, filling and summing it is most of its time, once per 16 channels, while
+//    wide plans of one K slice pay no reduce. At 8 rows 8192 x 512 0.70 and 10240 x 512 1.15; 22016 x 1024 0.91 and
+//    45056 x 1024 1.07 (131072: 1.74); 28672 x 2048 1.00 and 45056 x 2048 1.10; 45056 x 4096 1.02 and 65536 x 4096
+//    1.05 (1.15 at 4 rows); 65536 x 5120 and all longer ones below 1.02. One or two rows stage less of x: 65536 x
+//    2048 1.00, 131072 x 2048 1.16.
+//  * Long K, few channels: one workgroup walks the whole of K, on each of a few CUs. At 4 rows 1024 x 11008 0.89,
+//    512 x 11008 1.05, 2048 x 16384 0.94, 1024 x 16384 1.07, 3072 x 28672 0.99, 2048 x 28672 1.25.
+//  * 5 to 8 rows of a longer K: 8192 x 28672 at 8 rows in 48.1 us against 45.1.
+//  * 9 to 16 rows take 100 KB of LDS, one workgroup per CU, and read as much of x as of the weights from L2: small
+//    matrices only. At 9 rows 8192 x 4096 0.97 and 10240 x 4096 1.13, 12288 x 1024 0.92 and 14336 x 1024 1.10, under
+//    SwiGLU 12288 x 512 0.97 and 14336 x 512 1.14; at 16 rows 2048 x 11008 0.91 and 1024 x 11008 1.09.
+//
+// bf16 weights are twice the bytes for the same x and their only other kernel is the library's GEMM, which takes
+// longer at every one of 19 shapes from 512 x 1024 to 152064 x 5120 at 1, 2, 4, 8, 12 and 16 rows. us at 1 / 8 / 16
+// rows, here and the library: 4096 x 4096 8.4 / 8.5 / 9.4 and 15.4 / 15.6 / 15.5; 11008 x 4096 17.4 / 18.0 / 20.3 and
+// 26.7 / 25.7 / 25.6; 32000 x 4096 (a head) 42.2 / 42.1 / 47.8 and 58.9 / 56.8 / 56.9; 128256 x 4096 157 / 156 / 179
+// and 182 / 184 / 186; 8192 x 28672 71.7 / 74.7 / 85.1 and 85.9 / 86.5 / 87.9; closest 1024 x 8192 at 16 rows, 12.0
+// and 12.1.
+bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k, int epilogue) {
+  if (m > kDirectMaxRows || n_total > kDirectMaxChannels) return false;
+  const int64_t matrices = epilogue == kFp8EpilogueSwiglu ? 2 : 1;  // of a workgroup
+  const int64_t channels = n_total / matrices;                      // 16 of them to a workgroup
+  if (m > 8)
+    return n_total * k <= int64_t(48) << 20 &&
+           channels <= (matrices == 2 || (k >= 1024 && k <= 2048) ? 12288 : 8192) && (k < 8192 || k <= 6 * channels);
+  if (m > 4 && k > 16384) return false;
+  if ((k > 8192 && k >= 16 * channels) || (k > 12288 && k > 10 * channels)) return false;
+  const int64_t depth = matrices * k;
+  if (depth >= 5120) return true;
+  if (m <= 2 && k >= 1536) return channels <= 32 * std::max<int64_t>(k, 2048);
+  return channels <= (depth < 1024 ? 8192 : 11 * depth + 17407);
 }
 
 // Where tiles of 64 rows beat the split-K decode kernel, whose workgroups hold all rows of x for their slice of

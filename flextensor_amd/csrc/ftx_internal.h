@@ -106,7 +106,7 @@ struct Fp8LinearLaunch {
 // The one-launch decode kernel: its most rows, whether it is the faster one for an fp8 call, and its plan.
 constexpr int kDirectMaxRows = 16;
 constexpr int64_t kDirectMaxChannels = (int64_t(1) << 27) - 128;  // 512 threads for 16 of them, within kMaxThreads
-bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k);
+bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k, int epilogue);
 void plan_direct_linear(Fp8LinearLaunch *p);
 // Tiles of 64 rows for the batches between decode and prefill: whether they are faster, and their plan.
 bool mid_linear_wins(int64_t m, int64_t n_total, int64_t k);

@@ -973,7 +973,7 @@ int plan_fp8(int64_t m, const int64_t *n, int group, int64_t k, ftx::Fp8LinearLa
   *p = ftx::plan_fp8_linear(m, n, group, k, cus, xcds, waves, slice_k, epilogue);
   if (p->grid > (int64_t(1) << 31) - 1) return ftx::fail(FTX_ERR_INVALID, "fp8 linear grid too large");
   if (!waves && !slice_k && m <= ftx::kFp8LinearMaxRows) {  // no fixed launch shape
-    if (ftx::direct_linear_wins(m, p->n_total, k))
+    if (ftx::direct_linear_wins(m, p->n_total, k, epilogue))
       ftx::plan_direct_linear(p);
     else if (ftx::mid_linear_wins(m, p->n_total, k))
       ftx::plan_mid_linear(p, cus, xcds);

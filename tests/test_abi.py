@@ -260,7 +260,7 @@ def test_launches_beyond_the_threads_of_a_grid_are_refused_or_planned_otherwise(
     assert lib.ftx_bf16_linear(None, 1, ptr, ptr, n, 4, 64, 0, None, None) == nat.FTX_ERR_UNSUPPORTED
     for channels, split in ((1 << 26, False), (1 << 28, True)):
         n[0] = channels
-        assert lib.ftx_fp8_linear_scratch(4, n, 1, 4096, 0, ctypes.byref(b)) == nat.FTX_OK and (b.value > 0) == split
+        assert lib.ftx_fp8_linear_scratch(4, n, 1, 8192, 0, ctypes.byref(b)) == nat.FTX_OK and (b.value > 0) == split
 
 
 def test_static_scratch_refusal_names_the_workspace_it_is_measured_by():
@@ -276,3 +276,21 @@ def test_static_scratch_refusal_names_the_workspace_it_is_measured_by():
     assert touched.value < 64 << 20 < b.value
     assert lib.ftx_fp8_linear_static(None, None, None, None, m, n, k, None) == nat.FTX_ERR_UNSUPPORTED
     assert f"ftx_fp8_linear_workspace, {b.value} bytes" in lib.ftx_last_error().decode()
+
+
+@pytest.mark.parametrize("m,n,k,one_launch", [
+    (1, 65536, 2048, True), (1, 65552, 2048, False), (3, 39935, 2048, True), (3, 39936, 2048, False),
+    (8, 8192, 512, True), (8, 8193, 512, False), (1, 28671, 1024, True), (1, 28672, 1024, False),
+    (8, 131072, 5120, True), (4, 65536, 4096, False), (4, 1024, 11008, True), (4, 512, 11008, False),
+    (1, 2048, 16384, True), (1, 1024, 16384, False), (4, 4096, 28672, True), (5, 4096, 28672, False),
+    (9, 8192, 4096, True), (9, 8193, 4096, False), (16, 12288, 2048, True), (16, 32768, 1024, False),
+    (16, 4096, 11008, True), (16, 1024, 11008, False), (17, 64, 64, False)])
+def test_few_row_fp8_calls_take_the_kernel_measured_faster(m, n, k, one_launch):
+    """Under an epilogue every call but a one-launch one goes through partial sums, which shows the choice."""
+    import ctypes
+
+    from flextensor_amd import _native as nat
+
+    b = ctypes.c_size_t(0)
+    nat.call("ftx_fp8_linear_scratch", m, (ctypes.c_int64 * 1)(n), 1, k, nat.FP8_EPILOGUE_RESIDUAL, ctypes.byref(b))
+    assert (b.value == 0) == one_launch

@@ -763,6 +763,7 @@ def test_decoder_layer_fused_path_against_the_separate_operations(gpu, default_c
 
 # Both sides of the lines where the one-launch, 64-row-tile and split-K kernels meet, with ragged n and k.
 @pytest.mark.parametrize("m,n,k", [(4, 300, 16400), (5, 300, 16400), (9, 5003, 10064), (9, 5003, 10000),
+                                   (4, 1641, 16400), (3, 28900, 1040), (8, 8193, 528), (9, 12289, 1040), (16, 1825, 10960),
                                    (17, 8201, 4112), (32, 8201, 4080), (33, 2049, 4112), (33, 2049, 4080),
                                    (48, 2177, 8176), (64, 5003, 4080), (64, 65600, 144)])
 def test_kernel_choice_matches_the_oracle_on_both_sides(gpu, default_config, m, n, k):
