@@ -1132,12 +1132,12 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
 //    matrices only. At 9 rows 8192 x 4096 0.97 and 10240 x 4096 1.13, 12288 x 1024 0.92 and 14336 x 1024 1.10, under
 //    SwiGLU 12288 x 512 0.97 and 14336 x 512 1.14; at 16 rows 2048 x 11008 0.91 and 1024 x 11008 1.09.
 //
-// bf16 weights are twice the bytes for the same x and their only other kernel is the library's GEMM, which takes
-// longer at every one of 19 shapes from 512 x 1024 to 152064 x 5120 at 1, 2, 4, 8, 12 and 16 rows. us at 1 / 8 / 16
-// rows, here and the library: 4096 x 4096 8.4 / 8.5 / 9.4 and 15.4 / 15.6 / 15.5; 11008 x 4096 17.4 / 18.0 / 20.3 and
-// 26.7 / 25.7 / 25.6; 32000 x 4096 (a head) 42.2 / 42.1 / 47.8 and 58.9 / 56.8 / 56.9; 128256 x 4096 157 / 156 / 179
-// and 182 / 184 / 186; 8192 x 28672 71.7 / 74.7 / 85.1 and 85.9 / 86.5 / 87.9; closest 1024 x 8192 at 16 rows, 12.0
-// and 12.1.
+// bf16 weights are twice the bytes for the same x, and their only other kernel is the library's GEMM: faster for
+// wide matrices of a short K only, which callers leave to it (hip.bf16_linear_eligible). us at 1 / 8 / 16 rows, here
+// and the library: 4096 x 4096 8.4 / 8.5 / 9.4 and 15.4 / 15.6 / 15.5; 11008 x 4096 17.4 / 18.0 / 20.3 and 26.7 /
+// 25.7 / 25.6; 32000 x 4096 (a head) 42.2 / 42.1 / 47.8 and 58.9 / 56.8 / 56.9; 128256 x 4096 157 / 156 / 179 and
+// 182 / 184 / 186; 8192 x 28672 71.7 / 74.7 / 85.1 and 85.9 / 86.5 / 87.9; closest 1024 x 8192 at 16 rows, 12.0 and
+// 12.1.
 bool direct_linear_wins(int64_t m, int64_t n_total, int64_t k, int epilogue) {
   if (m > kDirectMaxRows || n_total > kDirectMaxChannels) return false;
   const int64_t matrices = epilogue == kFp8EpilogueSwiglu ? 2 : 1;  // of a workgroup

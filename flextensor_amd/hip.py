@@ -769,13 +769,30 @@ def fp8_linear_residual(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tens
 BF16_LINEAR_MAX_ROWS = 16
 
 
+def _bf16_linear_wins(m: int, n: int, k: int) -> bool:
+    """Whether the one-launch kernel is faster than the library's GEMM for ``m`` rows of one [n, k] weight.
+
+    It is at every n from K = 2048 on (1.05 times its time at worst, 131072 x 3072 at 16 rows). Of a shorter K each
+    workgroup has little to do for its 16 channels, so many of them lose. Its time by the library's at 4, 8 and 16
+    rows: 8192 x 64 0.76, 0.79, 0.91 and 32768 x 64 1.65, 1.82, 1.94; 16384 x 256 0.81, 0.89, 1.03 and 65536 x 256
+    1.49, 1.59, 1.80; 32768 x 512 0.81, 0.88, 0.97 and 65536 x 512 1.12, 1.19, 1.35; 65536 x 1024 0.92, 1.05, 1.28.
+    The choice looks at one weight, so a projection has the same bits alone and in a group.
+    """
+    return n <= 8192 or k >= 2048 or (m <= 8 and k >= 1536) or n <= (64 if m <= 4 else 48 if m <= 8 else 12) * k
+
+
 def bf16_linear_eligible(x: torch.Tensor, *weights: torch.Tensor) -> bool:
-    """Whether :func:`bf16_linear` takes ``x`` [..., k] and these weights [n, k]."""
+    """Whether ``x`` [..., k] and these weights [n, k] are better off in :func:`bf16_linear` than in torch's linear,
+    and may run there."""
     if type(x) not in _PLAIN_TYPES:  # a subclass, or a proxy of a symbolic trace
         return False
     k = x.shape[-1] if x.dim() else 0
-    return (0 < k <= 1 << 29 and 0 < x.numel() <= BF16_LINEAR_MAX_ROWS * k and k % 8 == 0 and kernel_call(x, *weights)
-            and all(w.dim() == 2 and w.shape[1] == k and w.shape[0] > 0 for w in weights)
+    if not 0 < k <= 1 << 29 or not 0 < x.numel() <= BF16_LINEAR_MAX_ROWS * k or k % 8:
+        return False
+    m = x.numel() // k
+    return (kernel_call(x, *weights)
+            and all(w.dim() == 2 and w.shape[1] == k and w.shape[0] > 0 and _bf16_linear_wins(m, w.shape[0], k)
+                    for w in weights)
             and sum(w.shape[0] for w in weights) <= (1 << 27) - 128  # channels of one launch
             and _packed(x, *weights))
 

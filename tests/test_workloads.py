@@ -199,7 +199,20 @@ def test_calls_beyond_one_launch_are_left_to_torch(monkeypatch):
         q = meta(tokens, 1, 64, 64)
         assert hip.attention_eligible(q, q, q) == takes
     for channels, takes in ((1 << 27, False), (1 << 26, True)):
-        assert hip.bf16_linear_eligible(meta(1, 8), meta(channels, 8)) == takes
+        assert hip.bf16_linear_eligible(meta(1, 2048), meta(channels, 2048)) == takes
+
+
+@pytest.mark.parametrize("m,n,k,takes", [(1, 8192, 8, True), (1, 32768, 512, True), (1, 32776, 512, False),
+                                          (8, 24576, 512, True), (8, 24584, 512, False), (16, 12288, 1024, True),
+                                          (16, 12296, 1024, False), (16, 131072, 2048, True), (8, 131072, 1536, True)])
+def test_bf16_rows_take_the_kernel_measured_faster_for_each_weight(monkeypatch, m, n, k, takes):
+    """The choice is one weight's: a wide one leaves a group to torch, and does not change with its neighbours."""
+    from flextensor_amd import hip
+
+    monkeypatch.setattr(hip, "kernel_call", lambda *ts: True)
+    x, w, small = (torch.empty(s, dtype=torch.bfloat16, device="meta") for s in ((m, k), (n, k), (16, k)))
+    assert hip.bf16_linear_eligible(x, w) == hip.bf16_linear_eligible(x, small, w) == takes
+    assert hip.bf16_linear_eligible(x, small)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
