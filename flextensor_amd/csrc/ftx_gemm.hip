@@ -607,16 +607,24 @@ SegTable seg_table(const Fp8LinearLaunch &p) {
 // step: its loads past K are clamped into the row and both operands are
 // zeroed for the lane groups past K.
 //
-// Block order: the hardware hands workgroup b to XCD b % xcds. An XCD walks up
-// to kPBand m-tiles of one n-tile, then the same m-tiles of its next one, so
-// weight tiles come from its L2 for the band's other m-tiles and the band's
-// activations for its other n-tiles. Its n-tiles are every xcds-th one where
-// tiles outnumber the CUs (4 waves); calls of at most one tile per CU, and
-// 64-row tiles, give each XCD an equal run of tiles: of 17 n-tiles dealt in
-// turn one XCD has 3 and the others 2 (887 rows x 2125 x 10064, 64-row tiles:
-// 86.1 us dealt, 67.7 in runs; 577 x 23553 x 10224, 4 waves: 368 and 388).
+// Block order: the hardware hands workgroup b to XCD b % xcds. An XCD walks up to kPBand m-tiles of one n-tile,
+// then the same m-tiles of its next one, so weight tiles come from its L2 for the band's other m-tiles and the
+// band's activations for its other n-tiles. us in bands and not: 4096 x 8192 of 4096 rows 231 and 298, 28672 x 528
+// of 2048 rows 109.5 and 134.6, 2056 x 4112 of 4096 rows 96.2 and 112.8. Calls of up to 16 m-tiles and a short K
+// whose tiles are resident nearly all at once walk whole columns: 8200 x 1024 of 1500 rows 37.2 and 35.3, 2056 x
+// 1024 of 2048 rows 20.6 and 18.9 (28672 x 1024 of 1500 rows, 3.5 rounds: 109.8 and 119.7).
+//
+// Its n-tiles are every xcds-th one where tiles outnumber the CUs (4 waves: 577 x 23553 x 10224 368 us, in runs
+// 388). Calls of at most one tile per CU and 64-row tiles give each XCD an equal run of tiles, since a CU that gets
+// two of them doubles the time: of 17 n-tiles dealt in turn one XCD has 3 and the others 2 (887 rows x 2125 x 10064,
+// 64-row tiles: 86.1 us dealt, 67.7 in runs). 8-wave calls whose uneven deal still fits one tile per CU are dealt:
+// 129 rows x 11520 x 21456 187 us against 202, 1024 x 2056 x 528 11.2 against 11.7 (a whole number of n-tiles per
+// XCD, 385 x 8192 x 8192: 67.9 dealt, 66.2 in runs).
+//
+// An XCD's spare workgroups come last: between its tiles they left CUs with none beside CUs with two (2048 rows x
+// 2056 x 1024: 21.2 us, 18.7 with them last).
 constexpr int kPTileK = 64;
-constexpr int kPBand = 8;                            // m-tiles an XCD walks before the next n-tile
+constexpr int kPBand = 8;                            // m-tiles of a band
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -656,15 +664,17 @@ __device__ __forceinline__ void ring_barrier() {
 // per-step address work leaves the vector ALU (about 3% per layer, measured).
 //
 // Tiles are TM activation rows x TN channels. The smaller ones serve calls that leave the chip idle otherwise
-// (plan_fp8_linear) and the batches between decode and prefill (mid_linear_wins); those also split K: workgroup sp of a tile takes the steps from sp * split_steps and writes fp32 sums for
-// fp8_linear_reduce_kernel. At 64 x 128 four waves of 32 channels x 64 rows, four stages of 16 KB, two
-// workgroups per CU;
-// bound by the weights' bytes (28672 x 8192 at 64 rows: 70.8 us, 3.3 TB/s). Five and eight stages, four steps
-// at least per split and three workgroups per CU were within 5% or slower.
-template <int TM, int TN, int WAVES, int S, bool SADDR>
-__global__ __launch_bounds__(WAVES * 64, TM == 128 && WAVES == 4 ? 3 : 2) void fp8_prefill_kernel(const uint8_t *__restrict__ x, SegTable seg, int M,
-                                                                 int K, int m_tiles, int n_tiles, int xcds, int splits,
-                                                                 int split_steps, float *__restrict__ part) {
+// (plan_fp8_linear) and the batches between decode and prefill (mid_linear_wins); those also split K: workgroup sp
+// of a tile takes the steps from sp * split_steps and writes fp32 sums for fp8_linear_reduce_kernel. At 64 x 128
+// four waves of 32 channels x 64 rows, four stages of 16 KB, two workgroups per CU; bound by the weights' bytes
+// (28672 x 8192 at 64 rows: 70.8 us, 3.3 TB/s). Five and eight stages, four steps at least per split and three
+// workgroups per CU were within 5% or slower.
+template <int TM, int TN, int WAVES, int S, bool SADDR, bool DEAL>
+__global__ __launch_bounds__(WAVES * 64, TM == 128 && WAVES == 4 ? 3 : 2) void fp8_prefill_kernel(
+    const uint8_t *__restrict__ x, SegTable seg, int M, int K, int m_tiles, int n_tiles, int xcds,
+    int splits_or_band, int split_steps, float *__restrict__ part) {
+  // 64-row tiles: how often K is split; dealt tiles: m-tiles of a band
+  const int splits = splits_or_band, band = splits_or_band;
   static_assert(TM == 128 ? TN == 128 && (WAVES == 4 || WAVES == 8) : TM == 64 && WAVES == 4, "4 or 8 waves");
   constexpr int WN = TM == 64 && TN == 128 ? 4 : 2;       // waves side by side along the channels
   constexpr int IT = TN / WN / 16;                        // 16-channel weight tiles per wave
@@ -676,20 +686,35 @@ __global__ __launch_bounds__(WAVES * 64, TM == 128 && WAVES == 4 ? 3 : 2) void f
   __shared__ __align__(1024) uint8_t lds[S * kStage];
   const int xcd = blockIdx.x % xcds;
   const int slot = blockIdx.x / xcds;
-  constexpr bool kDeal = TM == 128 && WAVES == 4;  // n-tiles dealt to the XCDs in turn, or equal runs of tiles
-  const int n_own = kDeal ? (n_tiles + xcds - 1) / xcds : n_tiles;
-  const int items = m_tiles * n_tiles * (TM == 128 ? 1 : splits);
-  const int per_xcd = (items + xcds - 1) / xcds;
-  const int item = kDeal ? slot : xcd * per_xcd + slot;
-  if (!kDeal && (slot >= per_xcd || item >= items)) return;  // the last run may be shorter
-  const int sp = TM == 128 ? 0 : item % splits;
-  const int tile = TM == 128 ? item : item / splits;
-  const int band = tile / (kPBand * n_own);
-  const int at = tile - band * kPBand * n_own;
-  const int rows = min(kPBand, m_tiles - band * kPBand);
-  const int mt = band * kPBand + at % rows;
-  const int nt = kDeal ? at / rows * xcds + xcd : at / rows;
-  if (nt >= n_tiles) return;  // the last round of dealt n-tiles does not fill every XCD
+  // The block order described above; workgroups past an XCD's tiles come last.
+  int mt, nt, sp = 0;
+  if constexpr (DEAL) {
+    if (WAVES == 8 || m_tiles <= band) {
+      mt = slot % m_tiles;
+      nt = slot / m_tiles * xcds + xcd;
+    } else {
+      const int n_own = (n_tiles - xcd + xcds - 1) / xcds;
+      if (slot >= m_tiles * n_own) return;
+      const int first = slot / (band * n_own) * band;
+      const int at = slot - first * n_own;
+      const int rows = min(band, m_tiles - first);
+      mt = first + at % rows;
+      nt = at / rows * xcds + xcd;
+    }
+    if (nt >= n_tiles) return;
+  } else {
+    const int items = m_tiles * n_tiles * (TM == 128 ? 1 : splits);
+    const int per_xcd = (items + xcds - 1) / xcds;
+    const int item = xcd * per_xcd + slot;
+    if (slot >= per_xcd || item >= items) return;  // the last run may be shorter
+    sp = TM == 128 ? 0 : item % splits;
+    const int tile = TM == 128 ? item : item / splits;
+    const int run = tile / (kPBand * n_tiles);
+    const int at = tile - run * kPBand * n_tiles;
+    const int rows = min(kPBand, m_tiles - run * kPBand);
+    mt = run * kPBand + at % rows;
+    nt = at / rows;
+  }
   int s = 0;
   while (s + 1 < seg.count && nt >= seg.rg0[s + 1]) ++s;
   const int N = seg.n[s];
@@ -1048,8 +1073,11 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
     // at most one tile per CU: 8 waves (two per SIMD) and 4 LDS stages in one
     // workgroup; more tiles: 4 waves and 2 stages, three workgroups per CU
     p.waves = (waves == 4 || waves == 8) ? waves : (m_tiles * n_tiles <= cus ? 8 : 4);
-    p.grid = p.waves == 4 ? p.xcds * m_tiles * ((n_tiles + p.xcds - 1) / p.xcds)
-                          : p.xcds * ((m_tiles * n_tiles + p.xcds - 1) / p.xcds);
+    const int64_t dealt = m_tiles * ((n_tiles + p.xcds - 1) / p.xcds);  // the most tiles of an XCD
+    p.deal = p.waves == 4 || (n_tiles % p.xcds && dealt <= cus / p.xcds);
+    p.grid = p.xcds * (p.deal ? dealt : (m_tiles * n_tiles + p.xcds - 1) / p.xcds);
+    // no bands where the tiles of a short K are all resident in a round and a half (three to a CU)
+    p.band = m_tiles <= 2 * kPBand && k <= 2048 && dealt * 2 * p.xcds <= 9 * cus ? static_cast<int>(m_tiles) : kPBand;
     p.small = offsets_fit(p);
     p.tile_n = kPTileN;
     // Half of the chip or more would be idle: 64 x 128 tiles, and 64 x 64 while those leave half idle too. A
@@ -1065,6 +1093,8 @@ Fp8LinearLaunch plan_fp8_linear(int64_t m, const int64_t *n, int group, int64_t 
       p.tile_n = p.m_tiles * n_tiles * 2 <= cus ? 64 : 128;
       p.row_groups = 0;
       for (int s = 0; s < group; ++s) p.row_groups += (n[s] + p.tile_n - 1) / p.tile_n;
+      p.deal = false;
+      p.band = kPBand;
       p.grid = p.xcds * ((p.m_tiles * p.row_groups + p.xcds - 1) / p.xcds);
     }
     return p;
@@ -1179,6 +1209,7 @@ void plan_mid_linear(Fp8LinearLaunch *p, int cus, int xcds) {
   p->kc = split_steps * kPTileK;
   p->tile_n = kPTileN;
   p->m_tiles = 1;
+  p->band = 1;
   p->row_groups = n_tiles;
   p->grid = p->xcds * ((p->splits * n_tiles + p->xcds - 1) / p->xcds);
   p->scratch_bytes = p->splits > 1 || p->epilogue != kFp8EpilogueNone
@@ -1233,19 +1264,19 @@ hipError_t launch_direct(const Fp8LinearLaunch &p, hipStream_t stream) {
   return p.m <= 8 ? launch_direct_rows<true, 4>(p, stream) : launch_direct_rows<true, 8>(p, stream);
 }
 
-template <int TM, int TN, int WAVES, int S>
+template <int TM, int TN, int WAVES, int S, bool DEAL>
 void launch_tiled(const Fp8LinearLaunch &p, const SegTable &seg, float *part, hipStream_t stream) {
   const auto *x = static_cast<const uint8_t *>(p.x);
   const int m = static_cast<int>(p.m), k = static_cast<int>(p.k), mt = static_cast<int>(p.m_tiles),
             nt = static_cast<int>(p.row_groups);
   const int split_steps = static_cast<int>(p.kc / kPTileK);
   const dim3 grid(static_cast<unsigned>(p.grid)), block(WAVES * kWave);
-  if (p.small)
-    hipLaunchKernelGGL((fp8_prefill_kernel<TM, TN, WAVES, S, true>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
-                       p.splits, split_steps, part);
-  else
-    hipLaunchKernelGGL((fp8_prefill_kernel<TM, TN, WAVES, S, false>), grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds,
-                       p.splits, split_steps, part);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, x, seg, m, k, mt, nt, p.xcds, DEAL ? p.band : p.splits,
+                       split_steps, part);
+  };
+  p.small ? launch(fp8_prefill_kernel<TM, TN, WAVES, S, true, DEAL>)
+          : launch(fp8_prefill_kernel<TM, TN, WAVES, S, false, DEAL>);
 }
 
 }  // namespace
@@ -1256,14 +1287,15 @@ hipError_t launch_fp8_linear(const Fp8LinearLaunch &p, hipStream_t stream) {
     const SegTable seg = seg_table(p);
     if (p.mid) {
       const bool reduce = p.scratch_bytes > 0;
-      (p.tile_n == 64 ? launch_tiled<64, 64, 4, 4> : launch_tiled<64, 128, 4, 4>)(p, seg, reduce ? static_cast<float *>(p.workspace) : nullptr, stream);
+      const auto tiles = p.tile_n == 64 ? launch_tiled<64, 64, 4, 4, false> : launch_tiled<64, 128, 4, 4, false>;
+      tiles(p, seg, reduce ? static_cast<float *>(p.workspace) : nullptr, stream);
       const hipError_t err = hipGetLastError();
       return err != hipSuccess || !reduce ? err : launch_reduce(p, seg, stream);
     }
-    if (p.waves == 8)
-      launch_tiled<128, 128, 8, 4>(p, seg, nullptr, stream);
+    if (p.waves == 4)
+      launch_tiled<128, 128, 4, 2, true>(p, seg, nullptr, stream);
     else
-      launch_tiled<128, 128, 4, 2>(p, seg, nullptr, stream);
+      (p.deal ? launch_tiled<128, 128, 8, 4, true> : launch_tiled<128, 128, 8, 4, false>)(p, seg, nullptr, stream);
     return hipGetLastError();
   }
   switch (p.batch_blocks) {

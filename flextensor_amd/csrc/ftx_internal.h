@@ -98,6 +98,8 @@ struct Fp8LinearLaunch {
   int64_t m_tiles;    // prefill: tiles of 128 or 64 activation rows (row_groups then counts tiles of tile_n channels)
   int tile_n;         // prefill: channels of a tile
   int xcds;           // prefill: L2 domains the block order is arranged for
+  int band;           // prefill of 4 waves: m-tiles an XCD walks before its next n-tile
+  bool deal;          // prefill: n-tiles dealt to the XCDs in turn, or equal runs of tiles
   bool small;         // prefill: 32-bit load offsets reach every operand
   bool mid;           // prefill kernel with 64-row tiles; up to 64 rows K may be split over workgroups
   bool direct;        // the one-launch decode kernel: no workspace, a workgroup per 16 channels

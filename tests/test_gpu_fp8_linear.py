@@ -783,7 +783,9 @@ def test_kernel_choice_matches_the_oracle_on_both_sides(gpu, default_config, m, 
     assert torch.equal(hip.fp8_linear_residual(xt, wt, st, resid), resid + want.to(gpu))
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 1000, 1040), (130, 4160, 528), (300, 5003, 208), (1100, 200, 272), (2100, 129, 80)])
+# The last three: n-tiles dealt unevenly to the XCDs in one round, in two, and in bands of the rows.
+@pytest.mark.parametrize("m,n,k", [(65, 1000, 1040), (130, 4160, 528), (300, 5003, 208), (1100, 200, 272), (2100, 129, 80),
+                                   (260, 2100, 272), (2048, 2056, 80), (1100, 3400, 2000)])
 def test_small_prefill_tiles_agree_bitwise_with_the_large_ones(gpu, default_config, m, n, k):
     """Calls that leave the chip idle run 64 x 128 or 64 x 64 tiles, long ones walk the rows in bands: the same
     sums in the same order as the fixed 128 x 128 launch shapes, also in a group."""
