@@ -417,7 +417,8 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void direct_linear_kernel(con
     const bool ok = at + lcol < row_bytes;
 #pragma unroll
     for (int j = 0; j < kLoads; ++j)
-      v[j] = ok ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w + row_at[j] + at)) : u32x4{0u, 0u, 0u, 0u};
+      v[j] = ok ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(w + row_at[j] + at))
+                : u32x4{0u, 0u, 0u, 0u};
   };
   auto load_x = [&](u32x4(&v)[XL], int win) {
     const int64_t at = static_cast<int64_t>(win) * kWindowX;

@@ -232,7 +232,9 @@ hipError_t launch_norm_residual(const NormLaunch &p, hipStream_t stream) {
   switch (p.norm) {
     case kNormNone: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormNone>), grid, block, lds, stream, p); break;
     case kNormRms: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormRms>), grid, block, lds, stream, p); break;
-    case kNormAffine: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormAffine>), grid, block, lds, stream, p); break;
+    case kNormAffine:
+      hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormAffine>), grid, block, lds, stream, p);
+      break;
     default: hipLaunchKernelGGL((norm_kernel<WAVES, RESIDUAL, kNormAdaln>), grid, block, lds, stream, p); break;
   }
   return hipGetLastError();

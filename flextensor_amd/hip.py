@@ -435,7 +435,8 @@ def _check_operands(what: str, **tensors: torch.Tensor) -> None:
             raise ValueError(f"{what} runs on the current GPU, {name} is on {t.device}")
         if torch.is_grad_enabled() and t.requires_grad:
             raise ValueError(f"{what} has no backward and {name} requires a gradient")
-        if torch.autograd.forward_ad._current_level >= 0 and torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+        fwd = torch.autograd.forward_ad
+        if fwd._current_level >= 0 and fwd.unpack_dual(t).tangent is not None:
             raise ValueError(f"{what} has no forward-mode derivative and {name} carries a tangent")
 
 
@@ -543,7 +544,8 @@ def _rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, 
         if cache.dim() != 4 or cache.shape[0] < b or cache.shape[1] < pos + t or cache.shape[2:] != (kv, d):
             return None
         strides.append(_head_strides(cache))
-        if strides[-1] is None or 0 in cache.stride() or (cache.is_inference() and not torch.is_inference_mode_enabled()):
+        if (strides[-1] is None or 0 in cache.stride()
+                or (cache.is_inference() and not torch.is_inference_mode_enabled())):
             return None
     if cache_k.data_ptr() == cache_v.data_ptr():
         return None

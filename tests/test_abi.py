@@ -252,8 +252,8 @@ def test_launches_beyond_the_threads_of_a_grid_are_refused_or_planned_otherwise(
     assert lib.ftx_attention_workspace(1 << 24, 1, 8, 64, 64, 64, ctypes.byref(b)) == nat.FTX_ERR_UNSUPPORTED
     assert lib.ftx_attention_workspace(1 << 19, 1, 8, 64, 64, 64, ctypes.byref(b)) == nat.FTX_OK
     for rows, dim in ((1 << 26, 2048), (1 << 24, 8192), (1 << 22, 32768)):
-        assert lib.ftx_norm(None, None, None, None, rows, dim, nat.NORM_RMS, None, None, None, None, 1, -1, -1, -1, 1e-5,
-                            None) == nat.FTX_ERR_UNSUPPORTED
+        assert lib.ftx_norm(None, None, None, None, rows, dim, nat.NORM_RMS, None, None, None, None, 1, -1, -1, -1,
+                            1e-5, None) == nat.FTX_ERR_UNSUPPORTED
     assert lib.ftx_silu_mul(None, None, None, 1 << 35, None) == nat.FTX_ERR_UNSUPPORTED
     ptr = (ctypes.c_void_p * 1)(None)
     n = (ctypes.c_int64 * 1)(1 << 27)

@@ -763,7 +763,8 @@ def test_decoder_layer_fused_path_against_the_separate_operations(gpu, default_c
 
 # Both sides of the lines where the one-launch, 64-row-tile and split-K kernels meet, with ragged n and k.
 @pytest.mark.parametrize("m,n,k", [(4, 300, 16400), (5, 300, 16400), (9, 5003, 10064), (9, 5003, 10000),
-                                   (4, 1641, 16400), (3, 28900, 1040), (8, 8193, 528), (9, 12289, 1040), (16, 1825, 10960),
+                                   (4, 1641, 16400), (3, 28900, 1040), (8, 8193, 528), (9, 12289, 1040),
+                                   (16, 1825, 10960),
                                    (17, 8201, 4112), (32, 8201, 4080), (33, 2049, 4112), (33, 2049, 4080),
                                    (48, 2177, 8176), (64, 5003, 4080), (64, 65600, 144)])
 def test_kernel_choice_matches_the_oracle_on_both_sides(gpu, default_config, m, n, k):
@@ -784,8 +785,8 @@ def test_kernel_choice_matches_the_oracle_on_both_sides(gpu, default_config, m, 
 
 
 # The last three: n-tiles dealt unevenly to the XCDs in one round, in two, and in bands of the rows.
-@pytest.mark.parametrize("m,n,k", [(65, 1000, 1040), (130, 4160, 528), (300, 5003, 208), (1100, 200, 272), (2100, 129, 80),
-                                   (260, 2100, 272), (2048, 2056, 80), (1100, 3400, 2000)])
+@pytest.mark.parametrize("m,n,k", [(65, 1000, 1040), (130, 4160, 528), (300, 5003, 208), (1100, 200, 272),
+                                   (2100, 129, 80), (260, 2100, 272), (2048, 2056, 80), (1100, 3400, 2000)])
 def test_small_prefill_tiles_agree_bitwise_with_the_large_ones(gpu, default_config, m, n, k):
     """Calls that leave the chip idle run 64 x 128 or 64 x 64 tiles, long ones walk the rows in bands: the same
     sums in the same order as the fixed 128 x 128 launch shapes, also in a group."""

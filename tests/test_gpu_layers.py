@@ -364,10 +364,12 @@ def test_public_kernel_functions_refuse_what_has_no_answer(gpu):
     hip.attention(q, q, q)
     hip.bf16_linear(x, [w])
     shifted = torch.empty(q.numel() + 4, dtype=torch.bfloat16, device=gpu)[4:].view_as(q)
-    for args in ((q, q.cpu(), q.cpu()), (shifted, q, q), (q, shifted, q), (q, q, q.transpose(2, 3).contiguous().transpose(2, 3))):
+    for args in ((q, q.cpu(), q.cpu()), (shifted, q, q), (q, shifted, q),
+                 (q, q, q.transpose(2, 3).contiguous().transpose(2, 3))):
         with pytest.raises(ValueError):
             hip.attention(*args)
-    for args in ((x, [w.cpu()]), (x[:, ::2], [w[:, :32].contiguous()]), (x, [w[:, :32].contiguous()]), (x.view(-1)[1:65], [w])):
+    for args in ((x, [w.cpu()]), (x[:, ::2], [w[:, :32].contiguous()]), (x, [w[:, :32].contiguous()]),
+                 (x.view(-1)[1:65], [w])):
         with pytest.raises(ValueError):
             hip.bf16_linear(*args)
     for call in (lambda t: hip.attention(t(q), q, q), lambda t: hip.bf16_linear(x, [t(w)])):

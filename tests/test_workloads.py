@@ -129,8 +129,9 @@ def test_public_kernel_functions_refuse_operands_the_kernel_would_misread():
     from flextensor_amd import hip
 
     q, kv = torch.zeros(2, 3, 4, 64, dtype=torch.bfloat16), torch.zeros(2, 5, 2, 64, dtype=torch.bfloat16)
-    for args, error in (((q, kv[:1], kv[:1]), "batch"), ((q, kv, kv[:, :4]), "differ"), ((q, kv[..., :32], kv[..., :32]), "head dim"),
-                        ((q[0], kv[0], kv[0]), "dimensions"), ((q, kv, kv), "current GPU")):
+    for args, error in (((q, kv[:1], kv[:1]), "batch"), ((q, kv, kv[:, :4]), "differ"),
+                        ((q, kv[..., :32], kv[..., :32]), "head dim"), ((q[0], kv[0], kv[0]), "dimensions"),
+                        ((q, kv, kv), "current GPU")):
         with pytest.raises(ValueError, match=error):
             hip.attention(*args)
     with pytest.raises(TypeError, match="bf16"):
@@ -138,9 +139,10 @@ def test_public_kernel_functions_refuse_operands_the_kernel_would_misread():
     x, w = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(8, 64, dtype=torch.bfloat16)
     r = torch.zeros(4, 8, dtype=torch.bfloat16)
     res = hip.nat.FP8_EPILOGUE_RESIDUAL
-    for args, error in (((x, [w[:, :32].contiguous()]), r"\[n, 64\]"), ((x[:, ::2], [w[:, :32].contiguous()]), "contiguous"),
-                        ((x, [w, w.t().contiguous().t()]), "contiguous"),
-                        ((x[:, :0], [w[:, :0]]), r"\[..., k\]"), ((x, [w], res, r[:2]), "residual"), ((x, [w]), "current GPU")):
+    for args, error in (((x, [w[:, :32].contiguous()]), r"\[n, 64\]"),
+                        ((x[:, ::2], [w[:, :32].contiguous()]), "contiguous"),
+                        ((x, [w, w.t().contiguous().t()]), "contiguous"), ((x[:, :0], [w[:, :0]]), r"\[..., k\]"),
+                        ((x, [w], res, r[:2]), "residual"), ((x, [w]), "current GPU")):
         with pytest.raises(ValueError, match=error):
             hip.bf16_linear(*args)
     for args in ((x.float(), [w.float()]), (x, [w.float()]), (x, [w], res, r.float())):
@@ -219,8 +221,8 @@ def test_bf16_rows_take_the_kernel_measured_faster_for_each_weight(monkeypatch, 
 def test_norms_and_projections_trace_symbolically_and_script(dtype):
     """``torch.fx.symbolic_trace`` and ``torch.jit.script`` of the modules that may run a kernel, with torch's
     operations in the graph: the results of the module itself."""
-    mods = [W.RMSNorm(32, 1e-5, dtype), W.LayerNorm(32, eps=1e-5, dtype=dtype), W.Linear(32, 16, bias=False, dtype=dtype),
-            W.Linear(32, 16, dtype=dtype)]
+    mods = [W.RMSNorm(32, 1e-5, dtype), W.LayerNorm(32, eps=1e-5, dtype=dtype),
+            W.Linear(32, 16, bias=False, dtype=dtype), W.Linear(32, 16, dtype=dtype)]
     x = torch.randn(2, 3, 32, generator=torch.Generator().manual_seed(1)).to(dtype)
     with torch.no_grad():
         for mod in mods:
