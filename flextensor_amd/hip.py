@@ -482,11 +482,13 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor 
     if type(x) not in _PLAIN_TYPES:  # a subclass, or a proxy of a symbolic trace
         return None
     dim = x.shape[-1] if x.dim() else 0
-    if (not dim or dim % 8 or dim > NORM_MAX_DIM or not x.numel() or not _norm_rows_fit(x.numel() // dim, dim)
+    numel = x.numel()
+    if (not dim or dim % 8 or dim > NORM_MAX_DIM or not numel
+            or (numel > 1 << 28 and not _norm_rows_fit(numel // dim, dim))
             or not kernel_call(x, weight) or weight.shape != (dim,) or not _packed(x, weight)):
         return None
     y = torch.empty_like(x)
-    nat.call("ftx_norm", x.data_ptr(), None, None, y.data_ptr(), x.numel() // dim, dim, nat.NORM_RMS,
+    nat.call("ftx_norm", x.data_ptr(), None, None, y.data_ptr(), numel // dim, dim, nat.NORM_RMS,
              weight.data_ptr(), None, None, None, 1, -1, -1, -1, eps, _stream())
     return y
 
@@ -528,9 +530,8 @@ def _rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, 
     """:func:`rope_cache`, with the caches' strides: ``(rotated q, cache_k strides, cache_v strides)``."""
     b, t, h, d = q.shape
     kv = k.shape[2]
-    if (type(pos) is not int or pos < 0 or d % 16 or d > 4096 or max(b, t) > 1 << 24 or max(h, kv) > 65536
-            or pos > 1 << 30 or b * t * (h + 2 * kv) * d > 1 << 35 or not q.numel() or k.shape != (b, t, kv, d)
-            or v.shape != k.shape or not _packed(q, k, v)):
+    if (type(pos) is not int or pos < 0 or d % 16 or not 0 < b * t * (h + 2 * kv) * d <= 1 << 35 or not h
+            or k.shape != (b, t, kv, d) or v.shape != k.shape or not _packed(q, k, v)):
         return None
     grad = torch.is_grad_enabled()
     device = q.get_device()
@@ -549,7 +550,7 @@ def _rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, 
             return None
     if cache_k.data_ptr() == cache_v.data_ptr():
         return None
-    torch.autograd.graph.increment_version((cache_k, cache_v))  # as an in-place operation, for what autograd saved
+    torch._C._increment_version((cache_k, cache_v))  # as an in-place operation, for what autograd saved
     out = torch.empty_like(q)
     nat.call("ftx_rope_cache", q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(),
              out.data_ptr(), cache_k.data_ptr(), cache_v.data_ptr(), b, t, h, kv, d, pos,
@@ -562,7 +563,11 @@ def rope_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.Ten
     """The rotated queries of [batch, t, head, d] ``q``; the rotated ``k`` and ``v`` go to positions ``pos ..
     pos + t - 1`` of the caches, in one launch (``ftx_rope_cache``). None when the kernel does not take the
     call."""
-    got = _rope(q, k, v, cos, sin, pos, cache_k, cache_v, _stream()) if kernel_call(q, k, v, cache_k, cache_v) else None
+    b, t, h, d = q.shape
+    if max(b, t) > 1 << 24 or max(h, k.shape[2]) > 65536 or d > 4096 or not kernel_call(q, k, v, cache_k, cache_v) or (
+            type(pos) is int and pos > 1 << 30):
+        return None
+    got = _rope(q, k, v, cos, sin, pos, cache_k, cache_v, _stream())
     return got[0] if got is not None else None
 
 
@@ -789,14 +794,17 @@ def bf16_linear_eligible(x: torch.Tensor, *weights: torch.Tensor) -> bool:
     if type(x) not in _PLAIN_TYPES:  # a subclass, or a proxy of a symbolic trace
         return False
     k = x.shape[-1] if x.dim() else 0
-    if not 0 < k <= 1 << 29 or not 0 < x.numel() <= BF16_LINEAR_MAX_ROWS * k or k % 8:
+    numel = x.numel()
+    if not 0 < k <= 1 << 29 or not 0 < numel <= BF16_LINEAR_MAX_ROWS * k or k % 8 or not kernel_call(x, *weights):
         return False
-    m = x.numel() // k
-    return (kernel_call(x, *weights)
-            and all(w.dim() == 2 and w.shape[1] == k and w.shape[0] > 0 and _bf16_linear_wins(m, w.shape[0], k)
-                    for w in weights)
-            and sum(w.shape[0] for w in weights) <= (1 << 27) - 128  # channels of one launch
-            and _packed(x, *weights))
+    channels = 0
+    for w in weights:
+        shape = w.shape
+        n = shape[0] if len(shape) == 2 and shape[1] == k else 0
+        if not n or (k < 2048 and not _bf16_linear_wins(numel // k, n, k)):
+            return False
+        channels += n
+    return channels <= (1 << 27) - 128 and _packed(x, *weights)  # channels of one launch
 
 
 def bf16_linear(x: torch.Tensor, weights: list[torch.Tensor], epilogue: int = nat.FP8_EPILOGUE_NONE,
