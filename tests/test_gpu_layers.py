@@ -300,7 +300,7 @@ def test_small_kernels_stay_off_the_cus_of_a_ring_copy(gpu):
             torch.cuda.synchronize()
             best[beside] = min(best.get(beside, math.inf), start.elapsed_time(end) * 20)
         print(f"{name}: {best[False]:.2f} us alone, {best[True]:.2f} beside the copy", flush=True)
-        assert best[True] < 7 * best[False]
+        assert best[True] < best[False] + 16
         del graph
 
 
